@@ -497,8 +497,8 @@ __global__ __launch_bounds__(SEL_WAVES * 64) void select_main_kernel(
 // around the previous row's crossing (window_cross: a few keys per lane, one
 // histogram pass), then in the window above or below it, and by the radix
 // passes only when both miss (a few rows in 10^4 at 720p).  A work-group
-// walks 16 batches (512 rows): the cluster sizes it loads once are amortised
-// over them, and the next batch's query rows load while the current batch is
+// walks up to 16 batches (sf_batches): the cluster sizes it loads once are
+// amortised over them, and the next batch's query rows load while the current batch is
 // being selected.  LDS: the batch's keys (128 KB; 16-byte chunks XOR
 // swizzled by row instead of padded), twelve 1.75 KB window histograms and the
 // cluster sizes.  The centroid fragments are reloaded from L2 per batch (held
@@ -508,7 +508,9 @@ __global__ __launch_bounds__(SEL_WAVES * 64) void select_main_kernel(
 // ---------------------------------------------------------------------------
 #define SF_WAVES 12
 #define SF_ROWS 32
-#define SF_BATCHES 16
+#define SF_BATCHES 16    // most batches a work-group takes (sf_batches)
+#define SF_CUS 256       // compute units: one work-group each
+#define SF_START 0.8     // a work-group's start (sizes, first rows by radix passes), in batches
 #define SF_PITCH SEL_NC  // halves per LDS key row (chunks swizzled by row, no padding)
 #define SF_TILES 6       // most 32-centroid score tiles a wave holds (64 tiles over 12 waves)
 
@@ -517,7 +519,7 @@ __global__ __launch_bounds__(SF_WAVES * 64, 1) void score_select_kernel(
     const uint16_t* __restrict__ QU, const uint16_t* __restrict__ cks,
     const int32_t* __restrict__ kcounts, const int32_t* __restrict__ qperm,
     const int32_t* __restrict__ off, const int32_t* __restrict__ ns_dev,
-    int32_t* __restrict__ unip, int32_t* __restrict__ rowcnt, int N, int CQ) {
+    int32_t* __restrict__ unip, int32_t* __restrict__ rowcnt, int N, int CQ, int batches) {
   __shared__ __attribute__((aligned(16))) uint16_t sKey[SF_ROWS * SF_PITCH];
   __shared__ __attribute__((aligned(16))) int hist_all[SF_WAVES][SEL_WHIST];
   // rows of a batch are handed out one at a time (a counter per batch
@@ -532,7 +534,7 @@ __global__ __launch_bounds__(SF_WAVES * 64, 1) void score_select_kernel(
   const int32_t* offh = off + (size_t)h * (CQ + 1);
   int lim = offh[CQ];
   if (lim > N) lim = N;  // qcounts summing past N is invalid input; never read past N
-  const int base = blockIdx.x * SF_ROWS * SF_BATCHES;
+  const int base = blockIdx.x * SF_ROWS * batches;
   if (base >= lim) return;
   // the key total
   int ktot = 0;
@@ -591,7 +593,7 @@ __global__ __launch_bounds__(SF_WAVES * 64, 1) void score_select_kernel(
   load_ca(ca0, ca1);
   if (threadIdx.x < 2) sNext[threadIdx.x] = 0;
   for (int c = threadIdx.x; c < SEL_NC; c += SF_WAVES * 64) sSz[c] = kcounts[(size_t)h * SEL_NC + c];
-  for (int b = 0; b < SF_BATCHES; ++b) {
+  for (int b = 0; b < batches; ++b) {
     const int j0 = base + SF_ROWS * b;
     if (j0 >= lim) break;
     {  // scores of rows j0 .. j0 + 31 against the wave's centroids -> keys in LDS
@@ -730,15 +732,41 @@ static int select_common(const void* gl, const int32_t* kcounts, const int32_t* 
   return T2T_OK;
 }
 
+// Batches per work-group.  One work-group fills a CU, so a launch runs in
+// rounds of SF_CUS work-groups of batches + SF_START batch times each (the
+// start: cluster sizes, and each wave's first row by the radix passes, having
+// no previous crossing); the fewest batch times win.  Fixed at 16 batches, a
+// call of few rows left most CUs idle (2 heads x 4096 rows: 16 work-groups,
+// 223 us against 30 at one batch) and one of slightly over a whole number of
+// rounds ran the last one nearly empty (5 x 32760: 402 us against 289 at 7
+// batches; 7 x 98304: 940 against 872 at 12).  Past eight rounds work-groups
+// drift apart and the last round fills up by itself: 16 (40 x 75600: 3930 us
+// against 3970 at the model's 15).
+static int sf_batches(int H, int N) {
+  if ((long long)H * cdiv(N, SF_ROWS * SF_BATCHES) > 8 * SF_CUS) return SF_BATCHES;
+  int best = SF_BATCHES;
+  double bc = 1e30;
+  for (int nb = SF_BATCHES; nb >= 1; --nb) {
+    const long long wgs = (long long)H * cdiv(N, SF_ROWS * nb);
+    const double cost = (double)((wgs + SF_CUS - 1) / SF_CUS) * (nb + SF_START);
+    if (cost < bc) {
+      bc = cost;
+      best = nb;
+    }
+  }
+  return best;
+}
+
 static int score_select_launch(const void* QU, const void* cks, const int32_t* kcounts,
                                const int32_t* qperm, const int32_t* qcounts,
                                const int32_t* ns_dev, int32_t* unip, int32_t* rowcnt, int H,
                                int N, int CQ, int32_t* off, hipStream_t st) {
   hipLaunchKernelGGL(select_prep_kernel, dim3(H), dim3(1024), 0, st, qcounts, off, unip, CQ);
   T2T_LAUNCH_CHECK("score_select prep");
-  hipLaunchKernelGGL(score_select_kernel, dim3(cdiv(N, SF_ROWS * SF_BATCHES), H),
+  const int batches = sf_batches(H, N);
+  hipLaunchKernelGGL(score_select_kernel, dim3(cdiv(N, SF_ROWS * batches), H),
                      dim3(SF_WAVES * 64), 0, st, (const uint16_t*)QU, (const uint16_t*)cks,
-                     kcounts, qperm, off, ns_dev, unip, rowcnt, N, CQ);
+                     kcounts, qperm, off, ns_dev, unip, rowcnt, N, CQ, batches);
   T2T_LAUNCH_CHECK("score_select");
   return T2T_OK;
 }
