@@ -332,6 +332,14 @@ int t2t_fused_update_vstats(const void* x, const int32_t* labels, const void* ol
                             const void* v, int v_dtype, float* cent, int32_t* counts,
                             float* vmean, int H, int N, int C, int D, void* ws,
                             size_t ws_bytes, void* stream);
+/* Warm Lloyd iterations in place on cen [H, C, D] fp16: `iters` times
+ * t2t_fast_assign and the fp32 means of t2t_fused_update_vstats (without v)
+ * rounded to fp16; empty clusters keep theirs.  D == 32; ws >=
+ * t2t_lloyd_ws_bytes.  Replaces the warm loop of init_state,
+ * operator/deploy_step.py:257-264. */
+size_t t2t_lloyd_ws_bytes(int H, int N, int C);
+int t2t_lloyd(const void* x, void* cen, int iters, int H, int N, int C, int D, void* ws,
+              size_t ws_bytes, void* stream);
 /* G[h] = x[h]^T x[h] / N in fp64 ([H, D, D]); bf16 x is rounded to fp16
  * first.  Replaces the Gram products of online_u,
  * operator/deploy_step.py:135-137. D <= 128.  ws holds the per-split partial

@@ -28,7 +28,7 @@ def structure(rng, H, N, CQ, CK=2048):
     return qlab, klab, qperm, qcounts, kperm, kcounts
 
 
-# one, two, seven and sixteen row batches per selection work-group, with
+# one, two, eight and ten row batches per selection work-group, with
 # partial last batches and work-groups
 @pytest.mark.parametrize("H,N,CQ", [(1, 2049, 5), (4, 2500, 40), (7, 8161, 64), (19, 8161, 33)])
 def test_score_select_batches_match_unfused(dev, H, N, CQ):
@@ -42,3 +42,42 @@ def test_score_select_batches_match_unfused(dev, H, N, CQ):
     u, r = ops.score_select(QU, cks, tk, tp, tq, ns)
     u2, r2 = ops.select_union(ops.score(QU, cks), tk, tp, tq, ns)
     assert torch.equal(u, u2) and torch.equal(r, r2)
+
+
+# row blocks of 1, 2 and 4 per wave; cluster counts around the 32-centroid
+# blocks and 512-centroid chunks; rows that end inside a block
+@pytest.mark.parametrize("H,N,C", [(1, 33, 1), (2, 1000, 31), (3, 4097, 513), (16, 16450, 100),
+                                   (4, 262500, 40), (2, 3000, 2048)])
+def test_fast_assign_rank32_equals_general_form(dev, H, N, C):
+    """D = 32 has its own kernel; zero dims appended change no sum, so the
+    general kernel at D = 64 must give the same labels, bit for bit."""
+    from token2tile_amd import ops
+    gen = torch.Generator(device=dev).manual_seed(N + C)
+    x = torch.randn(H, N, 32, generator=gen, device=dev).half()
+    cen = torch.randn(H, C, 32, generator=gen, device=dev).half()
+    if C > 30:
+        cen[:, 7] = cen[:, 29]               # equal distances: the lowest index wins
+        x[:, :20] = cen[:, 10:30]            # distance zero, of either sign
+        x[:, 21, 3] = float("inf")
+        x[:, 22, 5] = float("nan")
+        x[:, 23] = 60000.0
+    pad = lambda t: torch.cat([t, torch.zeros_like(t)], 2).contiguous()  # noqa: E731
+    want = ops.fast_assign_labels(pad(x), pad(cen))
+    assert torch.equal(ops.fast_assign_labels(x, cen), want)
+
+
+@pytest.mark.parametrize("H,N,C", [(2, 3001, 7), (3, 5000, 2048)])
+def test_lloyd_equals_separate_calls(dev, H, N, C):
+    """The in-place iterations (labels seeded by the previous ones) against
+    assign, update and cast called one by one."""
+    from token2tile_amd import ops
+    gen = torch.Generator(device=dev).manual_seed(N)
+    x = torch.randn(H, N, 32, generator=gen, device=dev).half()
+    cen = torch.randn(H, C, 32, generator=gen, device=dev).half()
+    cen[:, 3] = 100.0                        # an empty cluster
+    want = cen.clone()
+    for _ in range(3):
+        lab = ops.fast_assign_labels(x, want)
+        want = ops.fused_update_vstats(x, lab, want)[0].half()
+    assert torch.equal(ops.lloyd(x, cen.clone(), 3), want)
+    assert torch.equal(ops.lloyd(x, cen.clone(), 0), cen)

@@ -102,6 +102,195 @@ __global__ __launch_bounds__(256) void fast_assign_kernel(const uint16_t* __rest
 }
 
 // ---------------------------------------------------------------------------
+// fast_assign at D = 32, the rank of the projected space: the labels of
+// fast_assign_kernel, bit for bit (same operands, same fp32 operations, same
+// keys), in the loop shape of assign_km_kernel: eight waves of RB 32-row
+// blocks, so a centroid fragment read from LDS feeds RB MFMA chains, and the
+// centroids staged 512 at a time with their norms.
+//
+// The general form is bound by its VALU work, 3.5 operations per distance
+// against two MFMAs per 1024.  Here a block of 16 distances costs its 16
+// fused multiply-adds and a min tree; fp32 addition is monotone, so the least
+// distance is |x|^2 + the least (|c|^2 - 2 x.c), and when that is not
+// negative and its key's distance part is above the running key's, no key of
+// the block can win.  Only other blocks (and any with a NaN, which the tree
+// hands on) build their 16 keys.
+//
+// guess (optional): a label per row, any value.  The distance to that
+// centroid, summed here, plus 2^-15 of the sum of its terms' magnitudes is
+// above the MFMA's (33 terms in any order round under 2^-18 of that sum, the
+// two additions under 2^-22), so the running key may start at the largest key
+// of that distance: the guessed centroid's own key is not above it.
+// order (optional): a permutation of the rows, the order they are taken in.
+// Sorted by the guesses, the 32 rows of a block all stop at the same one or two
+// of the centroid blocks; in row order nearly half of the blocks stop some row.
+// Measured at 40 x 75600 rows, 2048 centroids: 1.2 ms in the general form, 0.81
+// without a guess, 0.54 with guess and order; 8 x 32760 113 -> 78 us.
+// ---------------------------------------------------------------------------
+#define FA_WAVES 8
+#define FA_CHUNK 512
+template <int RB>
+__global__ __launch_bounds__(FA_WAVES * 64) void fast_assign32_kernel(
+    const uint16_t* __restrict__ X, const uint16_t* __restrict__ cen, int32_t* labels, int N, int C,
+    int ibits, const int32_t* guess, const int32_t* __restrict__ order) {
+  constexpr int D = 32;
+  __shared__ __attribute__((aligned(16))) uint16_t sC[FA_CHUNK * D];
+  __shared__ __attribute__((aligned(16))) float sN[FA_CHUNK];
+  const int h = blockIdx.y;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int jl = lane & 31, hh = lane >> 5;
+  const int Cp = (C + 31) & ~31;
+  const int kmask = -(1 << ibits);
+  const uint16_t* xh = X + (size_t)h * N * D;
+  const uint16_t* ch = cen + (size_t)h * C * D;
+  const int rbase = blockIdx.x * (FA_WAVES * 32 * RB) + wave * 32 * RB + jl;
+  u32x4 bx[RB][2];
+  float xsq[RB];
+  int best[RB];
+  auto row_of = [&](int pos) { return order && pos < N ? order[(size_t)h * N + pos] : pos; };
+#pragma unroll
+  for (int k = 0; k < RB; ++k) {
+    const int row = row_of(rbase + 32 * k);
+    const bool ok = row < N;
+    float xs = 0.f;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      bx[k][s] = u32x4{0u, 0u, 0u, 0u};
+      if (ok) bx[k][s] = *(const u32x4*)(xh + (size_t)row * D + 16 * s + 8 * hh);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const float a = h2f((uint16_t)(bx[k][s][t] & 0xffff)), b = h2f((uint16_t)(bx[k][s][t] >> 16));
+        xs += a * a + b * b;
+      }
+    }
+    xsq[k] = half_sum(xs);
+    best[k] = 0x7fffffff;
+    const int g = (ok && guess) ? guess[(size_t)h * N + row] : -1;
+    const bool have = g >= 0 && g < C;
+    float part = 0.f, mag = 0.f, cn = 0.f;
+    if (have) {
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const u32x4 cv = *(const u32x4*)(ch + (size_t)g * D + 16 * s + 8 * hh);
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            const float x = h2f((uint16_t)(bx[k][s][t] >> (16 * e)));
+            const float cc = h2f((uint16_t)(cv[t] >> (16 * e)));
+            part = fmaf(x, cc, part);
+            mag = fmaf(fabsf(x), fabsf(cc), mag);
+            cn = fmaf(cc, cc, cn);
+          }
+      }
+    }
+    part = half_sum(part);
+    mag = half_sum(mag);
+    cn = half_sum(cn);
+    const float ub = xsq[k] + (cn - 2.0f * part) + 0x1p-15f * (xsq[k] + cn + 2.0f * mag) + 0x1p-120f;
+    if (have && ub >= 0.f && ub < 0x1p126f) best[k] = __builtin_bit_cast(int, ub) | ~kmask;
+  }
+  auto mn = [](float a, float b) { return __builtin_elementwise_minimum(a, b); };
+  for (int c0 = 0; c0 < Cp; c0 += FA_CHUNK) {
+    const int nc = Cp - c0 < FA_CHUNK ? Cp - c0 : FA_CHUNK;
+    if (c0 > 0) __syncthreads();  // every wave is done with the previous chunk
+    // a thread stages one centroid (16-byte chunk c of row r at c ^ ((r >> 2) & 3))
+    // and sums its norm over the dims in order; padding: zeros, norm inf
+    if (tid < nc) {
+      const bool in = c0 + tid < C;
+      const u32x4* cp = (const u32x4*)(ch + (size_t)(c0 + (in ? tid : 0)) * D);
+      float sum = 0.f;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const u32x4 v = in ? cp[c] : u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const float a = h2f((uint16_t)(v[t] & 0xffff)), b = h2f((uint16_t)(v[t] >> 16));
+          sum = sum + a * a;
+          sum = sum + b * b;
+        }
+        ((u32x4*)sC)[tid * 4 + (c ^ ((tid >> 2) & 3))] = v;
+      }
+      sN[tid] = in ? sum : __builtin_inff();
+    }
+    __syncthreads();
+    for (int cb = 0; cb < nc / 32; ++cb) {
+      const int r = cb * 32 + jl;
+      const bool part = c0 + cb * 32 + 32 > C;  // wave-uniform: the block holds padding
+      const u32x4* crow = (const u32x4*)sC + r * 4;
+      const u32x4 a0 = crow[(0 + hh) ^ ((r >> 2) & 3)];
+      const u32x4 a1 = crow[(2 + hh) ^ ((r >> 2) & 3)];
+      f32x4 cn[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) cn[q] = *(const f32x4*)(sN + cb * 32 + 8 * q + 4 * hh);
+#pragma unroll
+      for (int k = 0; k < RB; ++k) {
+        f32x16 acc = Mfma<F16T>::run(a0, bx[k][0], zero16());
+        acc = Mfma<F16T>::run(a1, bx[k][1], acc);
+        float t[16];
+#pragma unroll
+        for (int a = 0; a < 16; ++a) t[a] = cn[a / 4][a % 4] - 2.0f * acc[a];
+        float t8[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) t8[i] = mn(t[2 * i], t[2 * i + 1]);
+        const float d2 =
+            xsq[k] + mn(mn(mn(t8[0], t8[1]), mn(t8[2], t8[3])), mn(mn(t8[4], t8[5]), mn(t8[6], t8[7])));
+        const bool skip = d2 >= 0.f && (__builtin_bit_cast(int, d2) & kmask) > (best[k] & kmask);
+        if (__ballot(!skip) != 0ull) {  // wave-uniform
+          // the index bits below 32 first, the block's base (a multiple of 32)
+          // once at the end: both lie under the mask, so the order is the same
+          int kb = 0x7fffffff;
+          if (part) {
+            asm volatile("" ::: "memory");  // a branch of its own, not selects
+#pragma unroll
+            for (int a = 0; a < 16; ++a) {
+              const int key = (__builtin_bit_cast(int, xsq[k] + t[a]) & kmask) | (8 * (a / 4) + (a % 4));
+              const bool pad = c0 + cb * 32 + 4 * hh + 8 * (a / 4) + (a % 4) >= C;
+              kb = !pad && key < kb ? key : kb;
+            }
+          } else {
+#pragma unroll
+            for (int a = 0; a < 16; ++a) {
+              const int key = (__builtin_bit_cast(int, xsq[k] + t[a]) & kmask) | (8 * (a / 4) + (a % 4));
+              kb = key < kb ? key : kb;
+            }
+          }
+          kb |= c0 + cb * 32 + 4 * hh;
+          best[k] = kb < best[k] ? kb : best[k];
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < RB; ++k) {
+    const int o = (int)half_partner((uint32_t)best[k]);
+    const int b = o < best[k] ? o : best[k];
+    const int row = row_of(rbase + 32 * k);
+    if (row < N && hh == 0) labels[(size_t)h * N + row] = b & ~kmask;
+  }
+}
+
+// Row blocks per wave (LDS reads per distance fall with them): four while the
+// launch still has four work-groups per CU, fewer when it would not fill the
+// chip.
+static void launch_fast_assign32(const void* x, const void* c, int32_t* labels, int H, int N, int C,
+                                 int ibits, const int32_t* guess, const int32_t* order,
+                                 hipStream_t st) {
+#define FA_LAUNCH(RB)                                                                            \
+  hipLaunchKernelGGL(fast_assign32_kernel<RB>, dim3(cdiv(N, FA_WAVES * 32 * RB), H),             \
+                     dim3(FA_WAVES * 64), 0, st, (const uint16_t*)x, (const uint16_t*)c, labels, \
+                     N, C, ibits, guess, order)
+  if ((long long)H * cdiv(N, FA_WAVES * 128) >= 1024)
+    FA_LAUNCH(4);
+  else if ((long long)H * cdiv(N, FA_WAVES * 64) >= 512)
+    FA_LAUNCH(2);
+  else
+    FA_LAUNCH(1);
+#undef FA_LAUNCH
+}
+
+// ---------------------------------------------------------------------------
 // k-means assignment at rank 32: d = |c|^2 + x.(-2c),
 // argmin, ties to the lowest index.  One 8-wave work-group per 1024 rows, four
 // 32-row blocks per wave, so every centroid fragment and norm read from LDS
@@ -455,8 +644,10 @@ __global__ __launch_bounds__(256) void fixed_mean_kernel(const uint16_t* __restr
 // each) and V (two dims per lane) in sorted row order; V_sorted rows; ck2.
 // perm == nullptr: rows are already cluster ordered (V_sorted input).
 // ---------------------------------------------------------------------------
+// MEAN: vsum and ck2 hold the cluster's means of V (over max(n, 1)) and KU (the
+// fused_update_vstats outputs), and cmax is not written.
 #define KG_UNR 16
-template <typename T>
+template <typename T, bool MEAN>
 __global__ __launch_bounds__(256) void key_gather_kernel(
     const uint16_t* __restrict__ KU, const uint16_t* __restrict__ V,
     const int32_t* __restrict__ perm, const int32_t* __restrict__ counts,
@@ -529,11 +720,17 @@ __global__ __launch_bounds__(256) void key_gather_kernel(
   else
     run(std::false_type{});
   float* vo = vsum + ((size_t)h * C + c) * 128 + 2 * l;
-  vo[0] = v0;
-  vo[1] = v1;
-  // the cluster's largest |value sum|, for the per-head scale lam
-  const float mx = wave_max(fmaxf(fabsf(v0), fabsf(v1)));
-  if (l == 0) cmax[(size_t)h * C + c] = mx;
+  if constexpr (MEAN) {
+    const float d = n ? (float)n : 1.0f;
+    vo[0] = v0 / d;
+    vo[1] = v1 / d;
+  } else {
+    vo[0] = v0;
+    vo[1] = v1;
+    // the cluster's largest |value sum|, for the per-head scale lam
+    const float mx = wave_max(fmaxf(fabsf(v0), fabsf(v1)));
+    if (l == 0) cmax[(size_t)h * C + c] = mx;
+  }
   if (ck2 && l < 16) {
     const size_t o = ((size_t)h * C + c) * KM_R + 2 * l;
     ck2[o] = n ? ax0 / (float)n : h2f(ck0[o]);
@@ -663,7 +860,7 @@ static void launch_key_gather(const void* KU, const void* V, const int32_t* perm
                               const int32_t* counts, const int32_t* cbase, const void* ck0,
                               float* ck2, void* V_sorted, float* vsum, float* cmax, int H, int N,
                               int C, long long svh, long long svn, hipStream_t st) {
-  hipLaunchKernelGGL(key_gather_kernel<T>, dim3(cdiv(C, 4), H), dim3(256), 0, st,
+  hipLaunchKernelGGL((key_gather_kernel<T, false>), dim3(cdiv(C, 4), H), dim3(256), 0, st,
                      (const uint16_t*)KU, (const uint16_t*)V, perm, counts, cbase,
                      (const uint16_t*)ck0, ck2, (uint16_t*)V_sorted, vsum, cmax, N, C, svh, svn);
 }
@@ -842,8 +1039,7 @@ extern "C" int t2t_fast_assign(const void* x, const void* c, int32_t* labels, in
   while ((1 << ibits) < C) ++ibits;
   const dim3 g(cdiv(N, 128), H);
   if (D == 32)
-    hipLaunchKernelGGL((fast_assign_kernel<32>), g, dim3(256), 0, st, (const uint16_t*)x,
-                       (const uint16_t*)c, labels, N, C, ibits);
+    launch_fast_assign32(x, c, labels, H, N, C, ibits, nullptr, nullptr, st);
   else if (D == 64)
     hipLaunchKernelGGL((fast_assign_kernel<64>), g, dim3(256), 0, st, (const uint16_t*)x,
                        (const uint16_t*)c, labels, N, C, ibits);
@@ -875,48 +1071,52 @@ extern "C" size_t t2t_det_update_ws_bytes(int H, int N, int C) {
 }
 
 // ---------------------------------------------------------------------------
-// fp32 centroid means and per-cluster value means (the reference's
-// fused_update_vstats): one wave per cluster sums its rows in sorted order,
-// fp32 and sequential per dim (lanes 0..31: one dim of x each; all lanes: two
-// dims of v each).  Empty clusters: centroid = fp32(old), value mean = 0.
+// fp32 centroid means (the reference's fused_update_vstats without values):
+// 16 lanes per cluster, two dims each, sum its rows in sorted order, fp32 and
+// sequential per dim; an empty cluster keeps fp32(old).  The cluster's row
+// indices are read 16 at a time and passed around within the 16 lanes, so
+// each lane has 16 row loads in flight.  (One wave per cluster, its half idle
+// and waiting on every row before the next, took 318 us on average over the
+// 512 and 2048 cluster calls at 40 x 75600 rows.)  out16: fp16 means instead.
+// With values, key_gather_kernel<T, true> sums both.
 // ---------------------------------------------------------------------------
-template <typename T>
+#define SM_UNR 16
 __global__ __launch_bounds__(256) void seg_mean_kernel(
-    const uint16_t* __restrict__ X, const uint16_t* __restrict__ V,
-    const int32_t* __restrict__ perm, const int32_t* __restrict__ counts,
-    const int32_t* __restrict__ cbase, const uint16_t* __restrict__ old,
-    float* __restrict__ cent, float* __restrict__ vmean, int N, int C) {
+    const uint16_t* __restrict__ X, const int32_t* __restrict__ perm,
+    const int32_t* __restrict__ counts, const int32_t* __restrict__ cbase,
+    const uint16_t* old, float* __restrict__ cent, uint16_t* out16, int N, int C) {
   const int h = blockIdx.y;
-  const int l = threadIdx.x & 63;
-  const int c = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (c >= C) return;
-  const int n = counts[(size_t)h * C + c];
-  const int32_t* ph = perm + (size_t)h * N + cbase[(size_t)h * C + c];
-  const uint16_t* xh = X + (size_t)h * N * KM_R;
-  const uint32_t* vh = V ? (const uint32_t*)(V + (size_t)h * N * 128) : nullptr;
-  float ax = 0.f, v0 = 0.f, v1 = 0.f;
-  for (int i0 = 0; i0 < n; i0 += 64) {
-    const int myrow = i0 + l < n ? ph[i0 + l] : 0;
-    const int m = n - i0 < 64 ? n - i0 : 64;
-    for (int i = 0; i < m; ++i) {
-      const int rw = __builtin_amdgcn_readlane(myrow, i);
-      if (l < KM_R) ax += h2f(xh[(size_t)rw * KM_R + l]);
-      if (vh) {
-        const uint32_t u = vh[(size_t)rw * 64 + l];
-        v0 += T::to_f((uint16_t)(u & 0xffff));
-        v1 += T::to_f((uint16_t)(u >> 16));
+  const int l = threadIdx.x & 15, q0 = threadIdx.x & 48;
+  const int c = blockIdx.x * 16 + (threadIdx.x >> 4);
+  const bool in = c < C;
+  const int n = in ? counts[(size_t)h * C + c] : 0;
+  const int32_t* ph = perm + (size_t)h * N + (in ? cbase[(size_t)h * C + c] : 0);
+  const uint32_t* xh = (const uint32_t*)(X + (size_t)h * N * KM_R) + l;
+  float ax0 = 0.f, ax1 = 0.f;
+  int nxt = l < n ? ph[l] : 0;
+  // the wave runs to its longest cluster; a finished one loads row 0 unused
+  for (int i0 = 0; __ballot(i0 < n) != 0ull; i0 += SM_UNR) {
+    const int my = nxt;
+    nxt = i0 + SM_UNR + l < n ? ph[i0 + SM_UNR + l] : 0;
+    uint32_t v[SM_UNR];
+#pragma unroll
+    for (int u = 0; u < SM_UNR; ++u)
+      v[u] = xh[(size_t)__shfl(my, q0 + u, 64) * (KM_R / 2)];
+#pragma unroll
+    for (int u = 0; u < SM_UNR; ++u)
+      if (i0 + u < n) {
+        ax0 += h2f((uint16_t)(v[u] & 0xffff));
+        ax1 += h2f((uint16_t)(v[u] >> 16));
       }
-    }
   }
-  if (l < KM_R) {
-    const size_t o = ((size_t)h * C + c) * KM_R + l;
-    cent[o] = n ? ax / (float)n : h2f(old[o]);
-  }
-  if (vh) {
-    const float d = n ? (float)n : 1.0f;
-    float* vo = vmean + ((size_t)h * C + c) * 128 + 2 * l;
-    vo[0] = v0 / d;
-    vo[1] = v1 / d;
+  if (!in) return;
+  const size_t o = ((size_t)h * C + c) * KM_R + 2 * l;
+  const float m0 = n ? ax0 / (float)n : h2f(old[o]), m1 = n ? ax1 / (float)n : h2f(old[o + 1]);
+  if (out16) {
+    *(uint32_t*)(out16 + o) = (uint32_t)f2h(opaque(m0)) | ((uint32_t)f2h(opaque(m1)) << 16);
+  } else {
+    cent[o] = m0;
+    cent[o + 1] = m1;
   }
 }
 
@@ -939,16 +1139,70 @@ extern "C" int t2t_fused_update_vstats(const void* x, const int32_t* labels, con
   hipStream_t st = (hipStream_t)stream;
   DetWs w = det_layout(H, N, C, ws);
   KM_CHECK(run_sort(labels, counts, w.cbase, w.perm, w.chist, H, N, C, st));
+  const long long vs = (long long)N * 128;
   const dim3 g(cdiv(C, 4), H);
-  if (v && v_dtype == T2T_BF16)
-    hipLaunchKernelGGL(seg_mean_kernel<BF16T>, g, dim3(256), 0, st, (const uint16_t*)x,
+  if (!v)
+    hipLaunchKernelGGL(seg_mean_kernel, dim3(cdiv(C, 16), H), dim3(256), 0, st, (const uint16_t*)x,
+                       w.perm, counts, w.cbase, (const uint16_t*)old, cent, (uint16_t*)nullptr, N, C);
+  else if (v_dtype == T2T_BF16)
+    hipLaunchKernelGGL((key_gather_kernel<BF16T, true>), g, dim3(256), 0, st, (const uint16_t*)x,
                        (const uint16_t*)v, w.perm, counts, w.cbase, (const uint16_t*)old, cent,
-                       vmean, N, C);
+                       (uint16_t*)nullptr, vmean, (float*)nullptr, N, C, vs, 128ll);
   else
-    hipLaunchKernelGGL(seg_mean_kernel<F16T>, g, dim3(256), 0, st, (const uint16_t*)x,
+    hipLaunchKernelGGL((key_gather_kernel<F16T, true>), g, dim3(256), 0, st, (const uint16_t*)x,
                        (const uint16_t*)v, w.perm, counts, w.cbase, (const uint16_t*)old, cent,
-                       vmean, N, C);
+                       (uint16_t*)nullptr, vmean, (float*)nullptr, N, C, vs, 128ll);
   T2T_LAUNCH_CHECK("fused_update_vstats");
+  return T2T_OK;
+}
+
+// ---- warm Lloyd iterations (init_state) ----
+struct LloydWs {
+  int32_t* labels;
+  int32_t* counts;
+  DetWs sort;
+  size_t total;
+};
+static LloydWs lloyd_layout(int H, int N, int C, void* base) {
+  WsCarver w(base);
+  LloydWs l;
+  l.labels = w.take<int32_t>((size_t)H * N);
+  l.counts = w.take<int32_t>((size_t)H * C);
+  l.sort = det_layout(H, N, C, base ? (char*)base + w.off : nullptr);
+  l.total = w.off + l.sort.total;
+  return l;
+}
+
+extern "C" size_t t2t_lloyd_ws_bytes(int H, int N, int C) {
+  return lloyd_layout(H, N, C, nullptr).total;
+}
+
+extern "C" int t2t_lloyd(const void* x, void* cen, int iters, int H, int N, int C, int D, void* ws,
+                         size_t ws_bytes, void* stream) {
+  T2T_REQUIRE(x && cen, "lloyd: null pointer");
+  T2T_REQUIRE(H > 0 && N > 0 && C >= 1 && C <= KM_MAXC && iters >= 0, "lloyd: H=%d N=%d C=%d iters=%d",
+              H, N, C, iters);
+  T2T_REQUIRE(D == KM_R, "lloyd: D=%d (built for %d)", D, KM_R);
+  const size_t need = t2t_lloyd_ws_bytes(H, N, C);
+  if (!ws || ws_bytes < need) {
+    t2t_set_error("lloyd: workspace %zu < %zu bytes", ws_bytes, need);
+    return T2T_ERR_WORKSPACE;
+  }
+  hipStream_t st = (hipStream_t)stream;
+  LloydWs w = lloyd_layout(H, N, C, ws);
+  int ibits = 1;
+  while ((1 << ibits) < C) ++ibits;
+  for (int i = 0; i < iters; ++i) {
+    // an iteration's labels start from the previous one's, rows in their order
+    launch_fast_assign32(x, cen, w.labels, H, N, C, ibits, i ? w.labels : nullptr,
+                         i ? w.sort.perm : nullptr, st);
+    KM_CHECK(run_sort(w.labels, w.counts, w.sort.cbase, w.sort.perm, w.sort.chist, H, N, C, st));
+    // in place: a cluster's old centroid is read by its own lanes alone
+    hipLaunchKernelGGL(seg_mean_kernel, dim3(cdiv(C, 16), H), dim3(256), 0, st, (const uint16_t*)x,
+                       w.sort.perm, w.counts, w.sort.cbase, (const uint16_t*)cen, (float*)nullptr,
+                       (uint16_t*)cen, N, C);
+  }
+  T2T_LAUNCH_CHECK("lloyd");
   return T2T_OK;
 }
 

@@ -299,11 +299,9 @@ class MaskedStepDeploy:
         qidx = torch.randperm(N, generator=g)[: self.CQ].sort().values.to(self.dev)
         ck = KU[:, kidx, :].contiguous()
         cq = QU[:, qidx, :].contiguous()
-        for _ in range(warm_iters):
-            cent, _, _ = ops.fused_update_vstats(KU, fast_assign(KU, ck), ck, check_labels=False)
-            ck = cent.to(torch.float16)
-            cent, _, _ = ops.fused_update_vstats(QU, fast_assign(QU, cq), cq, check_labels=False)
-            cq = cent.to(torch.float16)
+        iters = len(range(warm_iters))
+        ops.lloyd(KU, ck, iters)
+        ops.lloyd(QU, cq, iters)
         torch.cuda.synchronize(self.dev)
         return {"Uq": Uq, "Uk": Uk, "ck": ck.contiguous(), "cq": cq.contiguous()}
 

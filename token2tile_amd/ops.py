@@ -588,6 +588,19 @@ def fused_update_vstats(x, labels, old, v=None, stream=None, check_labels=True):
     return cent, counts, vmean
 
 
+def lloyd(x, cen, iters, stream=None):
+    """``iters`` warm Lloyd iterations in place on cen [H, C, 32] fp16: the
+    labels of fast_assign_labels and the means of fused_update_vstats in fp16."""
+    H, N, D = x.shape
+    C = cen.shape[1]
+    dev = _dev(x)
+    _check(x, (H, N, D), _f16, "x", dev)
+    _check(cen, (H, C, D), _f16, "cen", dev)
+    ws = _ws(size_query("t2t_lloyd_ws_bytes", H, N, C), dev)
+    call("t2t_lloyd", x, cen, int(iters), H, N, C, D, ws, ws.numel(), stream_handle(stream))
+    return cen
+
+
 def gram(x, stream=None):
     """x^T x / N per head in fp64: [H, D, D]."""
     H, N, D = x.shape
