@@ -349,6 +349,19 @@ size_t t2t_gram_ws_bytes(int H, int N, int D);
 int t2t_gram(const void* x, int x_dtype, double* G, int H, int N, int D, void* ws,
              size_t ws_bytes, void* stream);
 
+/* t2t_gram of a strided [H, N, D] view (element strides, row stride >= D);
+ * nonfinite (may be NULL) [H] int32: 1 where the head holds an inf or NaN. */
+int t2t_gram_strided(const void* x, int x_dtype, long long x_head_stride, long long x_row_stride,
+                     double* G, int32_t* nonfinite, int H, int N, int D, void* ws,
+                     size_t ws_bytes, void* stream);
+/* Projection-fit factors: L [H, D, D] = lower Cholesky factor of Mk (zeros
+ * above the diagonal; undefined where Mk is not positive definite); small
+ * [2 H] int32: 1 where Mq[h] (first H) or Mk[h] (last H) has an eigenvalue
+ * not above floor.  D <= 128.  Takes the place of the two symmetric
+ * eigensolutions behind the square roots of operator/deploy_step.py:138-143. */
+int t2t_fit_chol(const double* Mq, const double* Mk, double* L, int32_t* small, int H, int D,
+                 double floor, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

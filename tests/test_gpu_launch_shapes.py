@@ -81,3 +81,60 @@ def test_lloyd_equals_separate_calls(dev, H, N, C):
         want = ops.fused_update_vstats(x, lab, want)[0].half()
     assert torch.equal(ops.lloyd(x, cen.clone(), 3), want)
     assert torch.equal(ops.lloyd(x, cen.clone(), 0), cen)
+
+
+# rows that end inside a staged step and a k-step, several splits, the element
+# path (D not 128, unaligned or odd strides), a token-major view
+@pytest.mark.parametrize("H,N,D,view", [(1, 3, 128, ""), (2, 257, 128, ""), (3, 5001, 128, "token"),
+                                        (2, 700, 128, "odd"), (2, 300, 100, ""), (1, 65, 16, "")])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_gram_strided(dev, H, N, D, view, dtype):
+    """fp64 Gram of every layout; products of fp16 values are exact, so only
+    the order of the fp64 sum differs from the reference's."""
+    from token2tile_amd import ops
+    gen = torch.Generator(device=dev).manual_seed(N + D)
+    x = torch.randn(H, N, D, generator=gen, device=dev).to(dtype)
+    if view == "token":
+        x = x.transpose(0, 1).contiguous().transpose(0, 1)
+    elif view == "odd":
+        x = torch.nn.functional.pad(x, (3, 2))[:, :, 3:3 + D]
+    flag = torch.full((H,), -1, dtype=torch.int32, device=dev)
+    G = ops.gram_strided(x, flag)
+    xd = x.half().double().cpu()
+    want = xd.transpose(1, 2) @ xd / N
+    bound = 2.0 ** -52 * N * (xd.abs().transpose(1, 2) @ xd.abs() / N)
+    assert bool(((G.cpu() - want).abs() <= bound).all())
+    assert torch.equal(G, G.transpose(1, 2)) and not flag.any()
+    x[H - 1, N - 1, D - 1] = float("-inf")
+    ops.gram_strided(x, flag)
+    assert flag.tolist() == [0] * (H - 1) + [1]
+
+
+@pytest.mark.parametrize("D", [8, 100, 128])
+def test_projection_fit_forms(dev, D):
+    """The Cholesky form against the square-root form on the same Grams (fp64,
+    up to the sign of a column pair), and its fall-back to the latter."""
+    from token2tile_amd import deploy_step as DS, ops
+    gen = torch.Generator(device=dev).manual_seed(D)
+    q, k = (torch.randn(3, 2000, D, generator=gen, device=dev) / D ** 0.5
+            * torch.linspace(0.2, 3.0, D, device=dev) for _ in range(2))
+    Mq, Mk = (ops.gram_strided(t.half()) for t in (q, k))
+    small = torch.empty(2, 3, dtype=torch.int32, device=dev)
+    L = ops.fit_chol(Mq, Mk, 1e-8, small)
+    assert not small.any()
+    assert float((L @ L.transpose(1, 2) - Mk).abs().max()) <= 1e-13 * float(Mk.abs().max())
+    r = min(32, D)
+    a, b = DS._fit_chol(Mq, Mk, L, r), DS._fit_eigh(Mq, Mk, r)
+    sign = (a[0] * b[0]).sum(1, keepdim=True).sign()
+    for x, y in zip(a, b):
+        assert float((x * sign - y).abs().max()) <= 1e-7 * float(y.abs().max())
+    Mq[1, :, 0] = Mq[1, 0, :] = 0.0            # a zero eigenvalue in one head of q
+    Mk[2, -1, :] = Mk[2, :, -1] = 0.0
+    Mk[2, -1, -1] = 1e-9                       # and one under the floor in one of k
+    ops.fit_chol(Mq, Mk, 1e-8, small)
+    assert small.tolist() == [[0, 1, 0], [0, 0, 1]]
+    qz = q.half().clone()
+    qz[:, :, 0] = 0                            # the operator takes the other form
+    Uq, Uk = DS.online_u(qz, k.half(), r)
+    Eq, Ek = DS._fit_eigh(*(ops.gram_strided(t) for t in (qz, k.half())), r)
+    assert torch.equal(Uq, Eq.float()) and torch.equal(Uk, Ek.float())

@@ -9,7 +9,7 @@ arguments.
 from __future__ import annotations
 
 import ctypes
-from ctypes import c_float, c_int, c_longlong, c_size_t, c_void_p
+from ctypes import c_double, c_float, c_int, c_longlong, c_size_t, c_void_p
 from pathlib import Path
 
 import torch
@@ -92,6 +92,9 @@ SIGNATURES = {
     "t2t_lloyd": (c_int, [_P, _P, c_int, c_int, c_int, c_int, c_int, _P, c_size_t, _P]),
     "t2t_gram_ws_bytes": (c_size_t, [c_int, c_int, c_int]),
     "t2t_gram": (c_int, [_P, c_int, _P, c_int, c_int, c_int, _P, c_size_t, _P]),
+    "t2t_gram_strided": (c_int, [_P, c_int, c_longlong, c_longlong, _P, _P, c_int, c_int, c_int, _P,
+                                 c_size_t, _P]),
+    "t2t_fit_chol": (c_int, [_P, _P, _P, _P, c_int, c_int, c_double, _P]),
 }
 
 _lib = None

@@ -360,93 +360,155 @@ extern "C" int t2t_score(const void* QU, const void* cks, void* gl, int H, int N
 // ---------------------------------------------------------------------------
 // S0: G = x^T x / N in fp64 (products of fp16 values are exact in fp64; the
 // sum runs over rows in order, so the result is deterministic).
-// grid (tiles, H); each work-group owns a 64 x 64 output tile.
 // ---------------------------------------------------------------------------
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 #define GR_ROWS 64      // rows staged per step
+#define GR_PITCH 144    // floats per staged row: the four rows of a fragment read start 16 banks apart
 #define GR_MAXSPLIT 64  // row splits per head (partial Grams in the workspace)
 
+// the 36 blocks (i <= j) of the upper triangle of 8 x 8 blocks of 16 columns,
+// nine per wave
+struct GrPairs {
+  int i[36], j[36];
+};
+constexpr GrPairs gr_pairs() {
+  GrPairs p{};
+  int n = 0;
+  for (int i = 0; i < 8; ++i)
+    for (int j = i; j < 8; ++j, ++n) {
+      p.i[n] = i;
+      p.j[n] = j;
+    }
+  return p;
+}
+__device__ constexpr GrPairs GR_PAIR = gr_pairs();
+
 // Partial Gram products on fp64 MFMA (v_mfma_f64_16x16x4_f64).  Block (s, h)
-// sums rows [s R, s R + R) of head h; wave w owns the 64 x 64 quadrant
-// (w / 2, w % 2) of the D x D result as 4 x 4 blocks of 16 x 16.  Rows are
-// staged through LDS as fp32 (exact for fp16 values; bf16 is rounded to fp16
-// first, as the reference's backend casts to fp16).  For a k-step of four
-// rows, lane l holds x[n + l / 16][c + l % 16] as both the A (Xt, 16 x 4)
-// and the B (X, 4 x 16) fragment of column block c, and the 16 x 16 result
-// block keeps G[c_i + l / 16 + 4 r][c_j + l % 16] in register r of lane l
-// (rows interleaved by four, as measured on the GPU).
+// sums rows [s R, s R + R) of head h; the result is symmetric, so only the
+// 36 blocks on and above the diagonal are formed, nine per wave (40 x 75600 x
+// 128: 2.83 ms with all 64 blocks, 1.16 with these, 48 TFLOP/s where a large
+// fp64 matrix product reaches 61).  Rows are staged through LDS as fp32 (exact for fp16 values; bf16 is
+// rounded to fp16 first, as the reference's backend casts to fp16), the next
+// rows' loads in flight meanwhile.  For a k-step of four rows, lane l holds
+// x[n + l / 16][c + l % 16] as both the A (Xt, 16 x 4) and the B (X, 4 x 16)
+// fragment of column block c, and the 16 x 16 result block keeps
+// G[c_i + l / 16 + 4 r][c_j + l % 16] in register r of lane l (rows
+// interleaved by four, as measured on the GPU).
 // Products of fp16 values are exact in fp64, and each output sums its rows in
 // a fixed order, so the result does not depend on the launch.
-template <typename T>
+// bad[s, h] = 1 when a row of the block holds an inf or NaN.
+// VEC: D == 128 and 16-byte aligned rows (16-byte loads); else element loads.
+template <typename T, bool VEC>
 __global__ __launch_bounds__(256) void gram_kernel(const uint16_t* __restrict__ x,
-                                                   double* __restrict__ part, int N, int D, int R) {
-  __shared__ float sx[GR_ROWS][128 + 4];
+                                                   double* __restrict__ part, int32_t* __restrict__ bad,
+                                                   int N, int D, int R, long long sxh, long long sxn) {
+  __shared__ __attribute__((aligned(16))) float sx[GR_ROWS][GR_PITCH];
+  __shared__ int sbad;
   const int s = blockIdx.x, h = blockIdx.y, H = gridDim.y;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int qi = w >> 1, qj = w & 1;
-  const bool act = qi * 64 < D && qj * 64 < D;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r0 = s * R;
   const int r1 = r0 + R < N ? r0 + R : N;
-  f64x4 acc[4][4];
+  const uint16_t* xh = x + (size_t)h * sxh;
+  constexpr uint32_t EXPM = T::code == T2T_BF16 ? 0x7f80u : 0x7c00u;
+  bool nf = false;
+  auto val = [&](uint32_t u) {
+    nf |= (u & EXPM) == EXPM;
+    return T::code == T2T_BF16 ? h2f(bf2h((uint16_t)u)) : h2f((uint16_t)u);
+  };
+  // 16-byte chunk i of a staged step: row i / 16, columns 8 (i % 16) ..
+  u32x4 nx[4];
+  auto load = [&](int n0) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
-  const uint16_t* xh = x + (size_t)h * N * D;
-  const int kr = lane >> 4, kc = lane & 15;
-  for (int n0 = r0; n0 < r1; n0 += GR_ROWS) {
-    __syncthreads();
-    for (int i = tid; i < GR_ROWS * 128; i += 256) {
-      const int rr = i >> 7, cc = i & 127;
-      const int n = n0 + rr;
-      float v = 0.f;
-      if (n < r1 && cc < D) {
-        const uint16_t u = xh[(size_t)n * D + cc];
-        v = (T::code == T2T_BF16) ? h2f(bf2h(u)) : h2f(u);
-      }
-      sx[rr][cc] = v;
+    for (int i = 0; i < 4; ++i) {
+      const int n = n0 + (tid >> 4) + 16 * i;
+      nx[i] = u32x4{0u, 0u, 0u, 0u};
+      if (n < r1) nx[i] = *(const u32x4*)(xh + (size_t)n * sxn + 8 * (tid & 15));
     }
-    __syncthreads();
-    if (act) {
+  };
+  if (tid == 0) sbad = 0;
+  if constexpr (VEC) load(r0);
+  auto run = [&](auto W) {
+    constexpr int P0 = 9 * decltype(W)::value;
+    f64x4 acc[9];
+#pragma unroll
+    for (int p = 0; p < 9; ++p) acc[p] = f64x4{0.0, 0.0, 0.0, 0.0};
+    const int kr = lane >> 4, kc = lane & 15;
+    for (int n0 = r0; n0 < r1; n0 += GR_ROWS) {
+      __syncthreads();
+      if constexpr (VEC) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float* o = &sx[(tid >> 4) + 16 * i][8 * (tid & 15)];
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            o[2 * t] = val(nx[i][t] & 0xffffu);
+            o[2 * t + 1] = val(nx[i][t] >> 16);
+          }
+        }
+      } else {
+        for (int i = tid; i < GR_ROWS * 128; i += 256) {
+          const int rr = i >> 7, cc = i & 127;
+          sx[rr][cc] = n0 + rr < r1 && cc < D ? val(xh[(size_t)(n0 + rr) * sxn + cc]) : 0.f;
+        }
+      }
+      __syncthreads();
+      if constexpr (VEC)
+        if (n0 + GR_ROWS < r1) load(n0 + GR_ROWS);
 #pragma unroll 2
       for (int k = 0; k < GR_ROWS; k += 4) {
-        double a[4], b[4];
+        double f[8];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          a[t] = (double)sx[k + kr][64 * qi + 16 * t + kc];
-          b[t] = (double)sx[k + kr][64 * qj + 16 * t + kc];
-        }
+        for (int t = 0; t < 8; ++t) f[t] = (double)sx[k + kr][16 * t + kc];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
+        for (int p = 0; p < 9; ++p)
+          acc[p] = __builtin_amdgcn_mfma_f64_16x16x4f64(f[GR_PAIR.i[P0 + p]], f[GR_PAIR.j[P0 + p]],
+                                                        acc[p], 0, 0, 0);
       }
     }
-  }
-  if (!act) return;
-  double* ph = part + ((size_t)s * H + h) * D * D;
+    double* ph = part + ((size_t)s * H + h) * D * D;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int p = 0; p < 9; ++p)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int gi = 64 * qi + 16 * i + kr + 4 * r, gj = 64 * qj + 16 * j + kc;
-        if (gi < D && gj < D) ph[(size_t)gi * D + gj] = acc[i][j][r];
+        const int gi = 16 * GR_PAIR.i[P0 + p] + kr + 4 * r, gj = 16 * GR_PAIR.j[P0 + p] + kc;
+        if (gi < D && gj < D) ph[(size_t)gi * D + gj] = acc[p][r];
       }
+  };
+  switch (w) {
+    case 0: run(std::integral_constant<int, 0>{}); break;
+    case 1: run(std::integral_constant<int, 1>{}); break;
+    case 2: run(std::integral_constant<int, 2>{}); break;
+    default: run(std::integral_constant<int, 3>{}); break;
+  }
+  if (nf) sbad = 1;  // every writer stores the same value
+  __syncthreads();
+  if (tid == 0) bad[(size_t)s * H + h] = sbad;
 }
 
-// G[h] = (sum over the splits, in split order, of the partial Grams) / N
+// G[h] = (sum over the splits, in split order, of the partial Grams) / N, the
+// blocks below the diagonal mirrored; nonfinite[h] = whether any split saw an
+// inf or NaN
 __global__ __launch_bounds__(256) void gram_reduce_kernel(const double* __restrict__ part,
-                                                          double* __restrict__ G, int S, int H,
-                                                          int N, int D) {
+                                                          const int32_t* __restrict__ bad,
+                                                          double* __restrict__ G,
+                                                          int32_t* __restrict__ nonfinite, int S,
+                                                          int H, int N, int D) {
   const int h = blockIdx.y;
   const int e = blockIdx.x * 256 + threadIdx.x;
+  if (nonfinite && e == 0) {
+    int b = 0;
+    for (int s = 0; s < S; ++s) b |= bad[(size_t)s * H + h];
+    nonfinite[h] = b;
+  }
   if (e >= D * D) return;
+  const int gi = e / D, gj = e % D;
+  if (gi / 16 > gj / 16) return;
   double acc = 0.0;
   for (int s = 0; s < S; ++s) acc += part[((size_t)s * H + h) * D * D + e];
-  G[(size_t)h * D * D + e] = acc / (double)N;
+  acc /= (double)N;
+  G[(size_t)h * D * D + e] = acc;
+  if (gi / 16 < gj / 16) G[(size_t)h * D * D + (size_t)gj * D + gi] = acc;
 }
 
 static int gram_splits(int H, int N) {
@@ -459,13 +521,17 @@ static int gram_splits(int H, int N) {
 
 extern "C" size_t t2t_gram_ws_bytes(int H, int N, int D) {
   if (H <= 0 || N <= 0 || D <= 0) return 0;
-  return t2t_align256((size_t)gram_splits(H, N) * H * D * D * sizeof(double));
+  const size_t S = gram_splits(H, N);
+  return t2t_align256(S * H * D * D * sizeof(double)) + t2t_align256(S * H * sizeof(int32_t));
 }
 
-extern "C" int t2t_gram(const void* x, int x_dtype, double* G, int H, int N, int D, void* ws,
-                        size_t ws_bytes, void* stream) {
+static int gram_impl(const void* x, int x_dtype, long long sxh, long long sxn, double* G,
+                     int32_t* nonfinite, int H, int N, int D, void* ws, size_t ws_bytes,
+                     void* stream) {
   T2T_REQUIRE(x && G, "gram: null pointer");
   T2T_REQUIRE(H > 0 && N > 0 && D > 0 && D <= 128, "gram: H=%d N=%d D=%d", H, N, D);
+  T2T_REQUIRE(sxh >= 0 && sxn >= D, "gram: strides (%lld, %lld)", sxh, sxn);
+  T2T_REQUIRE(x_dtype == T2T_F16 || x_dtype == T2T_BF16, "gram: dtype %d", x_dtype);
   const size_t need = t2t_gram_ws_bytes(H, N, D);
   if (!ws || ws_bytes < need) {
     t2t_set_error("gram: workspace %zu < %zu bytes", ws_bytes, need);
@@ -474,19 +540,97 @@ extern "C" int t2t_gram(const void* x, int x_dtype, double* G, int H, int N, int
   const int S = gram_splits(H, N);
   const int R = ((N + S - 1) / S + 3) / 4 * 4;
   hipStream_t st = (hipStream_t)stream;
-  double* part = (double*)ws;
-  if (x_dtype == T2T_F16)
-    hipLaunchKernelGGL(gram_kernel<F16T>, dim3(S, H), dim3(256), 0, st, (const uint16_t*)x, part,
-                       N, D, R);
-  else if (x_dtype == T2T_BF16)
-    hipLaunchKernelGGL(gram_kernel<BF16T>, dim3(S, H), dim3(256), 0, st, (const uint16_t*)x, part,
-                       N, D, R);
-  else {
-    t2t_set_error("gram: dtype %d", x_dtype);
-    return T2T_ERR_ARG;
+  WsCarver w(ws);
+  double* part = w.take<double>((size_t)S * H * D * D);
+  int32_t* bad = w.take<int32_t>((size_t)S * H);
+  const bool vec = D == 128 && sxn % 8 == 0 && sxh % 8 == 0 && (uintptr_t)x % 16 == 0;
+#define GR_LAUNCH(T, V)                                                                          \
+  hipLaunchKernelGGL((gram_kernel<T, V>), dim3(S, H), dim3(256), 0, st, (const uint16_t*)x, part, \
+                     bad, N, D, R, sxh, sxn)
+  if (x_dtype == T2T_F16) {
+    if (vec) GR_LAUNCH(F16T, true); else GR_LAUNCH(F16T, false);
+  } else {
+    if (vec) GR_LAUNCH(BF16T, true); else GR_LAUNCH(BF16T, false);
   }
-  hipLaunchKernelGGL(gram_reduce_kernel, dim3((D * D + 255) / 256, H), dim3(256), 0, st, part, G,
-                     S, H, N, D);
+#undef GR_LAUNCH
+  hipLaunchKernelGGL(gram_reduce_kernel, dim3((D * D + 255) / 256, H), dim3(256), 0, st, part, bad,
+                     G, nonfinite, S, H, N, D);
   T2T_LAUNCH_CHECK("gram");
+  return T2T_OK;
+}
+
+extern "C" int t2t_gram(const void* x, int x_dtype, double* G, int H, int N, int D, void* ws,
+                        size_t ws_bytes, void* stream) {
+  return gram_impl(x, x_dtype, (long long)N * D, D, G, nullptr, H, N, D, ws, ws_bytes, stream);
+}
+
+extern "C" int t2t_gram_strided(const void* x, int x_dtype, long long x_head_stride,
+                                long long x_row_stride, double* G, int32_t* nonfinite, int H, int N,
+                                int D, void* ws, size_t ws_bytes, void* stream) {
+  return gram_impl(x, x_dtype, x_head_stride, x_row_stride, G, nonfinite, H, N, D, ws, ws_bytes,
+                   stream);
+}
+
+// ---------------------------------------------------------------------------
+// S0: the projection fit's factors.  Work-group (h, 0): L[h] = lower Cholesky
+// factor of Mk[h] (zeros above the diagonal); (h, 1) and (h, 2): whether Mq[h]
+// and Mk[h] have every eigenvalue above floor, that is, whether M - floor I
+// has a Cholesky factor (small[h] / small[H + h] = 1 where not).  The matrix
+// sits in LDS (fp64, 132 KB); 128 dependent column steps, each a scale of the
+// column and a rank-1 update of the rest by 16 waves, bound it by latency, not
+// by the chip: one work-group per matrix, 0.12 ms for 40 heads where each
+// eigensolution it replaces took 2.5 ms.
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(1024) void fit_chol_kernel(const double* __restrict__ Mq,
+                                                        const double* __restrict__ Mk,
+                                                        double* __restrict__ L,
+                                                        int32_t* __restrict__ small, int D,
+                                                        double floor) {
+  __shared__ double A[128 * 129];
+  __shared__ int sbad;
+  const int h = blockIdx.x, H = gridDim.x, kind = blockIdx.y, tid = threadIdx.x;
+  const double* M = (kind == 1 ? Mq : Mk) + (size_t)h * D * D;
+  for (int e = tid; e < D * D; e += 1024) {
+    const int i = e / D, j = e % D;
+    A[i * 129 + j] = M[e] - (kind != 0 && i == j ? floor : 0.0);
+  }
+  if (tid == 0) sbad = 0;
+  __syncthreads();
+  const int ti = tid >> 5, tj = tid & 31;
+  for (int j = 0; j < D; ++j) {
+    const double p = A[j * 129 + j];  // all threads: the same pivot
+    if (!(p > 0.0)) {                 // uniform: not positive definite (or NaN)
+      if (tid == 0) sbad = 1;
+      break;
+    }
+    const double d = sqrt(p), inv = 1.0 / d;
+    __syncthreads();  // every thread has read the pivot
+    if (tid < D - j) A[(j + tid) * 129 + j] = tid == 0 ? d : A[(j + tid) * 129 + j] * inv;
+    __syncthreads();
+    for (int i = j + 1 + ti; i < D; i += 32) {
+      const double li = A[i * 129 + j];
+      for (int k = j + 1 + tj; k <= i; k += 32) A[i * 129 + k] -= li * A[k * 129 + j];
+    }
+    __syncthreads();
+  }
+  __syncthreads();
+  if (kind == 0) {
+    double* Lh = L + (size_t)h * D * D;
+    for (int e = tid; e < D * D; e += 1024) {
+      const int i = e / D, j = e % D;
+      Lh[e] = j <= i ? A[i * 129 + j] : 0.0;
+    }
+  } else if (tid == 0) {
+    small[(kind - 1) * H + h] = sbad;
+  }
+}
+
+extern "C" int t2t_fit_chol(const double* Mq, const double* Mk, double* L, int32_t* small, int H,
+                            int D, double floor, void* stream) {
+  T2T_REQUIRE(Mq && Mk && L && small, "fit_chol: null pointer");
+  T2T_REQUIRE(H > 0 && D > 0 && D <= 128, "fit_chol: H=%d D=%d", H, D);
+  hipLaunchKernelGGL(fit_chol_kernel, dim3(H, 3), dim3(1024), 0, (hipStream_t)stream, Mq, Mk, L,
+                     small, D, floor);
+  T2T_LAUNCH_CHECK("fit_chol");
   return T2T_OK;
 }

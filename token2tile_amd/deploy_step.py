@@ -61,30 +61,16 @@ def _require_finite(**tensors):
                                f"{int(per_head.sum())} non-finite values, in heads {heads}")
 
 
-def online_u(qf, kf, r=32):
-    """Matched rank-r projections Uq, Uk [H, D, r] (fp32) minimising
-    ||Q K^T - (Q Uq)(K Uk)^T||_F (deploy_step.py:122-149).
+_EIG_FLOOR = 1e-8   # least Gram eigenvalue of the fit (smaller ones are raised to it)
 
-    The Gram matrices come from the HIP fp64 Gram kernel (16-bit inputs) or
-    from fp64 matmul for fp32 inputs; the 128 x 128 problems run batched in
-    fp64 on the GPU.  The top-r singular pairs of M = Rq^T Rk come from the
-    eigendecomposition of M^T M (U_r = M V_r / s_r), as in the reference
-    backend's fast initialisation (t2t_attn.py:211-239): a batched
-    symmetric eigensolver is two orders of magnitude faster here than a
-    batched SVD.  Raises RuntimeError on non-finite input.
-    """
-    _require_finite(q=qf, k=kf)
 
-    def gram(x):
-        if x.dtype in (torch.float16, torch.bfloat16):
-            return ops.gram(x.contiguous())
-        xd = x.double()
-        return xd.transpose(1, 2) @ xd / x.shape[1]
-
-    Mq, Mk = gram(qf), gram(kf)
+def _fit_eigh(Mq, Mk, r):
+    """The fit from the symmetric square roots of the Grams, eigenvalues below
+    the floor raised to it: M = Rq Rk, whose top-r singular pairs come from the
+    eigendecomposition of M^T M (U_r = M V_r / s_r)."""
     eq, Vq = _eigh_robust(Mq)
     ek, Vk = _eigh_robust(Mk)
-    eq, ek = eq.clamp_min(1e-8), ek.clamp_min(1e-8)
+    eq, ek = eq.clamp_min(_EIG_FLOOR), ek.clamp_min(_EIG_FLOOR)
     Rq = Vq @ (eq.sqrt().unsqueeze(-1) * Vq.transpose(1, 2))
     Rk = Vk @ (ek.sqrt().unsqueeze(-1) * Vk.transpose(1, 2))
     Rqi = Vq @ (eq.rsqrt().unsqueeze(-1) * Vq.transpose(1, 2))
@@ -95,8 +81,60 @@ def online_u(qf, kf, r=32):
     sr = w[:, -r:].flip(-1).clamp_min(1e-30).sqrt()
     Ur = (M @ Vr) / sr.unsqueeze(1)
     root = sr.sqrt().unsqueeze(1)
-    Uq = (Rqi.transpose(1, 2) @ Ur) * root
-    Uk = (Rki @ Vr) * root
+    return (Rqi.transpose(1, 2) @ Ur) * root, (Rki @ Vr) * root
+
+
+def _fit_chol(Mq, Mk, L, r):
+    """The same fit where every Gram eigenvalue is above the floor.  Any factor
+    of a Gram serves as its root: with Mk = L L^T and Mq = F F^T, M = F^T L has
+    the singular values of Rq Rk and M^T M = L^T Mq L, so one eigensolution is
+    left.  The inverses cancel: Uq = F^-T U S^1/2 = L V S^-1/2 and
+    Uk = L^-T V S^1/2 = Mq Uq S^-1."""
+    MqL = torch.bmm(Mq, L)
+    w, V = _eigh_robust(torch.bmm(L.transpose(1, 2).contiguous(), MqL))
+    Vr = V[:, :, -r:].flip(-1).contiguous()
+    sr = w[:, -r:].flip(-1).clamp_min(1e-30).sqrt().unsqueeze(1)
+    return torch.bmm(L, Vr) * sr.rsqrt(), torch.bmm(MqL, Vr) * sr.pow(-1.5)
+
+
+def online_u(qf, kf, r=32):
+    """Matched rank-r projections Uq, Uk [H, D, r] (fp32) minimising
+    ||Q K^T - (Q Uq)(K Uk)^T||_F (deploy_step.py:122-149).
+
+    The Gram matrices come from the HIP fp64 Gram kernel (16-bit inputs, read
+    in place) or from fp64 matmul for fp32 inputs; the 128 x 128 problems run
+    batched in fp64 on the GPU: a Cholesky factor and one symmetric
+    eigensolution (_fit_chol), or three eigensolutions where a Gram has
+    eigenvalues at the floor (_fit_eigh).  The reference backend's fast
+    initialisation eigensolves in the same way (t2t_attn.py:211-239): a
+    batched symmetric eigensolver is two orders of magnitude faster here than
+    a batched SVD.  Raises RuntimeError on non-finite input."""
+    half = (torch.float16, torch.bfloat16)
+    if not (qf.is_cuda and kf.is_cuda and qf.dtype in half and kf.dtype in half
+            and qf.shape[0] == kf.shape[0]):
+        _require_finite(q=qf, k=kf)
+
+        def gram(x):
+            if x.dtype in half:
+                return ops.gram(x.contiguous())
+            xd = x.double()
+            return xd.transpose(1, 2) @ xd / x.shape[1]
+
+        Uq, Uk = _fit_eigh(gram(qf), gram(kf), r)
+        return Uq.float().contiguous(), Uk.float().contiguous()
+
+    H = qf.shape[0]
+    rows = lambda x: x if x.stride(2) == 1 and x.stride(1) >= x.shape[2] else x.contiguous()  # noqa: E731
+    # heads with non-finite q / k, heads with a small eigenvalue of Mq / Mk:
+    # read back together
+    flags = torch.empty(4, H, dtype=torch.int32, device=qf.device)
+    Mq = ops.gram_strided(rows(qf), flags[0])
+    Mk = ops.gram_strided(rows(kf), flags[1])
+    L = ops.fit_chol(Mq, Mk, _EIG_FLOOR, flags[2:])
+    bad_q, bad_k, *small = (any(f) for f in flags.tolist())
+    if bad_q or bad_k:
+        _require_finite(q=qf, k=kf)
+    Uq, Uk = _fit_eigh(Mq, Mk, r) if any(small) else _fit_chol(Mq, Mk, L, r)
     return Uq.float().contiguous(), Uk.float().contiguous()
 
 
@@ -292,8 +330,10 @@ class MaskedStepDeploy:
         Uq, Uk = online_u(q, k, r)
         Uq = Uq.to(torch.float16).contiguous()
         Uk = Uk.to(torch.float16).contiguous()
-        KU = ops.project(k.contiguous(), Uk)
-        QU = ops.project(q.contiguous(), Uq)
+        # strided views are read in place where the projection can (16-byte rows)
+        rows = lambda x: x if ops.rows_in_place(x) else x.contiguous()  # noqa: E731
+        KU = ops.project(rows(k), Uk)
+        QU = ops.project(rows(q), Uq)
         g = torch.Generator(device="cpu").manual_seed(seed)
         kidx = torch.randperm(N, generator=g)[: self.C].sort().values.to(self.dev)
         qidx = torch.randperm(N, generator=g)[: self.CQ].sort().values.to(self.dev)

@@ -77,6 +77,15 @@ def _rows(t, H, N, D, dtype, name, device):
     return sh, sn
 
 
+def rows_in_place(t):
+    """Whether a [H, N, D] GPU tensor can be passed as a strided view."""
+    try:
+        _rows(t, *t.shape, _HALF, "x", t.device)
+    except ValueError:
+        return False
+    return True
+
+
 def _check_ns(ns_t, device):
     if not isinstance(ns_t, torch.Tensor) or ns_t.numel() != 1 or ns_t.dtype != _i32 \
             or ns_t.device != device:
@@ -610,3 +619,34 @@ def gram(x, stream=None):
     ws = torch.empty(nws, dtype=torch.uint8, device=_dev(x))
     call("t2t_gram", x, dtype_code(x.dtype), G, H, N, D, ws, nws, stream_handle(stream))
     return G
+
+
+def gram_strided(x, nonfinite=None, stream=None):
+    """gram() of any [H, N, D] view with unit stride along D; ``nonfinite``
+    ([H] int32, optional) receives 1 for every head holding an inf or NaN."""
+    H, N, D = x.shape
+    dev = _dev(x)
+    if x.dtype not in _HALF or x.stride(2) != 1 or x.stride(1) < D or x.stride(0) < 0:
+        raise ValueError(f"t2t: gram_strided needs fp16 or bf16 rows of unit stride, got {x.dtype} "
+                         f"{tuple(x.shape)} strides {tuple(x.stride())}")
+    if nonfinite is not None:
+        _check(nonfinite, (H,), _i32, "nonfinite", dev)
+    G = torch.empty(H, D, D, dtype=torch.float64, device=dev)
+    nws = size_query("t2t_gram_ws_bytes", H, N, D)
+    ws = torch.empty(nws, dtype=torch.uint8, device=dev)
+    call("t2t_gram_strided", _lib.RowView(x), dtype_code(x.dtype), x.stride(0), x.stride(1), G,
+         nonfinite, H, N, D, ws, nws, stream_handle(stream))
+    return G
+
+
+def fit_chol(Mq, Mk, floor, small, stream=None):
+    """Lower Cholesky factor of Mk [H, D, D] fp64; ``small`` ([2, H] int32)
+    receives 1 where Mq[h] / Mk[h] has an eigenvalue not above ``floor``."""
+    H, D, _ = Mq.shape
+    dev = _dev(Mq)
+    _check(Mq, (H, D, D), torch.float64, "Mq", dev)
+    _check(Mk, (H, D, D), torch.float64, "Mk", dev)
+    _check(small, (2, H), _i32, "small", dev)
+    L = torch.empty_like(Mk)
+    call("t2t_fit_chol", Mq, Mk, L, small, H, D, float(floor), stream_handle(stream))
+    return L
