@@ -138,3 +138,35 @@ def test_projection_fit_forms(dev, D):
     Uq, Uk = DS.online_u(qz, k.half(), r)
     Eq, Ek = DS._fit_eigh(*(ops.gram_strided(t) for t in (qz, k.half())), r)
     assert torch.equal(Uq, Eq.float()) and torch.equal(Uk, Ek.float())
+
+
+# row blocks per wave 4, 2 and 1 (rows in whole, partial and single chunks), the
+# key pass sharing the first query pass's launches with more and fewer clusters
+@pytest.mark.parametrize("H,N,CQ,CK,pin", [(8, 131100, 200, 2048, 0), (16, 16450, 33, 500, 77),
+                                           (3, 4097, 4096, 64, 0), (2, 255, 7, 31, 255)])
+def test_kmeans_of_many_heads_equals_each_head_alone(dev, H, N, CQ, CK, pin):
+    """A head's clustering does not depend on how many heads share the launch,
+    so the launch shapes that follow H N agree bit for bit with the smallest;
+    the sort and the query means are checked against torch on the labels."""
+    from token2tile_amd import ops
+    gen = torch.Generator(device=dev).manual_seed(N)
+    r = lambda *s: torch.randn(*s, generator=gen, device=dev).half()  # noqa: E731
+    QU, KU, V = r(H, N, 32), r(H, N, 32), r(H, N, 128)
+    cq0, ck0 = r(H, CQ, 32), r(H, CK, 32)
+    cq0[:, 0] = 50.0                                    # an empty cluster
+    lab0 = lambda n: torch.zeros(n, N, dtype=torch.int32, device=dev)  # noqa: E731
+    o = ops.kmm_run(QU, KU, V, cq0, ck0, pin_tail=pin, out=dict(qlab=lab0(H), klab=lab0(H)))
+    for h in range(0, H, max(1, H // 3)):
+        one = ops.kmm_run(*(t[h:h + 1].contiguous() for t in (QU, KU, V, cq0, ck0)), pin_tail=pin,
+                          out=dict(qlab=lab0(1), klab=lab0(1)))
+        for name, t in one.items():
+            assert torch.equal(t[0], o[name][h]), name
+        for lab, perm, counts, C in ((o["qlab"], o["qperm"], o["qcounts"], CQ),
+                                     (o["klab"], o["kperm"], o["kcounts"], CK)):
+            assert torch.equal(perm[h].long(), torch.sort(lab[h], stable=True).indices)
+            assert torch.equal(counts[h].long(), torch.bincount(lab[h], minlength=C))
+        S = torch.zeros(CQ, 32, dtype=torch.int64, device=dev)
+        S.index_add_(0, o["qlab"][h].long(), torch.round(QU[h].float() * 32768.0).long())
+        n = o["qcounts"][h].float().unsqueeze(1)
+        full = o["qcounts"][h] > 0
+        assert torch.equal(o["cq2"][h][full], (S.float() / (32768.0 * n)).half()[full])

@@ -4,7 +4,7 @@
 // Pipeline of one maintenance call (all deterministic):
 //   prep centroids -> assign (MFMA distances + argmin) -> stable counting
 //   sort of the labels (chunk histograms, column scans, ballot-ranked
-//   scatter) -> per-cluster sums by one owner wave per cluster, in sorted
+//   scatter; the chunk histograms come with the labels) -> per-cluster sums by one owner wave per cluster, in sorted
 //   row order (exact int64 fixed point for query clusters; sequential fp32
 //   for key clusters, which also writes the cluster-ordered V) -> value
 //   statistics (lam, sumv).
@@ -12,7 +12,6 @@
 
 #define KM_R 32            // rank of the projected space
 #define AS_CHUNK 256       // centroids staged per LDS chunk in assign
-#define SORT_CH 1024       // rows per counting-sort chunk
 #define KM_MAXC 4096
 
 static inline int pad32(int c) { return (c + 31) & ~31; }
@@ -309,15 +308,35 @@ static void launch_fast_assign32(const void* x, const void* c, int32_t* labels, 
 // MFMA distance.  A block then costs a min tree and one compare; only a block
 // whose minimum improves on some lane's running minimum looks for its lowest
 // index at that value.
+//
+// The work-group's rows are one chunk of the counting sort: once the labels
+// are known, their histogram is taken in the LDS of the centroids and written
+// beside them.  RB, the row blocks per wave (km_rb), sets the chunk, 256 RB
+// rows.  One launch serves up to two row sets (blockIdx.z): the key pass and
+// the first query pass do not depend on each other.
 // ---------------------------------------------------------------------------
 #define AK_WAVES 8
 #define AK_CHUNK 512
-#define AK_RB 4
-template <int CMAX>
-__global__ __launch_bounds__(AK_WAVES * 64) void assign_km_kernel(
-    const uint16_t* __restrict__ X, const uint16_t* __restrict__ cprep,
-    const float* __restrict__ cnorm, int32_t* __restrict__ labels, int N, int C, int pin_begin,
-    int pin_label, const int32_t* __restrict__ guess) {
+struct AssignArgs {
+  const uint16_t* X;       // [H, N, 32]
+  const uint16_t* cprep;   // [H, C, 32] -2c
+  const float* cnorm;      // [H, C]
+  int32_t* labels;         // [H, N]
+  const int32_t* guess;    // [H, N] or null; may be labels itself
+  int32_t* chist;          // [H, chunks, C]
+  int C, pin_begin, pin_label;
+};
+template <int RB>
+__global__ __launch_bounds__(AK_WAVES * 64) void assign_km_kernel(AssignArgs g0, AssignArgs g1,
+                                                                  int N) {
+  constexpr int CMAX = AK_CHUNK, AK_RB = RB;
+  const AssignArgs& ga = blockIdx.z ? g1 : g0;
+  const uint16_t* __restrict__ X = ga.X;
+  const uint16_t* __restrict__ cprep = ga.cprep;
+  const float* __restrict__ cnorm = ga.cnorm;
+  int32_t* labels = ga.labels;
+  const int32_t* guess = ga.guess;
+  const int C = ga.C, pin_begin = ga.pin_begin, pin_label = ga.pin_label;
   constexpr int D = 32;
   __shared__ __attribute__((aligned(16))) uint16_t sC[CMAX * D];
   __shared__ __attribute__((aligned(16))) float sN[CMAX];
@@ -420,58 +439,100 @@ __global__ __launch_bounds__(AK_WAVES * 64) void assign_km_kernel(
     }
   }
   }
+  int lab[AK_RB];
 #pragma unroll
   for (int k = 0; k < AK_RB; ++k) {
     const float ob = __builtin_bit_cast(float, half_partner(__builtin_bit_cast(uint32_t, best[k])));
     const int oi = (int)half_partner((uint32_t)bidx[k]);
-    int lab = bidx[k];
-    if (ob < best[k] || (ob == best[k] && oi < bidx[k])) lab = oi;
+    lab[k] = bidx[k];
+    if (ob < best[k] || (ob == best[k] && oi < bidx[k])) lab[k] = oi;
     const int row = rbase + 32 * k;
-    if (row < N && hh == 0) labels[(size_t)h * N + row] = row >= pin_begin ? pin_label : lab;
+    lab[k] = row >= pin_begin ? pin_label : lab[k];
+    if (row < N && hh == 0) labels[(size_t)h * N + row] = lab[k];
   }
+  // the chunk's label histogram, in the LDS of the centroids
+  static_assert(CMAX * D * 2 >= KM_MAXC * 4, "the histogram fits the centroid chunk");
+  int* hist = (int*)sC;
+  __syncthreads();
+  for (int i = tid; i < C; i += AK_WAVES * 64) hist[i] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < AK_RB; ++k)
+    if (rbase + 32 * k < N && hh == 0) atomicAdd(&hist[lab[k]], 1);
+  __syncthreads();
+  int32_t* ho = ga.chist + ((size_t)h * gridDim.x + blockIdx.x) * C;
+  for (int i = tid; i < C; i += AK_WAVES * 64) ho[i] = hist[i];
 }
 
 // ---------------------------------------------------------------------------
-// stable counting sort of labels -> counts, cbase (exclusive scan), perm
+// stable counting sort of labels -> counts, cbase (exclusive scan), perm, over
+// chunks of 256 RB rows.  Like the assignment, each kernel takes up to two
+// label sets in one launch (blockIdx.z).
 // ---------------------------------------------------------------------------
+struct SortArgs {
+  const int32_t* lab;  // [H, N]
+  int32_t* chist;      // [H, chunks, C]
+  int32_t* counts;     // [H, C]
+  int32_t* cbase;      // [H, C]
+  int32_t* perm;       // [H, N]
+  int C;
+};
+
 __global__ __launch_bounds__(256) void sort_hist_kernel(const int32_t* __restrict__ lab,
                                                         int32_t* __restrict__ chist, int N, int C,
-                                                        int nChunk) {
+                                                        int rows) {
   __shared__ int hist[KM_MAXC];
   const int h = blockIdx.y, k = blockIdx.x, tid = threadIdx.x;
   for (int i = tid; i < C; i += 256) hist[i] = 0;
   __syncthreads();
-  const int r0 = k * SORT_CH;
-  const int r1 = (r0 + SORT_CH) < N ? (r0 + SORT_CH) : N;
+  const int r0 = k * rows;
+  const int r1 = (r0 + rows) < N ? (r0 + rows) : N;
   for (int r = r0 + tid; r < r1; r += 256) atomicAdd(&hist[lab[(size_t)h * N + r]], 1);
   __syncthreads();
-  int32_t* out = chist + ((size_t)h * nChunk + k) * C;
+  int32_t* out = chist + ((size_t)h * gridDim.x + k) * C;
   for (int i = tid; i < C; i += 256) out[i] = hist[i];
 }
 
 // chunk-local start offsets: chist[h, k, c] <- sum of chist[h, k', c] over
-// k' < k, and counts[h, c] <- the column total.  One wave per 64 clusters,
-// lane = cluster; the chunks are read 16 at a time (all in flight together),
-// so the latency is a few memory round trips, not one per chunk.
+// k' < k, and counts[h, c] <- the column total.  One work-group per 64
+// clusters, lane = cluster, a quarter of the chunks per wave: the quarters'
+// totals are taken first (their chunks read 16 at a time, all in flight
+// together), so the latency is a few memory round trips, not one per chunk.
 #define SCAN_GRP 16
-__global__ __launch_bounds__(64) void sort_colscan_kernel(int32_t* __restrict__ chist,
-                                                          int32_t* __restrict__ counts, int C,
-                                                          int nChunk) {
-  const int h = blockIdx.y, c = blockIdx.x * 64 + threadIdx.x;
-  if (c >= C) return;
-  int32_t* col = chist + (size_t)h * nChunk * C + c;
-  int run = 0;
-  for (int k0 = 0; k0 < nChunk; k0 += SCAN_GRP) {
-    int v[SCAN_GRP];
+__global__ __launch_bounds__(256) void sort_colscan_kernel(SortArgs g0, SortArgs g1, int nChunk) {
+  __shared__ int tot[4][64];
+  const SortArgs& g = blockIdx.z ? g1 : g0;
+  const int C = g.C;
+  const int h = blockIdx.y, l = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int c = blockIdx.x * 64 + l;
+  const bool in = c < C;
+  int32_t* col = g.chist + (size_t)h * nChunk * C + (in ? c : 0);
+  const int per = (nChunk + 3) / 4;
+  const int ka = w * per, kb = ka + per < nChunk ? ka + per : nChunk;
+  int v[SCAN_GRP];
+  auto load = [&](int k0) {
 #pragma unroll
-    for (int i = 0; i < SCAN_GRP; ++i) v[i] = k0 + i < nChunk ? col[(size_t)(k0 + i) * C] : 0;
+    for (int i = 0; i < SCAN_GRP; ++i) v[i] = in && k0 + i < kb ? col[(size_t)(k0 + i) * C] : 0;
+  };
+  int sum = 0;
+  for (int k0 = ka; k0 < kb; k0 += SCAN_GRP) {
+    load(k0);
+#pragma unroll
+    for (int i = 0; i < SCAN_GRP; ++i) sum += v[i];
+  }
+  tot[w][l] = sum;
+  __syncthreads();
+  int run = 0;
+  for (int i = 0; i < w; ++i) run += tot[i][l];
+  if (in && w == 3) g.counts[(size_t)h * C + c] = run + sum;
+  for (int k0 = ka; k0 < kb; k0 += SCAN_GRP) {
+    if (per > SCAN_GRP) load(k0);  // else the only group is still held
 #pragma unroll
     for (int i = 0; i < SCAN_GRP; ++i) {
-      if (k0 + i < nChunk) col[(size_t)(k0 + i) * C] = run;
+      if (in && k0 + i < kb) col[(size_t)(k0 + i) * C] = run;
       run += v[i];
     }
   }
-  counts[(size_t)h * C + c] = run;
 }
 
 __device__ inline void wave_sync_km() {
@@ -479,37 +540,69 @@ __device__ inline void wave_sync_km() {
   __builtin_amdgcn_wave_barrier();
 }
 
-// One wave per chunk of SORT_CH rows; rows of equal label keep their order
-// (ballot ranking).  A cluster's start in the permutation is cbase (the
-// exclusive scan of the counts over clusters) plus the chunk-local offset.
-// The chunk's labels are loaded up front, so the ranking loop waits on no
-// global load.
-#define SC_PER (SORT_CH / 64)
-__global__ __launch_bounds__(64) void sort_scatter_kernel(const int32_t* __restrict__ lab,
-                                                          const int32_t* __restrict__ chist,
-                                                          const int32_t* __restrict__ cbase,
-                                                          int32_t* __restrict__ perm, int N, int C,
-                                                          int nChunk, int lbits) {
-  extern __shared__ int cc[];  // C entries
-  const int h = blockIdx.y, k = blockIdx.x, l = threadIdx.x;
-  const int r0 = k * SORT_CH;
-  const int r1 = (r0 + SORT_CH) < N ? (r0 + SORT_CH) : N;
-  int labs[SC_PER];
+// One work-group of four waves per chunk, 64 RB consecutive rows per wave;
+// rows of equal label keep their order (each wave's own histogram gives the
+// waves' starts, ballot ranking the rows of a wave).  A cluster's start in the
+// permutation is the exclusive scan of the counts over clusters (formed here;
+// the first chunk's work-group writes it to cbase) plus the chunk-local
+// offset.  With one wave per 1024-row chunk its 16 dependent ranking steps took
+// 9-20 us of every sort of a small call, and the scan was a launch of its own.
+template <int RB>
+__global__ __launch_bounds__(256) void sort_scatter_kernel(SortArgs g0, SortArgs g1, int N,
+                                                           int nChunk) {
+  extern __shared__ int cc[];  // [4][C]
+  __shared__ int wsum[4];
+  const SortArgs& g = blockIdx.z ? g1 : g0;
+  const int C = g.C;
+  const int h = blockIdx.y, k = blockIdx.x, tid = threadIdx.x, l = tid & 63, w = tid >> 6;
+  const int r0 = k * 256 * RB + w * 64 * RB;
+  int* mine = cc + w * C;
+  int labs[RB];
 #pragma unroll
-  for (int i = 0; i < SC_PER; ++i) {
+  for (int i = 0; i < RB; ++i) {
     const int row = r0 + 64 * i + l;
-    labs[i] = row < r1 ? lab[(size_t)h * N + row] : 0;
+    labs[i] = row < N ? g.lab[(size_t)h * N + row] : 0;
   }
-  const int32_t* off = chist + ((size_t)h * nChunk + k) * C;
-  const int32_t* cb = cbase + (size_t)h * C;
-  for (int c = l; c < C; c += 64) cc[c] = cb[c] + off[c];
+  for (int c = l; c < C; c += 64) mine[c] = 0;
   wave_sync_km();
+#pragma unroll
+  for (int i = 0; i < RB; ++i)
+    if (r0 + 64 * i + l < N) atomicAdd(&mine[labs[i]], 1);
+  // exclusive scan of the head's counts: thread tid owns clusters per tid ..
+  const int per = (C + 255) / 256;
+  const int32_t* cnt = g.counts + (size_t)h * C;
+  int loc = 0;
+  for (int i = 0; i < per; ++i)
+    if (tid * per + i < C) loc += cnt[tid * per + i];
+  const int inc = wave_incl_scan(loc);
+  if (l == 63) wsum[w] = inc;
+  __syncthreads();
+  int run = inc - loc;
+  for (int i = 0; i < w; ++i) run += wsum[i];
+  const int32_t* off = g.chist + ((size_t)h * nChunk + k) * C;
+  for (int i = 0; i < per; ++i) {
+    const int c = tid * per + i;
+    if (c < C) {
+      if (k == 0) g.cbase[(size_t)h * C + c] = run;
+      int start = run + off[c];
+      run += cnt[c];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int t = cc[j * C + c];
+        cc[j * C + c] = start;
+        start += t;
+      }
+    }
+  }
+  __syncthreads();
+  int lbits = 1;
+  while ((1 << lbits) < C) ++lbits;
   const unsigned long long lt = (1ull << l) - 1ull;
 #pragma unroll
-  for (int i = 0; i < SC_PER; ++i) {
+  for (int i = 0; i < RB; ++i) {
     const int row = r0 + 64 * i + l;
-    if (r0 + 64 * i >= r1) break;  // wave-uniform
-    const bool valid = row < r1;
+    if (r0 + 64 * i >= N) break;  // wave-uniform
+    const bool valid = row < N;
     const int c = labs[i];
     unsigned long long peers = __ballot(valid);
     for (int b = 0; b < lbits; ++b) {
@@ -520,11 +613,11 @@ __global__ __launch_bounds__(64) void sort_scatter_kernel(const int32_t* __restr
     const int leader = (int)__ffsll((long long)peers) - 1;
     int base = 0;
     if (valid && l == leader) {
-      base = cc[c];
-      cc[c] = base + __popcll(peers);
+      base = mine[c];
+      mine[c] = base + __popcll(peers);
     }
     base = __shfl(base, leader < 0 ? 0 : leader, 64);
-    if (valid) perm[(size_t)h * N + base + rank] = row;
+    if (valid) g.perm[(size_t)h * N + base + rank] = row;
     wave_sync_km();
   }
 }
@@ -554,22 +647,38 @@ __global__ __launch_bounds__(1024) void cbase_kernel(const int32_t* __restrict__
   }
 }
 
-struct SortBufs {
-  int32_t* chist;  // [H, nChunk, C]
-};
+// Row blocks per wave of the assignment, and so the rows of a sort chunk
+// (256 RB): four where the launch still has four work-groups per CU, else
+// fewer, down to one.  At four throughout, 2 x 4096 rows gave the assignment 8
+// work-groups (both query passes and the key pass 70 us; 30 at one) and 5 x
+// 75600 gave it 370 of unequal share (172 us; 137 at two).
+static int km_rb(int H, int N) {
+  if ((long long)H * cdiv(N, 1024) >= 1024) return 4;
+  return (long long)H * cdiv(N, 512) >= 512 ? 2 : 1;
+}
+static int km_chunks(int H, int N) { return cdiv(N, 256 * km_rb(H, N)); }
+
+// the sort proper, from the chunk histograms; sets: 1 or 2
+static int run_scatter(const SortArgs& a, const SortArgs& b, int sets, int H, int N, hipStream_t st) {
+  const int nChunk = km_chunks(H, N);
+  const int C = sets == 2 && b.C > a.C ? b.C : a.C;
+  hipLaunchKernelGGL(sort_colscan_kernel, dim3(cdiv(C, 64), H, sets), dim3(256), 0, st, a, b, nChunk);
+  const dim3 g(nChunk, H, sets);
+  const size_t lds = (size_t)4 * C * sizeof(int);
+  switch (km_rb(H, N)) {
+    case 4: hipLaunchKernelGGL(sort_scatter_kernel<4>, g, dim3(256), lds, st, a, b, N, nChunk); break;
+    case 2: hipLaunchKernelGGL(sort_scatter_kernel<2>, g, dim3(256), lds, st, a, b, N, nChunk); break;
+    default: hipLaunchKernelGGL(sort_scatter_kernel<1>, g, dim3(256), lds, st, a, b, N, nChunk);
+  }
+  return t2t_check_launch("counting sort");
+}
 
 static int run_sort(const int32_t* lab, int32_t* counts, int32_t* cbase, int32_t* perm,
                     int32_t* chist, int H, int N, int C, hipStream_t st) {
-  const int nChunk = cdiv(N, SORT_CH);
-  int lbits = 1;
-  while ((1 << lbits) < C) ++lbits;
-  hipLaunchKernelGGL(sort_hist_kernel, dim3(nChunk, H), dim3(256), 0, st, lab, chist, N, C, nChunk);
-  hipLaunchKernelGGL(sort_colscan_kernel, dim3(cdiv(C, 64), H), dim3(64), 0, st, chist, counts, C,
-                     nChunk);
-  hipLaunchKernelGGL(cbase_kernel, dim3(H), dim3(1024), 0, st, counts, cbase, C);
-  hipLaunchKernelGGL(sort_scatter_kernel, dim3(nChunk, H), dim3(64), (size_t)C * sizeof(int), st,
-                     lab, chist, cbase, perm, N, C, nChunk, lbits);
-  return t2t_check_launch("counting sort");
+  const int rows = 256 * km_rb(H, N);
+  hipLaunchKernelGGL(sort_hist_kernel, dim3(cdiv(N, rows), H), dim3(256), 0, st, lab, chist, N, C, rows);
+  const SortArgs a{lab, chist, counts, cbase, perm, C};
+  return run_scatter(a, a, 1, H, N, st);
 }
 
 // ---------------------------------------------------------------------------
@@ -578,30 +687,39 @@ static int run_sort(const int32_t* lab, int32_t* counts, int32_t* cbase, int32_t
 //   MODE 1: rne(x * 2^20) sums, mean = fp16(f32(f64(S) / 2^20 / f64(n)))
 // empty clusters keep `old`.
 // ---------------------------------------------------------------------------
-template <int MODE>
-__global__ __launch_bounds__(256) void fixed_mean_kernel(const uint16_t* __restrict__ X,
-                                                         const int32_t* __restrict__ perm,
-                                                         const int32_t* __restrict__ counts,
-                                                         const int32_t* __restrict__ cbase,
-                                                         const uint16_t* __restrict__ old,
-                                                         uint16_t* __restrict__ out, int N, int C) {
+// WPC waves share a cluster (their sums are exact integers, so the split does
+// not change the result): four when the clusters alone would leave the chip
+// nearly empty and a wave walking its cluster 64 rows at a time is the whole
+// launch's time.  cprep / cnorm (optional): -2 mean and its squared norm, as
+// cen_prep_kernel gives them, for the next assignment.
+template <int MODE, int WPC>
+__global__ __launch_bounds__(256) void fixed_mean_kernel(
+    const uint16_t* __restrict__ X, const int32_t* __restrict__ perm,
+    const int32_t* __restrict__ counts, const int32_t* __restrict__ cbase,
+    const uint16_t* __restrict__ old, uint16_t* __restrict__ out, uint16_t* __restrict__ cprep,
+    float* __restrict__ cnorm, int N, int C) {
+  __shared__ long long part[WPC > 1 ? WPC : 1][32];
   const int h = blockIdx.y;
-  const int l = threadIdx.x & 63;
-  const int c = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int c = WPC > 1 ? blockIdx.x : blockIdx.x * 4 + w;
   if (c >= C) return;
   const int n = counts[(size_t)h * C + c];
   const int b = cbase[(size_t)h * C + c];
   // lane l sums dims 4 (l % 8) .. + 3 of rows i with i % 8 = l / 8: the
-  // cluster's row indices are read 64 at a time (one coalesced load) and
-  // broadcast, so eight independent row loads are in flight per lane.  The
-  // sums are exact integers, so their order does not change the result.
+  // cluster's row indices are read 64 at a time (one coalesced load, the next
+  // one's in flight) and broadcast, so eight independent row loads are in
+  // flight per lane.  The sums are exact integers, so their order does not
+  // change the result.
   const int dq = l & 7, rg = l >> 3;
   const float scale = MODE == 0 ? 32768.0f : 1048576.0f;
   long long S[4] = {0, 0, 0, 0};
   const int32_t* ph = perm + (size_t)h * N + b;
   const uint16_t* xh = X + (size_t)h * N * KM_R + 4 * dq;
-  for (int i0 = 0; i0 < n; i0 += 64) {
-    const int myrow = i0 + l < n ? ph[i0 + l] : -1;
+  const int first = WPC > 1 ? 64 * w : 0;
+  int nxt = first + l < n ? ph[first + l] : -1;
+  for (int i0 = first; i0 < n; i0 += 64 * WPC) {
+    const int myrow = nxt;
+    nxt = i0 + 64 * WPC + l < n ? ph[i0 + 64 * WPC + l] : -1;
     u32x2 v[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -616,27 +734,64 @@ __global__ __launch_bounds__(256) void fixed_mean_kernel(const uint16_t* __restr
         S[e] += (long long)rintf(h2f(x) * scale);
       }
   }
-  // sum over the eight row groups (lane bits 3..5)
+  // sum over the eight row groups (lane bits 3..5), then over the waves
 #pragma unroll
   for (int m = 8; m < 64; m <<= 1)
 #pragma unroll
     for (int e = 0; e < 4; ++e) S[e] += __shfl_xor(S[e], m, 64);
-  if (rg == 0) {
+  if constexpr (WPC > 1) {
+    if (rg == 0)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const size_t o = ((size_t)h * C + c) * KM_R + 4 * dq + e;
-      uint16_t v;
-      if (n == 0) {
-        v = old[o];
-      } else if (MODE == 0) {
-        v = f2h(opaque((float)S[e] / (32768.0f * (float)n)));
-      } else {
-        const double m = ((double)S[e] / 1048576.0) / (double)n;
-        v = f2h(opaque((float)m));
-      }
+      for (int e = 0; e < 4; ++e) part[w][4 * dq + e] = S[e];
+    __syncthreads();
+    if (w > 0) return;
+#pragma unroll
+    for (int i = 1; i < WPC; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) S[e] += part[i][4 * dq + e];
+  }
+  float mv[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const size_t o = ((size_t)h * C + c) * KM_R + 4 * dq + e;
+    uint16_t v;
+    if (n == 0) {
+      v = old[o];
+    } else if (MODE == 0) {
+      v = f2h(opaque((float)S[e] / (32768.0f * (float)n)));
+    } else {
+      const double m = ((double)S[e] / 1048576.0) / (double)n;
+      v = f2h(opaque((float)m));
+    }
+    mv[e] = h2f(v);
+    if (rg == 0) {
       out[o] = v;
+      if (cprep) cprep[o] = f2h(-2.0f * mv[e]);
     }
   }
+  if (cnorm) {  // dims in order: dim 4 i + e is lane i's mv[e]
+    float s = 0.f;
+#pragma unroll
+    for (int d = 0; d < KM_R; ++d) {
+      const float v = __builtin_bit_cast(
+          float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mv[d & 3]), d >> 2));
+      s = s + v * v;
+    }
+    if (l == 0) cnorm[(size_t)h * C + c] = s;
+  }
+}
+
+template <int MODE>
+static void launch_fixed_mean(const void* X, const int32_t* perm, const int32_t* counts,
+                              const int32_t* cbase, const void* old, void* out, uint16_t* cprep,
+                              float* cnorm, int H, int N, int C, hipStream_t st) {
+  if ((long long)H * C < 4096)
+    hipLaunchKernelGGL((fixed_mean_kernel<MODE, 4>), dim3(C, H), dim3(256), 0, st, (const uint16_t*)X,
+                       perm, counts, cbase, (const uint16_t*)old, (uint16_t*)out, cprep, cnorm, N, C);
+  else
+    hipLaunchKernelGGL((fixed_mean_kernel<MODE, 1>), dim3(cdiv(C, 4), H), dim3(256), 0, st,
+                       (const uint16_t*)X, perm, counts, cbase, (const uint16_t*)old, (uint16_t*)out,
+                       cprep, cnorm, N, C);
 }
 
 // ---------------------------------------------------------------------------
@@ -792,19 +947,21 @@ struct KmmWs {
   int32_t* cbase1;
   int32_t* cbaseq;
   int32_t* cbasek;
-  int32_t* chist;
+  int32_t* chistq;
+  int32_t* chistk;
   float* vsum;
   float* cmax;
-  uint16_t* cprep;  // -2c of the centroids of the assignment in flight
-  float* cnorm;     // and their squared norms
+  uint16_t* cprepq;  // -2c of the query centroids of the assignment in flight
+  float* cnormq;     // and their squared norms
+  uint16_t* cprepk;  // the same of the key centroids
+  float* cnormk;
   size_t total;
 };
 
 static KmmWs kmm_layout(int H, int N, int CQ, int CK, void* base) {
   WsCarver w(base);
   KmmWs k;
-  const int nChunk = cdiv(N, SORT_CH);
-  const int Cmax = CQ > CK ? CQ : CK;
+  const int nChunk = km_chunks(H, N);
   k.qlab1 = w.take<int32_t>((size_t)H * N);
   k.cq1 = w.take<uint16_t>((size_t)H * CQ * KM_R);
   k.perm1 = w.take<int32_t>((size_t)H * N);
@@ -812,11 +969,14 @@ static KmmWs kmm_layout(int H, int N, int CQ, int CK, void* base) {
   k.cbase1 = w.take<int32_t>((size_t)H * CQ);
   k.cbaseq = w.take<int32_t>((size_t)H * CQ);
   k.cbasek = w.take<int32_t>((size_t)H * CK);
-  k.chist = w.take<int32_t>((size_t)H * nChunk * Cmax);
+  k.chistq = w.take<int32_t>((size_t)H * nChunk * CQ);
+  k.chistk = w.take<int32_t>((size_t)H * nChunk * CK);
   k.vsum = w.take<float>((size_t)H * CK * 128);
   k.cmax = w.take<float>((size_t)H * CK);
-  k.cprep = w.take<uint16_t>((size_t)H * Cmax * KM_R);
-  k.cnorm = w.take<float>((size_t)H * Cmax);
+  k.cprepq = w.take<uint16_t>((size_t)H * CQ * KM_R);
+  k.cnormq = w.take<float>((size_t)H * CQ);
+  k.cprepk = w.take<uint16_t>((size_t)H * CK * KM_R);
+  k.cnormk = w.take<float>((size_t)H * CK);
   k.total = w.off;
   return k;
 }
@@ -827,31 +987,43 @@ extern "C" size_t t2t_kmm_ws_bytes(int H, int N, int CQ, int CK) {
 
 // -2c (exact in fp16) and the fp32 squared norm of every centroid, summed
 // sequentially over the dims (each square is exact): the operands of
-// assign_km_kernel
-__global__ __launch_bounds__(256) void cen_prep_kernel(const uint16_t* __restrict__ cen,
-                                                       uint16_t* __restrict__ cprep,
-                                                       float* __restrict__ cnorm, int C) {
+// assign_km_kernel, for the query (blockIdx.z 0) and key centroids
+__global__ __launch_bounds__(256) void cen_prep_kernel(
+    const uint16_t* __restrict__ cenq, uint16_t* __restrict__ cprepq, float* __restrict__ cnormq,
+    int CQ, const uint16_t* __restrict__ cenk, uint16_t* __restrict__ cprepk,
+    float* __restrict__ cnormk, int CK) {
+  const uint16_t* cen = blockIdx.z ? cenk : cenq;
+  const int C = blockIdx.z ? CK : CQ;
   const int h = blockIdx.y, ci = blockIdx.x * 256 + threadIdx.x;
   if (ci >= C) return;
-  const uint16_t* cp = cen + ((size_t)h * C + ci) * KM_R;
-  uint16_t* op = cprep + ((size_t)h * C + ci) * KM_R;
+  const u32x4* cp = (const u32x4*)(cen + ((size_t)h * C + ci) * KM_R);
+  u32x4* op = (u32x4*)((blockIdx.z ? cprepk : cprepq) + ((size_t)h * C + ci) * KM_R);
   float s = 0.f;
-  for (int d = 0; d < KM_R; ++d) {
-    const float v = h2f(cp[d]);
-    s = s + v * v;
-    op[d] = f2h(-2.0f * v);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const u32x4 v = cp[i];
+    u32x4 o;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const float a = h2f((uint16_t)(v[t] & 0xffff)), b = h2f((uint16_t)(v[t] >> 16));
+      s = s + a * a;
+      s = s + b * b;
+      o[t] = (uint32_t)f2h(-2.0f * a) | ((uint32_t)f2h(-2.0f * b) << 16);
+    }
+    op[i] = o;
   }
-  cnorm[(size_t)h * C + ci] = s;
+  (blockIdx.z ? cnormk : cnormq)[(size_t)h * C + ci] = s;
 }
 
-static int launch_assign_km(const void* X, const void* cen, int32_t* lab, int H, int N, int C,
-                            int pin_begin, int pin_label, uint16_t* cprep, float* cnorm,
-                            const int32_t* guess, hipStream_t st) {
-  hipLaunchKernelGGL(cen_prep_kernel, dim3(cdiv(C, 256), H), dim3(256), 0, st,
-                     (const uint16_t*)cen, cprep, cnorm, C);
-  hipLaunchKernelGGL(assign_km_kernel<AK_CHUNK>, dim3(cdiv(N, AK_WAVES * 32 * AK_RB), H),
-                     dim3(AK_WAVES * 64), 0, st, (const uint16_t*)X, (const uint16_t*)cprep,
-                     (const float*)cnorm, lab, N, C, pin_begin, pin_label, guess);
+// sets: 1 or 2 row sets in one launch
+static int launch_assign_km(const AssignArgs& a, const AssignArgs& b, int sets, int H, int N,
+                            hipStream_t st) {
+  const dim3 g(km_chunks(H, N), H, sets);
+  switch (km_rb(H, N)) {
+    case 4: hipLaunchKernelGGL(assign_km_kernel<4>, g, dim3(AK_WAVES * 64), 0, st, a, b, N); break;
+    case 2: hipLaunchKernelGGL(assign_km_kernel<2>, g, dim3(AK_WAVES * 64), 0, st, a, b, N); break;
+    default: hipLaunchKernelGGL(assign_km_kernel<1>, g, dim3(AK_WAVES * 64), 0, st, a, b, N);
+  }
   return t2t_check_launch("assign");
 }
 
@@ -895,27 +1067,30 @@ static int kmm_impl(const void* QU, const void* KU, const void* V, int v_dtype,
   hipStream_t st = (hipStream_t)stream;
   KmmWs w = kmm_layout(H, N, CQ, CK, ws);
   const int nores = N + 1;  // no pinned rows
-  // query pass 1
-  // the label buffers' previous contents (the caller's labels of the last
-  // call, or anything) are warm-start guesses: pass 1 starts from qlab, pass 2
-  // from pass 1's labels, the key pass from klab
-  KM_CHECK(launch_assign_km(QU, cq0, w.qlab1, H, N, CQ, nores, 0, w.cprep, w.cnorm, qlab, st));
-  KM_CHECK(run_sort(w.qlab1, w.counts1, w.cbase1, w.perm1, w.chist, H, N, CQ, st));
-  hipLaunchKernelGGL(fixed_mean_kernel<0>, dim3(cdiv(CQ, 4), H), dim3(256), 0, st,
-                     (const uint16_t*)QU, w.perm1, w.counts1, w.cbase1, (const uint16_t*)cq0,
-                     w.cq1, N, CQ);
+  // The key pass does not depend on the query passes, so it shares the
+  // launches of the first one.  The label buffers' previous contents (the
+  // caller's labels of the last call, or anything) are warm-start guesses:
+  // pass 1 starts from qlab, pass 2 from pass 1's labels, the key pass from klab
+  hipLaunchKernelGGL(cen_prep_kernel, dim3(cdiv(CQ > CK ? CQ : CK, 256), H, 2), dim3(256), 0, st,
+                     (const uint16_t*)cq0, w.cprepq, w.cnormq, CQ, (const uint16_t*)ck0, w.cprepk,
+                     w.cnormk, CK);
+  const AssignArgs ak{(const uint16_t*)KU, w.cprepk, w.cnormk, klab, klab, w.chistk, CK,
+                      pin_tail > 0 ? N - pin_tail : nores, CK - 1};
+  const AssignArgs aq1{(const uint16_t*)QU, w.cprepq, w.cnormq, w.qlab1, qlab, w.chistq, CQ, nores, 0};
+  KM_CHECK(launch_assign_km(ak, aq1, 2, H, N, st));
+  const SortArgs sk{klab, w.chistk, kcounts, w.cbasek, kperm, CK};
+  const SortArgs sq1{w.qlab1, w.chistq, w.counts1, w.cbase1, w.perm1, CQ};
+  KM_CHECK(run_scatter(sk, sq1, 2, H, N, st));
+  launch_fixed_mean<0>(QU, w.perm1, w.counts1, w.cbase1, cq0, w.cq1, w.cprepq, w.cnormq, H, N, CQ, st);
   T2T_LAUNCH_CHECK("qmean 1");
   // query pass 2
-  KM_CHECK(launch_assign_km(QU, w.cq1, qlab, H, N, CQ, nores, 0, w.cprep, w.cnorm, w.qlab1, st));
-  KM_CHECK(run_sort(qlab, qcounts, w.cbaseq, qperm, w.chist, H, N, CQ, st));
-  hipLaunchKernelGGL(fixed_mean_kernel<0>, dim3(cdiv(CQ, 4), H), dim3(256), 0, st,
-                     (const uint16_t*)QU, qperm, qcounts, w.cbaseq, (const uint16_t*)w.cq1,
-                     (uint16_t*)cq2, N, CQ);
+  const AssignArgs aq2{(const uint16_t*)QU, w.cprepq, w.cnormq, qlab, w.qlab1, w.chistq, CQ, nores, 0};
+  KM_CHECK(launch_assign_km(aq2, aq2, 1, H, N, st));
+  const SortArgs sq2{qlab, w.chistq, qcounts, w.cbaseq, qperm, CQ};
+  KM_CHECK(run_scatter(sq2, sq2, 1, H, N, st));
+  launch_fixed_mean<0>(QU, qperm, qcounts, w.cbaseq, w.cq1, cq2, nullptr, nullptr, H, N, CQ, st);
   T2T_LAUNCH_CHECK("qmean 2");
-  // key pass
-  KM_CHECK(launch_assign_km(KU, ck0, klab, H, N, CK, pin_tail > 0 ? N - pin_tail : nores,
-                            CK - 1, w.cprep, w.cnorm, klab, st));
-  KM_CHECK(run_sort(klab, kcounts, w.cbasek, kperm, w.chist, H, N, CK, st));
+  // key sums and value statistics
   if (v_dtype == T2T_F16)
     launch_key_gather<F16T>(KU, V, kperm, kcounts, w.cbasek, ck0, ck2, V_sorted, w.vsum, w.cmax, H, N, CK,
                             svh, svn, st);
@@ -1061,7 +1236,7 @@ static DetWs det_layout(int H, int N, int C, void* base) {
   DetWs d;
   d.perm = w.take<int32_t>((size_t)H * N);
   d.cbase = w.take<int32_t>((size_t)H * C);
-  d.chist = w.take<int32_t>((size_t)H * cdiv(N, SORT_CH) * C);
+  d.chist = w.take<int32_t>((size_t)H * km_chunks(H, N) * C);
   d.total = w.off;
   return d;
 }
@@ -1220,9 +1395,7 @@ extern "C" int t2t_det_centroid_update(const void* x, const int32_t* labels, con
   hipStream_t st = (hipStream_t)stream;
   DetWs w = det_layout(H, N, C, ws);
   KM_CHECK(run_sort(labels, counts, w.cbase, w.perm, w.chist, H, N, C, st));
-  hipLaunchKernelGGL(fixed_mean_kernel<1>, dim3(cdiv(C, 4), H), dim3(256), 0, st,
-                     (const uint16_t*)x, w.perm, counts, w.cbase, (const uint16_t*)old,
-                     (uint16_t*)out, N, C);
+  launch_fixed_mean<1>(x, w.perm, counts, w.cbase, old, out, nullptr, nullptr, H, N, C, st);
   T2T_LAUNCH_CHECK("det_update");
   return T2T_OK;
 }
