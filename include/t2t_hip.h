@@ -244,6 +244,20 @@ int t2t_tile_attn_exact_orig_gather_kv_strided(
     const int32_t* unip, const int32_t* qperm, const int32_t* plan, void* out,
     long long out_head_stride, long long out_row_stride, float* lse, int H, int N, int CQ,
     void* stream);
+/* The three calls above with a workspace (t2t_tile_attn_split_ws_bytes; 0 where
+ * the sizes fill the GPU and nothing is split): a small call's tasks are split
+ * along the keys and their parts added in fp32.  gather 0: k and v are the
+ * cluster-ordered kp and vp (contiguous; kperm unused); 1: k in the original
+ * order through kperm; 2: k and v.  qlab: the query labels that qperm sorts.
+ * The results do not depend on gather.  No counterpart in the reference. */
+size_t t2t_tile_attn_split_ws_bytes(int H, int N, int CQ);
+int t2t_tile_attn_exact_split(
+    const void* q, long long q_head_stride, long long q_row_stride, const void* k,
+    long long k_head_stride, long long k_row_stride, const void* v, long long v_head_stride,
+    long long v_row_stride, const int32_t* kperm, int gather, int dtype, const int32_t* kcounts,
+    const int32_t* unip, const int32_t* qlab, const int32_t* qperm, const int32_t* plan, void* out,
+    long long out_head_stride, long long out_row_stride, float* lse, int H, int N, int CQ, void* ws,
+    size_t ws_bytes, void* stream);
 /* ---- strided variants ---------------------------------------------------
  * No counterpart in the reference: its SGLang backend copies q, k and v from
  * the model's token-major [1, N, H, 128] into head-major [H, N, 128] and the

@@ -170,3 +170,53 @@ def test_kmeans_of_many_heads_equals_each_head_alone(dev, H, N, CQ, CK, pin):
         n = o["qcounts"][h].float().unsqueeze(1)
         full = o["qcounts"][h] > 0
         assert torch.equal(o["cq2"][h][full], (S.float() / (32768.0 * n)).half()[full])
+
+
+# 8, 4, 2 and 1 parts per task at most; unions from empty over one tile and a
+# few keys around the least part length to all keys; ragged tasks and tiles
+@pytest.mark.parametrize("H,N,CQ", [(1, 2500, 3), (2, 8190, 100), (3, 20011, 201), (5, 32760, 256)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_exact_split_matches_whole_tasks(dev, H, N, CQ, dtype):
+    """The split call against the unsplit kernel on the same plan.  Both round
+    every weight to the type (a relative u) against a max of their own, so each
+    is within u (sum w |v| / sum w + |o|) of the exact result, and rounds the
+    output once more.  (fp16 scores stay small: no weight is subnormal.)"""
+    from token2tile_amd import ops
+    rng = np.random.default_rng(N)
+    qlab, klab, qperm, qcounts, kperm, kcounts = structure(rng, H, N, CQ)
+    density = rng.choice([0.0, 0.002, 0.05, 0.2, 0.7, 1.0], (H, CQ, 1))
+    density[:, 0], density[:, 1 % CQ] = 0.0, 1.0
+    sel = (rng.random((H, CQ, 2048)) < density).astype(np.uint8)
+    unip = np.packbits(sel, axis=2, bitorder="little").view(np.int32)
+    gen = torch.Generator(device=dev).manual_seed(N)
+    q, k, v = (torch.randn(H, N, 128, generator=gen, device=dev).to(dtype) for _ in range(3))
+    q *= 0.5
+    if dtype == torch.bfloat16:
+        k[:, N // 2] *= 40                    # a score far above the earlier parts' max
+    t = lambda a: g(a, dev)                   # noqa: E731
+    tq, tk, tu, tqp, tkp, tql = map(t, (qcounts, kcounts, unip, qperm, kperm, qlab))
+    plan = ops.tile_plan(tq, tk, tu, N)
+    out = [torch.full_like(q, float("nan")) for _ in range(2)]
+    lse = [torch.full((H, N), float("nan"), device=dev) for _ in range(2)]
+    ops.tile_attn_exact_orig_gather_kv(q, k, v, tkp, tk, tu, tqp, plan, out[0], lse[0])
+    ops.tile_attn_exact_split(q, k, v, tkp, tk, tu, tql, tqp, plan, out[1], lse[1])
+    # tokens of an even view, as the backend passes them
+    qs, ks, vs, os_ = (x.transpose(0, 1).contiguous().transpose(0, 1) for x in (q, k, v, out[1]))
+    lse2 = lse[1].clone()
+    ops.tile_attn_exact_split(qs, ks, vs, tkp, tk, tu, tql, tqp, plan, os_, lse2)
+    assert torch.equal(os_, out[1]) and torch.equal(lse2, lse[1])
+    # and the gathered forms, bit for bit
+    kp, vp = ops.fast_gather(k, tkp), ops.fast_gather(v, tkp)
+    for kk, vv, gather in ((kp, vp, 0), (k, vp, 1)):
+        o2 = torch.full_like(q, float("nan"))
+        ops.tile_attn_exact_split(q, kk, vv, tkp, tk, tu, tql, tqp, plan, o2, lse2, gather=gather)
+        assert torch.equal(o2, out[1]) and torch.equal(lse2, lse[1])
+    a, b = (o.float() for o in out)
+    mean, lse3 = torch.empty_like(q), torch.empty_like(lse2)
+    ops.tile_attn_exact_orig_gather_kv(q, k, v.abs(), tkp, tk, tu, tqp, plan, mean, lse3)
+    u = 2.0 ** (-11 if dtype == torch.float16 else -8)   # unit roundoff of 11 and 8 bits
+    bound = 4 * u * 1.01 * mean.float() + 2 * u * a.abs() + 1e-6
+    assert not a.isnan().any() and bool(((a - b).abs() <= bound).all())
+    fin = lse[0].isfinite()
+    assert torch.equal(fin, lse[1].isfinite())
+    assert float((lse[0] - lse[1])[fin].abs().max()) <= 2 * u * 1.4427 * 1.01 + 2e-5

@@ -61,6 +61,11 @@ SIGNATURES = {
                                                            _P, c_int, _P, _P, _P, _P, _P,
                                                            c_longlong, c_longlong, _P, c_int,
                                                            c_int, c_int, _P]),
+    "t2t_tile_attn_split_ws_bytes": (c_size_t, [c_int, c_int, c_int]),
+    "t2t_tile_attn_exact_split": (c_int, [_P, c_longlong, c_longlong, _P, c_longlong, c_longlong, _P,
+                                          c_longlong, c_longlong, _P, c_int, c_int, _P, _P, _P, _P,
+                                          _P, _P, c_longlong, c_longlong, _P, c_int, c_int, c_int,
+                                          _P, c_size_t, _P]),
     "t2t_project_strided": (c_int, [_P, c_int, _P, _P, c_int, c_int, c_int, c_int, c_longlong,
                                     c_longlong, _P]),
     "t2t_kmm_run_strided": (c_int, [_P, _P, _P, c_int, c_longlong, c_longlong] + [_P] * 13 +

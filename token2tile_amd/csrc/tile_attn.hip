@@ -230,6 +230,28 @@ __device__ inline int xcd_remap(int bid, int total) {
   return (r / 8) * 64 + (bid % 8) * 8 + r % 8;
 }
 
+// ---- small calls -----------------------------------------------------------
+// A call of few tasks leaves most of the 512 work-group slots idle and lasts as
+// long as its longest task.  Its tasks are split along the keys: part p of P
+// takes the tiles [p n / P, (p + 1) n / P) of the task's n, keeps its sums
+// unnormalised in fp32 and combine_kernel adds the parts.  P follows the
+// task's own length, at least TA_SPLIT_TILES tiles a part (below that a
+// part's start, the union runs and the first tile's fetch, costs more than
+// its tiles).
+#define TA_SPLIT_MAX 8
+#define TA_SPLIT_TILES 6
+__host__ __device__ inline int split_parts(int kvlen, int S) {
+  const int n = (kvlen + TA_KT - 1) / TA_KT / TA_SPLIT_TILES;
+  return n < 1 ? 1 : (n < S ? n : S);
+}
+// Most parts per task (1: the call is not split): about three work-groups per
+// slot, counting a task per 128 queries and half a task more per query cluster.
+static int split_max(int H, int N, int CQ) {
+  const long long tasks = (long long)H * (cdiv(N, TA_QT) + CQ / 2) + 1;
+  const long long S = (3 * 512 + tasks - 1) / tasks;
+  return (int)(S < 1 ? 1 : (S > TA_SPLIT_MAX ? TA_SPLIT_MAX : S));
+}
+
 #define T2T_SPIN_CAP (1 << 20)  // polls before a producer/consumer wait gives up
 #define TA_MARGIN 3.0f   // log2 units of headroom when the exact-part max advances
 // a tile is redone with a new max when one lane's weight sum passes this: far
@@ -290,7 +312,10 @@ __device__ inline uint32_t pack_hi(uint32_t a, uint32_t b) { return __builtin_am
 // MODE 3: as MODE 2, with the V gather fused as well: vp is v in its original
 // order, read through kperm like K (no V_sorted)
 // (the residual kernel merges into out in place).
-template <typename T, int MODE>
+// SPLIT (MODE 1 to 3): S work-groups per task, see split_parts; a part of a split task
+// leaves its unnormalised O, max and sum in opart / mlpart at sorted row
+// part * H * N + h * N + j.
+template <typename T, int MODE, bool SPLIT>
 __global__ __launch_bounds__(TA_WAVES * 64, 2) void attn_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ kp,
     const uint16_t* __restrict__ vp, const uint32_t* __restrict__ unip,
@@ -299,7 +324,7 @@ __global__ __launch_bounds__(TA_WAVES * 64, 2) void attn_kernel(
     const int32_t* __restrict__ tasks, uint16_t* __restrict__ attn_out, float* __restrict__ lse,
     uint16_t* __restrict__ out, const int32_t* __restrict__ kperm, int H, int N, int CQ, int maxT,
     long long sqh, long long sqn, long long skh, long long skn, long long soh, long long son,
-    long long svh, long long svn) {
+    long long svh, long long svn, int S, float* __restrict__ opart, float* __restrict__ mlpart) {
   // row n of head h of q / k (MODE 2) / out (MODE 1, 2) sits at base + h s_h + n s_n
   // (elements): [H, N, 128] contiguous or a strided view such as token-major [N, H, 128]
   constexpr bool KG = MODE >= 2;
@@ -332,10 +357,14 @@ __global__ __launch_bounds__(TA_WAVES * 64, 2) void attn_kernel(
   // (with NaN in the task's output) instead of hanging it
   __shared__ int sReady[2], sDone[2], sAbort;
   __shared__ int wsc[TA_WAVES], wsr[TA_WAVES];
-  const int total = H * maxT;
-  const int lin = xcd_remap(blockIdx.x, total);
-  if (lin >= total) return;
-  const int h = lin / maxT, ti = lin % maxT;
+  const int total = H * maxT * (SPLIT ? S : 1);
+  const int lin0 = xcd_remap(blockIdx.x, total);
+  if (lin0 >= total) return;
+  // split: the parts of a task next to each other, the heads' tasks interleaved
+  // so that every head's longest come first
+  const int part = SPLIT ? lin0 % S : 0;
+  const int lin = SPLIT ? lin0 / S : lin0;
+  const int h = SPLIT ? lin % H : lin / maxT, ti = SPLIT ? lin / H : lin % maxT;
   if (ti >= ntask[h]) return;
   const int32_t* tk = tasks + ((size_t)h * maxT + ti) * 4;
   const int t = tk[0], qs = tk[1], qrows = tk[2];
@@ -372,6 +401,8 @@ __global__ __launch_bounds__(TA_WAVES * 64, 2) void attn_kernel(
     nrun += wsc[i];
     kvlen += wsr[i];
   }
+  const int nparts = SPLIT ? split_parts(kvlen, S) : 1;
+  if (SPLIT && part >= nparts) return;  // uniform
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
     if (cnts[j] > 0) {
@@ -467,7 +498,9 @@ __global__ __launch_bounds__(TA_WAVES * 64, 2) void attn_kernel(
   };
 
   const float c = 0.08838834764831845f * 1.4426950408889634f;  // 1/sqrt(128) * log2(e)
-  float m = -__builtin_inff(), lsum = 0.f;
+  // a part's first max is finite, so that a part whose scores are all -inf adds
+  // weight 0 like such tiles of a whole task, whose max is set by others
+  float m = SPLIT ? -1.0e30f : -__builtin_inff(), lsum = 0.f;
   f32x16 O[4];
 #pragma unroll
   for (int nb = 0; nb < 4; ++nb) O[nb] = zero16();
@@ -486,7 +519,11 @@ __global__ __launch_bounds__(TA_WAVES * 64, 2) void attn_kernel(
     const uint32_t krow_bytes = KG ? (uint32_t)(skn * 2) : 256u;
     const char* vh = (const char*)(vp + (VG ? (size_t)h * svh : (size_t)h * N * TA_D));
     const uint32_t vrow_bytes = VG ? (uint32_t)(svn * 2) : 256u;
-    const int ntile = (kvlen + TA_KT - 1) / TA_KT;
+    // tiles tb .. tb + ntile - 1 of the task's, the last one partial or not
+    const int nall = (kvlen + TA_KT - 1) / TA_KT;
+    const int tb = SPLIT ? (int)((long long)part * nall / nparts) : 0;
+    const int ntile = SPLIT ? (int)((long long)(part + 1) * nall / nparts) - tb : nall;
+    const bool partial = kvlen % TA_KT != 0 && tb + ntile == nall;
     // source rows of tile `tile` -> sIdx[tile & 1]; past the end -> row 0
     // (its keys are masked and its values multiply a zero probability).
     // Built by the last wave (idle in tasks of <= 96 rows) without loops:
@@ -502,7 +539,7 @@ __global__ __launch_bounds__(TA_WAVES * 64, 2) void attn_kernel(
     const int32_t* kph = KG ? kperm + (size_t)h * N : nullptr;
     auto build_idx = [&](int tile) __attribute__((always_inline)) {
       if (wave == TA_WAVES - 1) {
-        const int base = tile * TA_KT;
+        const int base = (tb + tile) * TA_KT;
         const int r = r0 + lane;
         int cs = 0x7fffffff, rw = 0;
         if (r < nrun) {
@@ -644,6 +681,16 @@ __global__ __launch_bounds__(TA_WAVES * 64, 2) void attn_kernel(
     }
     if (tid == 0) sAbort = 0;
     __syncthreads();  // runs visible
+    if constexpr (SPLIT) {
+      // the run holding the part's first position: the last one starting at
+      // or before it
+      int lo = 0, hi = nrun - 1;
+      while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (run_cum(mid) <= tb * TA_KT) lo = mid; else hi = mid - 1;
+      }
+      r0 = lo;
+    }
     if (qrows <= 32 * (TA_WAVES - 1)) {
       // the last wave stages every tile (all 16 row groups of K and V) and
       // publishes it; the consumer waves wait only for the tile they read and
@@ -719,7 +766,7 @@ __global__ __launch_bounds__(TA_WAVES * 64, 2) void attn_kernel(
           if (lane == 0)
             __hip_atomic_fetch_add(&sDone[buf], 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
         };
-        const int nfull = (kvlen % TA_KT) ? ntile - 1 : ntile;
+        const int nfull = partial ? ntile - 1 : ntile;
         int tile = 0;
         for (; tile + 2 <= nfull; tile += 2) {
           consume(tile, B0{}, TA_KT, std::false_type{});
@@ -727,7 +774,7 @@ __global__ __launch_bounds__(TA_WAVES * 64, 2) void attn_kernel(
         }
         if (tile < nfull) consume(tile++, B0{}, TA_KT, std::false_type{});
         if (tile < ntile) {
-          const int valid = kvlen - tile * TA_KT;
+          const int valid = kvlen - (tb + tile) * TA_KT;
           if (tile & 1)
             consume(tile, B1{}, valid, std::true_type{});
           else
@@ -766,7 +813,7 @@ __global__ __launch_bounds__(TA_WAVES * 64, 2) void attn_kernel(
     // full tiles two at a time, so that each buffer is a compile-time
     // constant; a partial last tile is peeled after the loop (a masked copy of
     // the tile body inside the loop would raise its register pressure)
-    const int nfull = (kvlen % TA_KT) ? ntile - 1 : ntile;
+    const int nfull = partial ? ntile - 1 : ntile;
     int tile = 0;
     for (; tile + 2 <= nfull; tile += 2) {
       body(tile, B0{});
@@ -774,7 +821,7 @@ __global__ __launch_bounds__(TA_WAVES * 64, 2) void attn_kernel(
     }
     if (tile < nfull) body(tile++, B0{});
     if (tile < ntile && wave_active) {
-      const int valid = kvlen - tile * TA_KT;
+      const int valid = kvlen - (tb + tile) * TA_KT;
       if (tile & 1)
         tile_step(B1{}, valid, std::true_type{});
       else
@@ -783,6 +830,25 @@ __global__ __launch_bounds__(TA_WAVES * 64, 2) void attn_kernel(
     }
   }
   const float lt = half_sum(lsum);
+  if constexpr (SPLIT) {
+    if (nparts > 1) {  // uniform
+      if (qok) {
+        const size_t pr = (size_t)part * H * N + obase + qrow;
+        float* op = opart + pr * TA_D + 4 * hh;
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb)
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+            *(f32x4*)(op + 32 * nb + 8 * g) =
+                f32x4{O[nb][4 * g], O[nb][4 * g + 1], O[nb][4 * g + 2], O[nb][4 * g + 3]};
+        if (hh == 0) {
+          mlpart[2 * pr] = m;
+          mlpart[2 * pr + 1] = lt;
+        }
+      }
+      return;
+    }
+  }
   const float inv = kvlen > 0 ? 1.0f / lt : 0.f;
   const float lse2 = kvlen > 0 ? m + __log2f(lt) : -__builtin_inff();
   // exact output of the lane's 64 dims, rounded to T as the exact buffer
@@ -817,11 +883,82 @@ static void launch_attn(const void* q, const void* kp, const void* vp, const int
   if (soh < 0) soh = (long long)N * TA_D;
   const int total = H * p.maxT;
   const int grid = ((total + 63) / 64) * 64;
-  hipLaunchKernelGGL((attn_kernel<T, MODE>), dim3(grid), dim3(TA_WAVES * 64), 0, st,
+  hipLaunchKernelGGL((attn_kernel<T, MODE, false>), dim3(grid), dim3(TA_WAVES * 64), 0, st,
                      (const uint16_t*)q, (const uint16_t*)kp, (const uint16_t*)vp,
                      (const uint32_t*)unip, qperm, kcounts, p.k_off, p.ntask, p.tasks,
                      (uint16_t*)attn_out, lse, (uint16_t*)out, kperm, H, N, CQ, p.maxT, sqh, sqn,
-                     skh, skn, soh, son, svh, svn);
+                     skh, skn, soh, son, svh, svn, 1, (float*)nullptr, (float*)nullptr);
+}
+
+// adds the parts of the split tasks: 32 lanes per sorted row, four dims each
+template <typename T>
+__global__ __launch_bounds__(256) void combine_kernel(
+    const float* __restrict__ opart, const float* __restrict__ mlpart,
+    const int32_t* __restrict__ kvlen, const int32_t* __restrict__ qlab,
+    const int32_t* __restrict__ qperm, uint16_t* __restrict__ out, float* __restrict__ lse, int H,
+    int N, int CQ, int S, long long soh, long long son) {
+  const int h = blockIdx.y, l = threadIdx.x & 31;
+  const int j = blockIdx.x * 8 + (threadIdx.x >> 5);
+  if (j >= N) return;
+  const int orig = qperm[(size_t)h * N + j];
+  const int P = split_parts(kvlen[(size_t)h * CQ + qlab[(size_t)h * N + orig]], S);
+  if (P < 2) return;  // the task wrote its rows itself
+  float mi[TA_SPLIT_MAX], li[TA_SPLIT_MAX];
+  f32x4 oi[TA_SPLIT_MAX];
+  float M = -__builtin_inff();
+#pragma unroll
+  for (int i = 0; i < TA_SPLIT_MAX; ++i)
+    if (i < P) {
+      const size_t pr = (size_t)i * H * N + (size_t)h * N + j;
+      mi[i] = mlpart[2 * pr];
+      li[i] = mlpart[2 * pr + 1];
+      oi[i] = *(const f32x4*)(opart + pr * TA_D + 4 * l);
+      M = vmax(M, mi[i]);
+    }
+  float lt = 0.f;
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < TA_SPLIT_MAX; ++i)
+    if (i < P) {
+      const float a = __builtin_amdgcn_exp2f(mi[i] - M);
+      lt = fmaf(a, li[i], lt);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = fmaf(a, oi[i][e], o[e]);
+    }
+  const float inv = 1.0f / lt;
+  *(u32x2*)(out + (size_t)h * soh + (size_t)orig * son + 4 * l) =
+      u32x2{Pk<T>::pack(o[0] * inv, o[1] * inv), Pk<T>::pack(o[2] * inv, o[3] * inv)};
+  if (l == 0) lse[(size_t)h * N + j] = M + __log2f(lt);
+}
+
+struct SplitWs {
+  float* opart;
+  float* mlpart;
+  size_t total;
+};
+static SplitWs split_layout(int H, int N, int S, void* base) {
+  WsCarver w(base);
+  SplitWs v;
+  v.opart = w.take<float>((size_t)S * H * N * TA_D);
+  v.mlpart = w.take<float>((size_t)S * H * N * 2);
+  v.total = w.off;
+  return v;
+}
+
+template <typename T, int MODE>
+static void launch_attn_split(const void* q, const void* k, const void* v, const int32_t* unip,
+                              const int32_t* qlab, const int32_t* qperm, const int32_t* kcounts,
+                              const PlanView& p, float* lse, void* out, int H, int N, int CQ, int S,
+                              const SplitWs& w, const int32_t* kperm, const long long (&sd)[8],
+                              hipStream_t st) {
+  const int grid = ((H * p.maxT * S + 63) / 64) * 64;
+  hipLaunchKernelGGL((attn_kernel<T, MODE, true>), dim3(grid), dim3(TA_WAVES * 64), 0, st,
+                     (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v,
+                     (const uint32_t*)unip, qperm, kcounts, p.k_off, p.ntask, p.tasks,
+                     (uint16_t*)nullptr, lse, (uint16_t*)out, kperm, H, N, CQ, p.maxT, sd[0], sd[1],
+                     sd[2], sd[3], sd[6], sd[7], sd[4], sd[5], S, w.opart, w.mlpart);
+  hipLaunchKernelGGL(combine_kernel<T>, dim3(cdiv(N, 8), H), dim3(256), 0, st, w.opart, w.mlpart,
+                     p.kvlen, qlab, qperm, (uint16_t*)out, lse, H, N, CQ, S, sd[6], sd[7]);
 }
 
 // ---------------------------------------------------------------------------
@@ -1225,6 +1362,64 @@ extern "C" int t2t_tile_attn_exact_orig_gather_strided(
                            out_row_stride, lse, H, N, CQ, stream);
 }
 
+template <typename T>
+static void exact_launch(int mode, const void* q, const void* k, const void* v, const long long (&sd)[8],
+                         const int32_t* kperm, const int32_t* kcounts, const int32_t* unip,
+                         const int32_t* qlab, const int32_t* qperm, const PlanView& p, void* out,
+                         float* lse, int H, int N, int CQ, int S, const SplitWs& w, hipStream_t st) {
+#define EX_LAUNCH(M)                                                                                \
+  if (S > 1)                                                                                        \
+    launch_attn_split<T, M>(q, k, v, unip, qlab, qperm, kcounts, p, lse, out, H, N, CQ, S, w, kperm, \
+                            sd, st);                                                                \
+  else                                                                                              \
+    launch_attn<T, M>(q, k, v, unip, qperm, kcounts, p, nullptr, lse, out, H, N, CQ, st, kperm,     \
+                      sd[0], sd[1], sd[2], sd[3], sd[6], sd[7], sd[4], sd[5])
+  if (mode == 1) {
+    EX_LAUNCH(1);
+  } else if (mode == 2) {
+    EX_LAUNCH(2);
+  } else {
+    EX_LAUNCH(3);
+  }
+#undef EX_LAUNCH
+}
+
+// mode: how K and V rows are read (see attn_kernel); qlab null: never split
+static int exact_impl(int mode, const void* q, const void* k, const void* v, const long long (&sd)[8],
+                      const int32_t* kperm, int dtype, const int32_t* kcounts, const int32_t* unip,
+                      const int32_t* qlab, const int32_t* qperm, const int32_t* plan, void* out,
+                      float* lse, int H, int N, int CQ, void* ws, size_t ws_bytes, void* stream) {
+  T2T_REQUIRE(q && k && v && (kperm || mode < 2) && kcounts && unip && qperm && plan && out && lse,
+              "tile_attn_exact_orig_gather_kv: null pointer");
+  T2T_REQUIRE(check_dtype(dtype), "tile_attn_exact_orig_gather_kv: dtype %d", dtype);
+  T2T_REQUIRE(H > 0 && N > 0 && N < (1 << 24) && CQ > 0,
+              "tile_attn_exact_orig_gather_kv: H=%d N=%d CQ=%d", H, N, CQ);
+  for (int i = 0; i < 8; ++i)
+    T2T_REQUIRE(sd[i] >= 0 && sd[i] % 8 == 0 && (i % 2 == 0 || sd[i] >= TA_D),
+                "tile_attn_exact_orig_gather_kv: strides must be non-negative multiples of 8 "
+                "elements with row strides >= 128");
+  for (long long rs : {sd[3], sd[5]})
+    T2T_REQUIRE((unsigned long long)(N - 1) * (unsigned long long)rs * 2ull + 256ull <= 0xFFFFFFFFull,
+                "tile_attn_exact_orig_gather_kv: one head's K or V rows span (N - 1) * %lld "
+                "elements, more than 4 GiB", rs);
+  PlanView p = plan_view((int32_t*)plan, H, N, CQ);
+  hipStream_t st = (hipStream_t)stream;
+  const int S = qlab ? split_max(H, N, CQ) : 1;
+  const SplitWs w = split_layout(H, N, S, ws);
+  if (S > 1 && (!ws || ws_bytes < w.total)) {
+    t2t_set_error("tile_attn_exact_split: workspace %zu < %zu bytes", ws_bytes, w.total);
+    return T2T_ERR_WORKSPACE;
+  }
+  if (dtype == T2T_F16)
+    exact_launch<F16T>(mode, q, k, v, sd, kperm, kcounts, unip, qlab, qperm, p, out, lse, H, N, CQ, S,
+                       w, st);
+  else
+    exact_launch<BF16T>(mode, q, k, v, sd, kperm, kcounts, unip, qlab, qperm, p, out, lse, H, N, CQ, S,
+                        w, st);
+  T2T_LAUNCH_CHECK("tile_attn_exact_orig_gather_kv");
+  return T2T_OK;
+}
+
 extern "C" int t2t_tile_attn_exact_orig_gather_kv_strided(
     const void* q, long long q_head_stride, long long q_row_stride, const void* k,
     long long k_head_stride, long long k_row_stride, const void* v, long long v_head_stride,
@@ -1232,33 +1427,37 @@ extern "C" int t2t_tile_attn_exact_orig_gather_kv_strided(
     const int32_t* unip, const int32_t* qperm, const int32_t* plan, void* out,
     long long out_head_stride, long long out_row_stride, float* lse, int H, int N, int CQ,
     void* stream) {
-  T2T_REQUIRE(q && k && v && kperm && kcounts && unip && qperm && plan && out && lse,
-              "tile_attn_exact_orig_gather_kv: null pointer");
-  T2T_REQUIRE(check_dtype(dtype), "tile_attn_exact_orig_gather_kv: dtype %d", dtype);
-  T2T_REQUIRE(H > 0 && N > 0 && N < (1 << 24) && CQ > 0,
-              "tile_attn_exact_orig_gather_kv: H=%d N=%d CQ=%d", H, N, CQ);
-  const long long st4[8] = {q_head_stride, q_row_stride, k_head_stride, k_row_stride,
-                            v_head_stride, v_row_stride, out_head_stride, out_row_stride};
-  for (int i = 0; i < 8; ++i)
-    T2T_REQUIRE(st4[i] >= 0 && st4[i] % 8 == 0 && (i % 2 == 0 || st4[i] >= TA_D),
-                "tile_attn_exact_orig_gather_kv: strides must be non-negative multiples of 8 "
-                "elements with row strides >= 128");
-  for (long long rs : {k_row_stride, v_row_stride})
-    T2T_REQUIRE((unsigned long long)(N - 1) * (unsigned long long)rs * 2ull + 256ull <= 0xFFFFFFFFull,
-                "tile_attn_exact_orig_gather_kv: one head's K or V rows span (N - 1) * %lld "
-                "elements, more than 4 GiB", rs);
-  PlanView p = plan_view((int32_t*)plan, H, N, CQ);
-  hipStream_t st = (hipStream_t)stream;
-  if (dtype == T2T_F16)
-    launch_attn<F16T, 3>(q, k, v, unip, qperm, kcounts, p, nullptr, lse, out, H, N, CQ, st, kperm,
-                         q_head_stride, q_row_stride, k_head_stride, k_row_stride, out_head_stride,
-                         out_row_stride, v_head_stride, v_row_stride);
-  else
-    launch_attn<BF16T, 3>(q, k, v, unip, qperm, kcounts, p, nullptr, lse, out, H, N, CQ, st, kperm,
-                          q_head_stride, q_row_stride, k_head_stride, k_row_stride,
-                          out_head_stride, out_row_stride, v_head_stride, v_row_stride);
-  T2T_LAUNCH_CHECK("tile_attn_exact_orig_gather_kv");
-  return T2T_OK;
+  const long long sd[8] = {q_head_stride, q_row_stride, k_head_stride, k_row_stride,
+                           v_head_stride, v_row_stride, out_head_stride, out_row_stride};
+  return exact_impl(3, q, k, v, sd, kperm, dtype, kcounts, unip, nullptr, qperm, plan, out, lse, H, N,
+                    CQ, nullptr, 0, stream);
+}
+
+extern "C" size_t t2t_tile_attn_split_ws_bytes(int H, int N, int CQ) {
+  if (H <= 0 || N <= 0 || CQ <= 0) return 0;
+  const int S = split_max(H, N, CQ);
+  return S > 1 ? split_layout(H, N, S, nullptr).total : 0;
+}
+
+extern "C" int t2t_tile_attn_exact_split(
+    const void* q, long long q_head_stride, long long q_row_stride, const void* k,
+    long long k_head_stride, long long k_row_stride, const void* v, long long v_head_stride,
+    long long v_row_stride, const int32_t* kperm, int gather, int dtype, const int32_t* kcounts,
+    const int32_t* unip, const int32_t* qlab, const int32_t* qperm, const int32_t* plan, void* out,
+    long long out_head_stride, long long out_row_stride, float* lse, int H, int N, int CQ, void* ws,
+    size_t ws_bytes, void* stream) {
+  T2T_REQUIRE(qlab, "tile_attn_exact_split: null qlab");
+  T2T_REQUIRE(gather >= 0 && gather <= 2, "tile_attn_exact_split: gather=%d not in [0, 2]", gather);
+  // cluster-ordered rows are read from contiguous [H, N, 128] buffers
+  const long long hs = (long long)N * TA_D;
+  T2T_REQUIRE(gather >= 1 || (k_head_stride == hs && k_row_stride == TA_D),
+              "tile_attn_exact_split: cluster-ordered k must be contiguous");
+  T2T_REQUIRE(gather == 2 || (v_head_stride == hs && v_row_stride == TA_D),
+              "tile_attn_exact_split: cluster-ordered v must be contiguous");
+  const long long sd[8] = {q_head_stride, q_row_stride, k_head_stride, k_row_stride,
+                           v_head_stride, v_row_stride, out_head_stride, out_row_stride};
+  return exact_impl(1 + gather, q, k, v, sd, kperm, dtype, kcounts, unip, qlab, qperm, plan, out, lse,
+                    H, N, CQ, ws, ws_bytes, stream);
 }
 
 extern "C" int t2t_tile_attn_exact_orig(const void* q, const void* kp, const void* vp, int dtype,

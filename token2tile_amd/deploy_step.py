@@ -245,6 +245,9 @@ class MaskedStepDeploy:
         self._ctiles = torch.empty(ops.size_query("t2t_centroid_tiles_bytes", H), dtype=torch.uint8,
                                    device=dev)
 
+        # fp32 parts of the exact attention of a small call (empty otherwise)
+        self._ws_split = torch.empty(ops.attn_split_ws_bytes(H, N, CQ), dtype=torch.uint8, device=dev)
+
         self.cfg_reuse = bool(cfg_reuse)
         self.mask_refresh = max(1, int(mask_refresh))
         self._cfg_on = self.cfg_reuse or self.mask_refresh > 1
@@ -503,15 +506,11 @@ class MaskedStepDeploy:
             # (the centroid tile image after the side stream's value
             # statistics on reuse calls)
             with self._stage("attention_exact"):
-                if self._fused_kv:
-                    ops.tile_attn_exact_orig_gather_kv(q, k, v, kperm, counts, unip, qperm, plan,
-                                                       dst, self._lse, stream=s0)
-                elif self.fuse_k_gather:
-                    ops.tile_attn_exact_orig_gather(q, k, kperm, self._vp(v.dtype), counts, unip,
-                                                    qperm, plan, dst, self._lse, stream=s0)
-                else:
-                    ops.tile_attn_exact_orig(q, io["kp"], self._vp(v.dtype), counts, unip, qperm,
-                                             plan, dst, self._lse, stream=s0)
+                kk = k if self.fuse_k_gather else io["kp"]
+                vv = v if self._fused_kv else self._vp(v.dtype)
+                ops.tile_attn_exact_split(q, kk, vv, kperm, counts, unip, qlab_cur, qperm, plan, dst,
+                                          self._lse, ws=self._ws_split, stream=s0,
+                                          gather=int(self.fuse_k_gather) + int(self._fused_kv))
             if qu_ready is not None:
                 s0.wait_event(qu_ready)
             with self._stage("attention_prep"):

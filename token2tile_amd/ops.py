@@ -502,6 +502,36 @@ def tile_attn_exact_orig_gather_kv(q, k, v, kperm, kcounts, unip, qperm, plan, o
     return out
 
 
+def attn_split_ws_bytes(H, N, CQ):
+    """Workspace of tile_attn_exact_split (0: these sizes are not split)."""
+    return size_query("t2t_tile_attn_split_ws_bytes", H, N, CQ)
+
+
+def tile_attn_exact_split(q, k, v, kperm, kcounts, unip, qlab, qperm, plan, out, lse, ws=None,
+                          stream=None, gather=2):
+    """Exact attention at the original rows of out with the tasks of a small
+    call split along the keys (fp32 parts in ``ws``).  ``gather`` 2: as
+    tile_attn_exact_orig_gather_kv; 1: as tile_attn_exact_orig_gather (v is
+    cluster ordered); 0: as tile_attn_exact_orig (k and v are, kperm unused).
+    qlab are the labels that qperm sorts."""
+    H, N, D = q.shape
+    CQ = unip.shape[1]
+    dev = _dev(q)
+    sq = _rows(q, H, N, HEAD_DIM, _HALF, "q", dev)
+    sk = _rows(k, H, N, HEAD_DIM, q.dtype, "k", dev)
+    sv = _rows(v, H, N, HEAD_DIM, q.dtype, "v", dev)
+    so = _rows(out, H, N, HEAD_DIM, q.dtype, "out", dev)
+    _check_attn(dev, H, N, CQ, kcounts=kcounts, unip=unip, qlab=qlab, qperm=qperm, plan=plan,
+                lse=lse, dt=q.dtype)
+    if gather:
+        _check(kperm, (H, N), _i32, "kperm", dev)
+    ws = _ws_for(ws, attn_split_ws_bytes(H, N, CQ), dev)
+    call("t2t_tile_attn_exact_split", _lib.RowView(q), *sq, _lib.RowView(k), *sk, _lib.RowView(v),
+         *sv, kperm if gather else None, int(gather), dtype_code(q.dtype), kcounts, unip, qlab,
+         qperm, plan, _lib.RowView(out), *so, lse, H, N, CQ, ws, ws.numel(), stream_handle(stream))
+    return out
+
+
 def resid_merge_inplace(out, lse, QU, tiles, kcounts, unip, qlab, qperm, lam, tailw_t,
                         stream=None):
     """Residual + merge into the exact part held at the original rows of out
