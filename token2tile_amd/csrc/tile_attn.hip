@@ -1517,9 +1517,13 @@ extern "C" int t2t_resid_merge_inplace_strided(void* out, long long out_head_str
                             qlab, qperm, lam, tailw_dev, dtype, H, N, CQ, stream);
 }
 
+// lse, the centroid tile image, and the parts of a split call at the fewest
+// query clusters (the most parts)
 extern "C" size_t t2t_tile_attn_ws_bytes(int H, int N, int dtype) {
   (void)dtype;
-  return t2t_align256((size_t)H * N * sizeof(float)) + t2t_centroid_tiles_bytes(H);
+  if (H <= 0 || N <= 0) return 0;
+  return t2t_align256((size_t)H * N * sizeof(float)) + t2t_align256(t2t_centroid_tiles_bytes(H)) +
+         t2t_tile_attn_split_ws_bytes(H, N, 1);
 }
 
 extern "C" int t2t_tile_attn_run_planned(const void* q, const void* kp, const void* vp, int dtype,
@@ -1544,14 +1548,21 @@ extern "C" int t2t_tile_attn_run_planned(const void* q, const void* kp, const vo
     t2t_set_error("tile_attn_run_planned: workspace of %zu bytes, need %zu", ws_bytes, need);
     return T2T_ERR_WORKSPACE;
   }
-  float* lse = (float*)ws;
-  void* tiles = (char*)ws + t2t_align256((size_t)H * N * sizeof(float));
+  WsCarver w(ws);
+  float* lse = w.take<float>((size_t)H * N);
+  void* tiles = w.take<char>(t2t_centroid_tiles_bytes(H));
   PlanView p = plan_view(plan, H, N, CQ);
   launch_centroid_tiles(cks, sumv, tiles, H, st);
+  const long long hs = (long long)N * TA_D;
+  const long long sd[8] = {hs, TA_D, hs, TA_D, hs, TA_D, hs, TA_D};
+  const int S = split_max(H, N, CQ);
+  const SplitWs sw = split_layout(H, N, S, (char*)ws + w.off);
   if (dtype == T2T_F16)
-    launch_attn<F16T, 1>(q, kp, vp, unip, qperm, kcounts, p, nullptr, lse, out, H, N, CQ, st);
+    exact_launch<F16T>(1, q, kp, vp, sd, nullptr, kcounts, unip, qlab, qperm, p, out, lse, H, N, CQ, S,
+                       sw, st);
   else
-    launch_attn<BF16T, 1>(q, kp, vp, unip, qperm, kcounts, p, nullptr, lse, out, H, N, CQ, st);
+    exact_launch<BF16T>(1, q, kp, vp, sd, nullptr, kcounts, unip, qlab, qperm, p, out, lse, H, N, CQ, S,
+                        sw, st);
   launch_resid<false>(dtype, nullptr, lse, QU, tiles, kcounts, unip, qlab, qperm, lam, tailw_dev,
                       out, H, N, CQ, st);
   T2T_LAUNCH_CHECK("tile_attn_run_planned");
