@@ -300,14 +300,14 @@ int t2t_resid_merge_inplace(void* out, const float* lse, const void* QU, const v
                             const int32_t* kcounts, const int32_t* unip, const int32_t* qlab,
                             const int32_t* qperm, const float* lam, const float* tailw_dev,
                             int dtype, int H, int N, int CQ, void* stream);
-/* Workspace bytes of t2t_tile_attn_run_planned: lse [H, N] fp32 and the
- * centroid tile image. */
+/* Workspace bytes of t2t_tile_attn_run_planned: lse [H, N] fp32, the centroid
+ * tile image and the parts of a small call's split tasks. */
 size_t t2t_tile_attn_ws_bytes(int H, int N, int dtype);
 /* Plan (when rebuild_plan != 0), exact attention, residual and merge in
  * one call: the exact part is written to the original rows of out and the
  * residual kernel merges into them in place.  Replaces
  * tile_attn_ext.run_planned, kernels/tile_attn/src/main.cpp:67-79; ws holds
- * lse and the centroid tiles (the reference allocates attn_out and lse per
+ * lse, the centroid tiles and the parts of split tasks (the reference allocates attn_out and lse per
  * call). */
 int t2t_tile_attn_run_planned(const void* q, const void* kp, const void* vp, int dtype,
                               const int32_t* qcounts, const int32_t* kcounts,
@@ -318,6 +318,48 @@ int t2t_tile_attn_run_planned(const void* q, const void* kp, const void* vp, int
                               int32_t* plan, int rebuild_plan,
                               int H, int N, int CQ,
                               void* ws, size_t ws_bytes, void* stream);
+
+/* ---- one attention call ------------------------------------------------ */
+/* The stages of MaskedStepDeploy.step (operator/deploy_step.py:286-477), run in
+ * the order of their bits: a structure-rebuilding call is every bit but
+ * VSTATS, a reuse call PROJECT_Q | VSTATS (on any stream the RESIDUAL waits
+ * for) and EXACT | TILES | RESIDUAL.  Each stage is the entry point named, with
+ * its argument checks. */
+#define T2T_STEP_PROJECT_Q 1u  /* t2t_project_strided: q, Uq -> QU             */
+#define T2T_STEP_PROJECT_K 2u  /* t2t_project_strided: k, Uk -> KU             */
+#define T2T_STEP_KMEANS    4u  /* t2t_kmm_run_strided                          */
+#define T2T_STEP_VSTATS    8u  /* t2t_kmm_run_vstats_gather_strided            */
+#define T2T_STEP_FINALIZE 16u  /* t2t_centroid_finalize                        */
+#define T2T_STEP_SELECT   32u  /* t2t_score_select_packed, t2t_union_or_last   */
+#define T2T_STEP_GATHER_K 64u  /* t2t_fast_gather when kp is given             */
+#define T2T_STEP_PLAN    128u  /* t2t_tile_plan                                */
+#define T2T_STEP_EXACT   256u  /* t2t_tile_attn_exact_split                    */
+#define T2T_STEP_TILES   512u  /* t2t_centroid_tiles                           */
+#define T2T_STEP_RESIDUAL 1024u /* t2t_resid_merge_inplace_strided             */
+typedef struct t2t_step_args {
+  size_t struct_bytes; /* sizeof(t2t_step_args) */
+  int H, N, CQ, CK, dtype, pin_tail;
+  float scale;
+  const void *q, *k, *v; /* strided [H, N, 128] views */
+  void* out;
+  long long q_head_stride, q_row_stride, k_head_stride, k_row_stride, v_head_stride, v_row_stride,
+      out_head_stride, out_row_stride;
+  const void *Uq, *Uk, *cq0, *ck0;
+  void *QU, *KU;
+  void *kp, *vp; /* cluster-ordered K / V buffers, NULL: rows read in place */
+  int32_t *qlab, *klab, *qcounts, *qperm, *kcounts, *kperm, *unip, *rowcnt, *plan;
+  void *cq2, *ck16, *cks;
+  float* ck2;
+  void* sumv;
+  float* lam;
+  void* tiles;
+  float* lse;
+  const int32_t* ns;
+  const float* tailw;
+  void *ws_kmm, *ws_vst, *ws_sel, *ws_split;
+  size_t ws_kmm_bytes, ws_vst_bytes, ws_sel_bytes, ws_split_bytes;
+} t2t_step_args;
+int t2t_step(const t2t_step_args* args, unsigned stages, void* stream);
 
 /* ---- init_state helpers ----------------------------------------------- */
 /* labels[h, n] = nearest centroid of x[h, n] (||x||^2 - 2 x.c + ||c||^2,

@@ -220,3 +220,37 @@ def test_exact_split_matches_whole_tasks(dev, H, N, CQ, dtype):
     fin = lse[0].isfinite()
     assert torch.equal(fin, lse[1].isfinite())
     assert float((lse[0] - lse[1])[fin].abs().max()) <= 2 * u * 1.4427 * 1.01 + 2e-5
+
+
+def test_step_stages_and_streams(dev):
+    """One call's stages in one library call, launched stage by stage
+    (stage_events) and from another stream: same bits."""
+    from token2tile_amd.deploy_step import MaskedStepDeploy
+    from token2tile_amd.synth import generate
+    H, N, CQ = 2, 3000, 40
+    q, k, v = generate(H, N, grid=(1, 1, N), seed=3, device=dev, dtype=torch.bfloat16)
+    op = MaskedStepDeploy(H, N, CQ, s_frac=0.05, mask_refresh=4, device=dev)
+    state = op.init_state(q, k, seed=1)
+
+    def call(step, **kw):
+        op.set_cfg_call(0, key=0, step=step)
+        st = dict(state)
+        out = op.step(q, k, v, st, **kw).clone()
+        return out, st["ck"].clone(), st["cq"].clone()
+
+    full, reuse = call(0), call(1)
+    assert torch.equal(reuse[1], state["ck"])
+    op.stage_events = []
+    staged = call(4), call(5)
+    names = [n for n, _, _ in op.stage_events]
+    assert names == ["project", "kmeans", "score", "select", "plan", "attention_exact",
+                     "attention_prep", "attention_residual", "attention_exact", "attention_prep",
+                     "attention_residual"]
+    op.stage_events = None
+    side = torch.cuda.Stream(device=dev)
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        other = call(8), call(9)
+    torch.cuda.current_stream().wait_stream(side)
+    for a, b in (staged, other):
+        assert all(torch.equal(x, y) for x, y in zip(full + reuse, a + b))

@@ -19,6 +19,26 @@ LIB_PATH = Path(__file__).resolve().parent / "libt2t_hip.so"
 F16, BF16 = 0, 1
 _P = c_void_p
 
+class StepArgs(ctypes.Structure):
+    """t2t_step_args of include/t2t_hip.h."""
+    _fields_ = ([("struct_bytes", c_size_t)]
+                + [(n, c_int) for n in ("H", "N", "CQ", "CK", "dtype", "pin_tail")]
+                + [("scale", c_float)]
+                + [(n, _P) for n in ("q", "k", "v", "out")]
+                + [(f"{t}_{s}_stride", c_longlong) for t in ("q", "k", "v", "out")
+                   for s in ("head", "row")]
+                + [(n, _P) for n in ("Uq", "Uk", "cq0", "ck0", "QU", "KU", "kp", "vp", "qlab", "klab",
+                                     "qcounts", "qperm", "kcounts", "kperm", "unip", "rowcnt", "plan",
+                                     "cq2", "ck16", "cks", "ck2", "sumv", "lam", "tiles", "lse", "ns",
+                                     "tailw", "ws_kmm", "ws_vst", "ws_sel", "ws_split")]
+                + [(n, c_size_t) for n in ("ws_kmm_bytes", "ws_vst_bytes", "ws_sel_bytes",
+                                           "ws_split_bytes")])
+
+
+# the stages of t2t_step, in order
+(STEP_PROJECT_Q, STEP_PROJECT_K, STEP_KMEANS, STEP_VSTATS, STEP_FINALIZE, STEP_SELECT,
+ STEP_GATHER_K, STEP_PLAN, STEP_EXACT, STEP_TILES, STEP_RESIDUAL) = (1 << i for i in range(11))
+
 # name -> (restype, argtypes)
 SIGNATURES = {
     "t2t_last_error": (ctypes.c_char_p, []),
@@ -97,6 +117,7 @@ SIGNATURES = {
     "t2t_lloyd": (c_int, [_P, _P, c_int, c_int, c_int, c_int, c_int, _P, c_size_t, _P]),
     "t2t_gram_ws_bytes": (c_size_t, [c_int, c_int, c_int]),
     "t2t_gram": (c_int, [_P, c_int, _P, c_int, c_int, c_int, _P, c_size_t, _P]),
+    "t2t_step": (c_int, [ctypes.POINTER(StepArgs), ctypes.c_uint, _P]),
     "t2t_gram_strided": (c_int, [_P, c_int, c_longlong, c_longlong, _P, _P, c_int, c_int, c_int, _P,
                                  c_size_t, _P]),
     "t2t_fit_chol": (c_int, [_P, _P, _P, _P, c_int, c_int, c_double, _P]),

@@ -24,11 +24,14 @@ rebuilt every R annotated steps and reused in between (deploy_step.py:296-316).
 """
 from __future__ import annotations
 
+import ctypes
 import math
+import threading
+from contextlib import nullcontext
 
 import torch
 
-from . import ops
+from . import _lib, ops
 from .ops import fast_gather  # noqa: F401  (module surface of the reference)
 
 __all__ = ["MaskedStepDeploy", "online_u", "fast_assign", "fast_gather", "fused_update_vstats"]
@@ -230,7 +233,6 @@ class MaskedStepDeploy:
         # the value statistics of a reuse call then run on s_side beside the
         # exact attention.  False restores the V_sorted buffer
         self.fuse_v_gather = True
-        self._kmm_cq2 = torch.empty(H, CQ, r, device=dev, dtype=f16)
         self._kmm_ck2 = torch.empty(H, C, r, device=dev, dtype=f32)
         self._kmm_kcounts = torch.empty(H, C, device=dev, dtype=i32)
         self._kmm_sumv = torch.empty(H, C, D, device=dev, dtype=f16)
@@ -256,9 +258,27 @@ class MaskedStepDeploy:
         self._cfg_key = 0
         self._cfg_step = 0
 
+        # the fields of a call's arguments that never change: its own buffers
+        a = self._args = _lib.StepArgs()
+        a.struct_bytes = ctypes.sizeof(a)
+        a.H, a.N, a.CQ, a.CK, a.pin_tail, a.scale = H, N, CQ, C, self.pin_tail, self.scale
+        for name, t in (("QU", self.QU), ("KU", self.KU), ("rowcnt", self.rowcnt),
+                        ("ck2", self._kmm_ck2), ("sumv", self._kmm_sumv), ("lam", self._kmm_lam),
+                        ("tiles", self._ctiles), ("lse", self._lse)):
+            setattr(a, name, t.data_ptr())
+        for name, t in (("ws_kmm", self._ws_kmm), ("ws_vst", self._ws_vst),
+                        ("ws_sel", self._ws_sel), ("ws_split", self._ws_split)):
+            setattr(a, name, t.data_ptr())
+            setattr(a, name + "_bytes", t.numel())
+
         # default-priority streams (the two-stream schedule of the reference)
         self.s_main = torch.cuda.Stream(device=dev)
         self.s_side = torch.cuda.Stream(device=dev)
+        self._lock = threading.Lock()
+        # caller, fork, join, done (recorded once: torch creates the event then)
+        self._ev = [torch.cuda.Event() for _ in range(4)]
+        for ev in self._ev:
+            ev.record(self.s_main)
         self.last_call_full = None
         # optional list: (stage name, start event, end event) per launch group
         # recorded on s_main, for the benchmark's per-kernel timing
@@ -360,6 +380,18 @@ class MaskedStepDeploy:
         self._cfg_parity = None
 
     # -- the attention call (deploy_step.py:286-477) -------------------------
+    def _launch(self, args, stages, stream):
+        """Enqueue a call's stages on ``stream``: in one library call, or one
+        per named stage between its two events while stage_events is set."""
+        if self.stage_events is None or stream is not self.s_main:
+            stages = (("", sum(bits for _, bits in stages)),)
+        for name, bits in stages:
+            with self._stage(name) if name else nullcontext():
+                rc = _lib.lib().t2t_step(args, bits, stream.cuda_stream)
+            if rc != 0:
+                msg = _lib.lib().t2t_last_error().decode(errors="replace")
+                raise RuntimeError(f"t2t_step failed (code {rc}): {msg}")
+
     def step(self, q, k, v, state, out=None):
         """q, k, v: [H, N, 128] fp16 (or bf16), original row order: contiguous,
         or strided views with contiguous rows, such as token-major [N, H, 128]
@@ -368,14 +400,25 @@ class MaskedStepDeploy:
         holding the centroids that warm-start the next call.  Returns out
         [H, N, 128] in q's dtype: the given ``out`` view (written in place), or
         a buffer reused by the next call."""
+        with self._lock:  # the events and buffers serve one call at a time
+            return self._step(q, k, v, state, out)
+
+    def _step(self, q, k, v, state, out):
         H, N, C, CQ, D = self.H, self.N, self.C, self.CQ, self.D
         if not (q.dtype == k.dtype == v.dtype) or q.dtype not in (torch.float16, torch.bfloat16):
             raise TypeError("step: q, k, v must share dtype fp16 or bf16")
-        for name, t in (("q", q), ("k", k), ("v", v)) + ((("out", out),) if out is not None else ()):
+        a = _lib.StepArgs.from_buffer_copy(self._args)
+        a.dtype = _lib.dtype_code(q.dtype)
+        io = self._buffers(q.dtype)
+        dst = io["out"] if out is None else out
+        for name, t in (("q", q), ("k", k), ("v", v), ("out", dst)):
             try:
-                ops._rows(t, H, N, D, q.dtype, name, self.dev)
+                sh, sn = ops._rows(t, H, N, D, q.dtype, name, self.dev)
             except ValueError as e:
                 raise ValueError(f"step: {e}") from None
+            setattr(a, name, t.data_ptr())
+            setattr(a, name + "_head_stride", sh)
+            setattr(a, name + "_row_stride", sn)
         if not self.fuse_k_gather and not (q.is_contiguous() and k.is_contiguous()
                                            and (out is None or out.is_contiguous())):
             raise ValueError("step: strided q, k or out need fuse_k_gather (the separate gather "
@@ -389,12 +432,28 @@ class MaskedStepDeploy:
                     or t.device != self.dev):
                 raise ValueError(f"step: state[{name!r}] must be an fp16 {list(shape)} tensor on "
                                  f"{self.dev}")
+        ops._check(self.tailw_t, (), torch.float32, "tailw_t", self.dev)
+        a.tailw = self.tailw_t.data_ptr()
+        # with the separate gathers K and V are copied to cluster order first
+        if not self.fuse_k_gather:
+            a.kp = self._kp(k.dtype).data_ptr()
+        if not self._fused_kv:
+            a.vp = self._vp(v.dtype).data_ptr()
         caller = torch.cuda.current_stream(self.dev)
         s0, s1 = self.s_main, self.s_side
+        # this object's events order the streams; a call under graph capture
+        # takes events of its own, which live and die with that capture
+        capturing = torch.cuda.is_current_stream_capturing()
+
+        def after(waits, which, signals):
+            if capturing:
+                waits.wait_stream(signals)
+            else:
+                self._ev[which].record(signals)
+                waits.wait_event(self._ev[which])
+
         if caller != s0:
-            s0.wait_stream(caller)
-        io = self._buffers(q.dtype)
-        dst = io["out"] if out is None else out
+            after(s0, 0, caller)
 
         snap = None
         held = None
@@ -409,119 +468,85 @@ class MaskedStepDeploy:
         recycle = held is not None and snap is None
         self.last_call_full = snap is None
 
-        qu_ready = None
-        with torch.cuda.stream(s0):
-            if snap is not None:
-                # reuse: project with the snapshot's Uq, group K and V through
-                # the stored kperm, fresh value statistics from this call's V.
-                # Only the residual reads QU, sumv and lam: with the fused
-                # gathers the projection and the value statistics run on the
-                # side stream, under the exact attention.
-                s1.wait_stream(s0)
-                ops.project(q, snap["Uq"], out=self.QU, stream=s1)
-                if self._fused_kv:
-                    ops.vstats_gather(v, snap["kperm"], snap["counts"], sumv=self._kmm_sumv,
-                                      lam=self._kmm_lam, ws=self._ws_vst, stream=s1,
-                                      write_v_sorted=False)
-                qu_ready = torch.cuda.Event()
-                qu_ready.record(s1)
-                if not self.fuse_k_gather:
-                    with self._stage("gather_k"):
-                        ops.fast_gather(k, snap["kperm"], out=self._kp(k.dtype), stream=s0)
-                kperm = snap["kperm"]
-                if not self._fused_kv:
-                    with self._stage("vstats"):
-                        ops.vstats_gather(v, snap["kperm"], snap["counts"],
-                                          V_sorted=self._vp(v.dtype), sumv=self._kmm_sumv,
-                                          lam=self._kmm_lam, ws=self._ws_vst, stream=s0)
-                tile_sizes, qperm, counts = snap["tile_sizes"], snap["qperm"], snap["counts"]
-                qlab_cur, cks, unip = snap["qlab"], snap["cks"], snap["unip"]
-                plan, rebuild = snap["tile_attn_plan"], False
-            else:
-                with self._stage("project"):
-                    ops.project(q, state["Uq"], out=self.QU, stream=s0)
-                    ops.project(k, state["Uk"], out=self.KU, stream=s0)
+        if snap is not None:
+            st = snap
+            self._point(a, st)
+            a.Uq = st["Uq"].data_ptr()
+            # reuse: project with the snapshot's Uq, group K and V through the
+            # stored kperm, fresh value statistics from this call's V.  Only
+            # the residual reads QU, sumv and lam: with the fused gathers the
+            # projection and the value statistics run on the side stream,
+            # under the exact attention.
+            after(s1, 1, s0)
+            side = (("", _lib.STEP_PROJECT_Q),)
+            if self._fused_kv:
+                side += (("", _lib.STEP_VSTATS),)
+            self._launch(a, side, s1)
+            joined = torch.cuda.Event() if capturing else self._ev[2]
+            joined.record(s1)
+            main = ()
+            if not self.fuse_k_gather:
+                main += (("gather_k", _lib.STEP_GATHER_K),)
+            if not self._fused_kv:
+                main += (("vstats", _lib.STEP_VSTATS),)
+            self._launch(a, main + (("attention_exact", _lib.STEP_EXACT),), s0)
+            s0.wait_event(joined)
+        else:
+            for name in ("Uq", "Uk", "ck", "cq"):
+                if not state[name].is_contiguous():
+                    raise ValueError(f"step: state[{name!r}] must be contiguous")
+            ops._check_ns(self.ns_t, self.dev)
+            a.ns = self.ns_t.data_ptr()
+            a.Uq, a.Uk = state["Uq"].data_ptr(), state["Uk"].data_ptr()
+            a.cq0, a.ck0 = state["cq"].data_ptr(), state["ck"].data_ptr()
+            with torch.cuda.stream(s0):
+                e = lambda *shape, dtype=torch.int32: torch.empty(*shape, device=self.dev, dtype=dtype)  # noqa: E731
+                f16 = torch.float16
+                cq2, ck16, cks = (e(H, CQ, self.r, dtype=f16), e(H, C, self.r, dtype=f16),
+                                  e(H, C, self.r, dtype=f16))
                 if recycle:
-                    km_out = dict(qlab=held["qlab"], klab=held["klab"], qcounts=held["tile_sizes"],
-                                  qperm=held["qperm"], kperm=held["kperm"],
-                                  kcounts=held["counts"])
+                    st = dict(held, cks=cks)
                 else:
-                    km_out = dict(qlab=self.qlab, klab=self.klab,
-                                  qcounts=torch.empty(H, CQ, device=self.dev, dtype=torch.int32),
-                                  qperm=torch.empty(H, N, device=self.dev, dtype=torch.int32),
-                                  kperm=torch.empty(H, N, device=self.dev, dtype=torch.int32),
-                                  kcounts=self._kmm_kcounts)
-                km_out.update(cq2=self._kmm_cq2, ck2=self._kmm_ck2, sumv=self._kmm_sumv,
-                              lam=self._kmm_lam)
-                if not self._fused_kv:
-                    km_out.update(V_sorted=self._vp(v.dtype))
-                with self._stage("kmeans"):
-                    ops.kmm_run(self.QU, self.KU, v, state["cq"], state["ck"],
-                                pin_tail=self.pin_tail, out=km_out, ws=self._ws_kmm, stream=s0,
-                                write_v_sorted=not self._fused_kv)
-                tile_sizes, qperm, counts = km_out["qcounts"], km_out["qperm"], km_out["kcounts"]
-                with self._stage("score"):
-                    ck16, cks = ops.centroid_finalize(self._kmm_ck2, self.scale, stream=s0)
-                    state["ck"] = ck16
-                    state["cq"] = self._kmm_cq2.clone()
-                unip = held["unip"] if recycle else torch.empty(H, CQ, C // 32, device=self.dev,
-                                                                dtype=torch.int32)
+                    st = {"qlab": self.qlab, "klab": self.klab, "counts": self._kmm_kcounts,
+                          "tile_sizes": e(H, CQ), "qperm": e(H, N), "kperm": e(H, N),
+                          "unip": e(H, CQ, C // 32), "tile_attn_plan": e(self._tile_attn_plan_ints),
+                          "cks": cks}
+                self._point(a, st)
+                a.cq2, a.ck16 = cq2.data_ptr(), ck16.data_ptr()
                 # scores fp16(QU . cks^T) and the selection in one kernel: the
                 # [H, N, 2048] score tensor is never stored (the split variant
                 # of the reference yields the same bitmap, so split_cap has no
                 # effect here)
-                with self._stage("select"):
-                    ops.score_select(self.QU, cks, counts, qperm, tile_sizes, self.ns_t, unip=unip,
-                                     rowcnt=self.rowcnt, ws=self._ws_sel, stream=s0)
-                    if self.pin_tail:
-                        ops.union_or_last(unip, stream=s0)
-                if not self.fuse_k_gather:
-                    with self._stage("gather_k"):
-                        ops.fast_gather(k, km_out["kperm"], out=self._kp(k.dtype), stream=s0)
-                kperm = km_out["kperm"]
-                plan = (held["tile_attn_plan"] if recycle else
-                        torch.empty(self._tile_attn_plan_ints, device=self.dev, dtype=torch.int32))
-                rebuild = True
-                qlab_cur = km_out["qlab"]
+                gather = () if self.fuse_k_gather else (("gather_k", _lib.STEP_GATHER_K),)
+                self._launch(a, (("project", _lib.STEP_PROJECT_Q | _lib.STEP_PROJECT_K),
+                                 ("kmeans", _lib.STEP_KMEANS), ("score", _lib.STEP_FINALIZE),
+                                 ("select", _lib.STEP_SELECT), *gather, ("plan", _lib.STEP_PLAN),
+                                 ("attention_exact", _lib.STEP_EXACT)), s0)
+                state["ck"], state["cq"] = ck16, cq2
                 if self._cfg_on:
-                    self._cfg_hold[self._cfg_key] = {
-                        "qlab": qlab_cur if recycle else qlab_cur.clone(),
-                        "qperm": qperm,
-                        "tile_sizes": tile_sizes,
-                        "klab": km_out["klab"] if recycle else km_out["klab"].clone(),
-                        "kperm": km_out["kperm"],
-                        "counts": counts if recycle else counts.clone(),
-                        "cks": cks,
-                        "Uq": state["Uq"],
-                        "unip": unip,
-                        "tile_attn_plan": plan,
-                        "step": self._cfg_step,
-                    }
-            # step 5: plan (structure rebuilds only), exact attention over the
-            # unions, residual over the other clusters and the merge
-            if rebuild:
-                with self._stage("plan"):
-                    ops.tile_plan(tile_sizes, counts, unip, N, plan=plan, stream=s0)
-            # the steps of t2t_tile_attn_run_planned, one launch per stage
-            # (the centroid tile image after the side stream's value
-            # statistics on reuse calls)
-            with self._stage("attention_exact"):
-                kk = k if self.fuse_k_gather else io["kp"]
-                vv = v if self._fused_kv else self._vp(v.dtype)
-                ops.tile_attn_exact_split(q, kk, vv, kperm, counts, unip, qlab_cur, qperm, plan, dst,
-                                          self._lse, ws=self._ws_split, stream=s0,
-                                          gather=int(self.fuse_k_gather) + int(self._fused_kv))
-            if qu_ready is not None:
-                s0.wait_event(qu_ready)
-            with self._stage("attention_prep"):
-                ops.centroid_tiles(cks, self._kmm_sumv, tiles=self._ctiles, stream=s0)
-            with self._stage("attention_residual"):
-                ops.resid_merge_inplace(dst, self._lse, self.QU, self._ctiles, counts, unip,
-                                        qlab_cur, qperm, self._kmm_lam, self.tailw_t, stream=s0)
-        s1.wait_stream(s0)
-        cur = torch.cuda.current_stream(self.dev)
-        cur.wait_stream(s0)
-        cur.wait_stream(s1)
-        self._last = dict(unip=unip, qperm=qperm, tile_sizes=tile_sizes, counts=counts,
-                          qlab=qlab_cur, cks=cks, plan=plan, kperm=kperm)
+                    if recycle:
+                        own = st
+                    else:  # qlab, klab and counts are this object's own: copied
+                        own = dict(st, **{n: st[n].clone() for n in ("qlab", "klab", "counts")})
+                    self._cfg_hold[self._cfg_key] = dict(own, Uq=state["Uq"], step=self._cfg_step)
+        # the centroid tile image (after the side stream's value statistics on
+        # reuse calls), residual over the other clusters and the merge
+        self._launch(a, (("attention_prep", _lib.STEP_TILES),
+                         ("attention_residual", _lib.STEP_RESIDUAL)), s0)
+        if capturing:
+            s1.wait_stream(s0)
+            caller.wait_stream(s1)
+        if caller != s0:
+            after(caller, 3, s0)
+        self._last = dict(unip=st["unip"], qperm=st["qperm"], tile_sizes=st["tile_sizes"],
+                          counts=st["counts"], qlab=st["qlab"], cks=st["cks"],
+                          plan=st["tile_attn_plan"], kperm=st["kperm"])
         return dst
+
+    @staticmethod
+    def _point(a, st):
+        """The structure's tensors as call arguments."""
+        for name, key in (("qlab", "qlab"), ("klab", "klab"), ("qcounts", "tile_sizes"),
+                          ("qperm", "qperm"), ("kcounts", "counts"), ("kperm", "kperm"),
+                          ("unip", "unip"), ("plan", "tile_attn_plan"), ("cks", "cks")):
+            setattr(a, name, st[key].data_ptr())
