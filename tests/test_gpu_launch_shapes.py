@@ -254,3 +254,78 @@ def test_step_stages_and_streams(dev):
     torch.cuda.current_stream().wait_stream(side)
     for a, b in (staged, other):
         assert all(torch.equal(x, y) for x, y in zip(full + reuse, a + b))
+
+
+# one wave's sort, strides across waves, several keys per thread, more clusters
+# than key clusters, and a list past the sort's limit (cluster order)
+@pytest.mark.parametrize("H,N,CQ,kind", [(2, 5000, 1, "mix"), (2, 9000, 65, "mix"),
+                                         (3, 20000, 513, "mix"), (1, 30000, 2049, "mix"),
+                                         (1, 40000, 4096, "mix"), (1, 60000, 4096, "full")])
+def test_plan_order(dev, H, N, CQ, kind):
+    from token2tile_amd import ops
+    rng = np.random.default_rng(CQ)
+    lab = np.minimum(rng.integers(0, CQ, (H, N)), rng.integers(0, CQ, (H, N)))
+    if kind == "full":                         # every cluster, a few of them long
+        lab[:, :CQ] = np.arange(CQ)
+        lab[:, CQ:CQ + 3000] = 7
+    qcounts = np.stack([np.bincount(x, minlength=CQ) for x in lab]).astype(np.int32)
+    kcounts = np.stack([np.bincount(rng.integers(0, 2048, N) // 2 * 2, minlength=2048)
+                        for _ in range(H)]).astype(np.int32)
+    sel = rng.random((H, CQ, 2048)) < rng.choice([0.0, 0.05, 0.05, 1.0], (H, CQ, 1))
+    unip = np.packbits(sel.astype(np.uint8), axis=2, bitorder="little").view(np.int32)
+    plan = ops.tile_plan(g(qcounts, dev), g(kcounts, dev), g(unip, dev), N)
+    pv = {k: c(v) for k, v in ops.plan_views(plan, H, N, CQ).items()}
+    for h in range(H):
+        assert np.array_equal(pv["k_off"][h], np.concatenate([[0], np.cumsum(kcounts[h])]))
+        kv = np.where(qcounts[h] > 0, sel[h] @ kcounts[h], 0)
+        assert np.array_equal(pv["kvlen"][h], kv)
+        tasks, start = [], 0
+        for t, n in enumerate(qcounts[h]):
+            nt, nw = -(-n // 128), -(-n // 32)
+            s = start
+            for i in range(nt):
+                rows = min(32 * (nw // nt + (i < nw % nt)), start + n - s)
+                big = 32 * (nw // nt + (nw % nt > 0))
+                tasks.append((t, s, rows, big))
+                s += rows
+            start += n
+        if len(tasks) <= 4096:
+            tasks.sort(key=lambda x: -min(x[3] * int(kv[x[0]]), 2 ** 32 - 1))  # stable
+        else:
+            assert kind == "full"
+        assert pv["ntask"][h] == len(tasks)
+        assert np.array_equal(pv["tasks"][h][:len(tasks)], np.array(tasks))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_residual_groups(dev, dtype):
+    """288 work-groups walk all centroid tiles; a head alone has 32, whose two
+    wave groups share them.  Both round every weight to fp16 (a relative u)
+    against a max of their own, so each is within u (sum w |v| / sum w + |o|)
+    of the exact sums, and rounds the output once more."""
+    from token2tile_amd import ops
+    H, N, CQ = 9, 4000, 50
+    rng = np.random.default_rng(5)
+    qlab, _, qperm, qcounts, _, kcounts = structure(rng, H, N, CQ)
+    density = rng.choice([0.0, 0.1, 0.9, 1.0], (H, CQ, 1))
+    sel = (rng.random((H, CQ, 2048)) < density).astype(np.uint8)
+    sel[0, :, 1024:] = 1                       # nothing outside the union in the second half
+    unip = np.packbits(sel, axis=2, bitorder="little").view(np.int32)
+    gen = torch.Generator(device=dev).manual_seed(1)
+    r = lambda *s: torch.randn(*s, generator=gen, device=dev)  # noqa: E731
+    QU, cks, sumv = r(H, N, 32).half(), (0.1 * r(H, 2048, 32)).half(), r(H, 2048, 128).half()
+    exact, lse = r(H, N, 128).to(dtype), 9.0 + r(H, N)
+    lam, tw = torch.linspace(1, 2, H, device=dev), torch.tensor(0.7, device=dev)
+    tk, tu, tl, tp = g(kcounts, dev), g(unip, dev), g(qlab, dev), g(qperm, dev)
+
+    def merge(x, s, hs):
+        o = x[hs].clone()
+        tiles = ops.centroid_tiles(cks[hs].contiguous(), s[hs].contiguous())
+        return ops.resid_merge_inplace(o, lse[hs].contiguous(), QU[hs].contiguous(), tiles, tk[hs],
+                                       tu[hs], tl[hs], tp[hs], lam[hs], tw)
+    every = slice(0, H)
+    a, mean = merge(exact, sumv, every), merge(exact.abs(), sumv.abs(), every)
+    b = torch.cat([merge(exact, sumv, slice(h, h + 1)) for h in range(H)])
+    u = 2.0 ** -11
+    bound = 4 * u * 1.01 * mean.float() + 2.0 ** (-10 if dtype == torch.float16 else -7) * a.float().abs() + 1e-6
+    assert not a.isnan().any() and bool(((a - b).float().abs() <= bound).all())

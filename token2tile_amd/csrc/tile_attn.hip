@@ -62,6 +62,16 @@ extern "C" size_t t2t_tile_plan_ints(int H, int N, int CQ) {
 
 #define PLAN_SORT_MAX 4096
 
+// One work-group per head: its ~15 us are latency, of which reading a union
+// word per cluster one after the other and a barrier for every step of a
+// task sort were most (28 us at 201 clusters, 52 at 512, 77 at 768; now 17, 30, 40).  The words of
+// sixteen clusters are in flight per wave, and a word's clusters are summed from
+// the bit planes of their sizes (one bit count per plane that any size has,
+// not one LDS read per cluster); the clusters are sorted, not their tasks (a
+// cluster's tasks share its key and stay together), and the sort's strides
+// under 64 stay in a wave's registers.
+#define PLAN_KV 16      // clusters in flight per wave
+#define PLAN_PLANES 31  // bits of a cluster size
 __global__ __launch_bounds__(1024) void plan_kernel(const int32_t* __restrict__ qcounts,
                                                     const int32_t* __restrict__ kcounts,
                                                     const uint32_t* __restrict__ unip,
@@ -69,138 +79,191 @@ __global__ __launch_bounds__(1024) void plan_kernel(const int32_t* __restrict__ 
                                                     int32_t* __restrict__ kvlen,
                                                     int32_t* __restrict__ ntask,
                                                     int32_t* __restrict__ tasks, int CQ, int maxT) {
-  __shared__ int sk[TA_CK];
+  __shared__ int sk[PLAN_SORT_MAX];  // key-cluster sizes, then query-cluster starts
   __shared__ int wsum[16];
-  __shared__ int carry;
   __shared__ unsigned long long skey[PLAN_SORT_MAX];
+  static_assert(PLAN_SORT_MAX >= TA_CK, "the sizes fit");
+  // bit i of spl[b][l]: bit b of the size of cluster 32 l + i
+  __shared__ uint32_t spl[PLAN_PLANES][64];
+  __shared__ int nplane;
   const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  // exclusive block scan of one value per thread; *total = the sum
+  auto block_scan = [&](int v, int* total) {
+    const int inc = wave_incl_scan(v);
+    __syncthreads();  // wsum of the previous scan has been read
+    if (lane == 63) wsum[w] = inc;
+    __syncthreads();
+    int ex = inc - v, tot = 0;
+    for (int i = 0; i < 16; ++i) {
+      const int s = wsum[i];
+      ex += i < w ? s : 0;
+      tot += s;
+    }
+    *total = tot;
+    return ex;
+  };
   // key-cluster offsets (2 clusters per thread, in order)
   const int c0 = 2 * tid;
   const int a0 = kcounts[(size_t)h * TA_CK + c0], a1 = kcounts[(size_t)h * TA_CK + c0 + 1];
   sk[c0] = a0;
   sk[c0 + 1] = a1;
-  int inc = wave_incl_scan(a0 + a1);
-  if (lane == 63) wsum[w] = inc;
-  __syncthreads();
-  int ex = inc - a0 - a1;
-  for (int i = 0; i < w; ++i) ex += wsum[i];
+  int ktot;
+  const int ex = block_scan(a0 + a1, &ktot);
   int32_t* ko = k_off + (size_t)h * (TA_CK + 1);
   ko[c0] = ex;
   ko[c0 + 1] = ex + a0;
-  if (tid == 1023) ko[TA_CK] = ex + a0 + a1;
+  if (tid == 1023) ko[TA_CK] = ktot;
+  if (tid == 0) nplane = 0;
   __syncthreads();
-  // union lengths: one wave per query cluster
-  for (int t = w; t < CQ; t += 16) {
-    int s = 0;
-    if (qcounts[(size_t)h * CQ + t] > 0) {
-      uint32_t bits = unip[((size_t)h * CQ + t) * (TA_CK / 32) + lane];
-      while (bits) {
-        const int b = __builtin_ctz(bits);
-        s += sk[lane * 32 + b];
-        bits &= bits - 1;
-      }
+  for (int b = w; b < PLAN_PLANES; b += 16) {
+    uint32_t pl = 0;
+#pragma unroll
+    for (int i0 = 0; i0 < 32; ++i0) {
+      const int i = (i0 + lane) & 31;  // rotated: the lanes read distinct banks
+      pl |= (((uint32_t)sk[lane * 32 + i] >> b) & 1u) << i;
     }
-    s = wave_sum(s);
-    if (lane == 0) kvlen[(size_t)h * CQ + t] = s;
+    spl[b][lane] = pl;
+    if (__ballot(pl != 0u) != 0ull && lane == 0) atomicMax(&nplane, b + 1);
   }
   __syncthreads();
-  // task list: cluster t splits into ceil(n / QT) tasks of whole waves
-  if (tid == 0) carry = 0;
+  const int np = __builtin_amdgcn_readfirstlane(nplane);
+  // union lengths: one wave per query cluster
+  const int32_t* qc = qcounts + (size_t)h * CQ;
+  for (int t0 = w; t0 < CQ; t0 += 16 * PLAN_KV) {
+    uint32_t bits[PLAN_KV];
+    int n[PLAN_KV];
+#pragma unroll
+    for (int u = 0; u < PLAN_KV; ++u) {
+      const int t = t0 + 16 * u;
+      n[u] = t < CQ ? qc[t] : 0;
+      bits[u] = t < CQ ? unip[((size_t)h * CQ + t) * (TA_CK / 32) + lane] : 0u;
+    }
+#pragma unroll
+    for (int u = 0; u < PLAN_KV; ++u) {
+      const int t = t0 + 16 * u;
+      if (t >= CQ) break;
+      if (n[u] == 0) bits[u] = 0u;
+    }
+    int sum[PLAN_KV];
+#pragma unroll
+    for (int u = 0; u < PLAN_KV; ++u) sum[u] = 0;
+    for (int b = np - 1; b >= 0; --b) {
+      const uint32_t pl = spl[b][lane];
+#pragma unroll
+      for (int u = 0; u < PLAN_KV; ++u) sum[u] = 2 * sum[u] + __popc(bits[u] & pl);
+    }
+#pragma unroll
+    for (int u = 0; u < PLAN_KV; ++u) {
+      const int t = t0 + 16 * u;
+      if (t >= CQ) break;
+      const int s = wave_sum(sum[u]);
+      if (lane == 0) {
+        kvlen[(size_t)h * CQ + t] = s;
+        if (t < PLAN_SORT_MAX) skey[t] = (unsigned long long)(uint32_t)s;
+      }
+    }
+  }
+  // queries before each cluster (sorted order), in LDS over the sizes
   __syncthreads();
-  __shared__ int qcarry;
-  if (tid == 0) qcarry = 0;
-  __syncthreads();
-  int32_t* th = tasks + (size_t)h * maxT * 4;
+  int nT = 0, qrun = 0;
   for (int b0 = 0; b0 < CQ; b0 += 1024) {
     const int t = b0 + tid;
-    const int n = t < CQ ? qcounts[(size_t)h * CQ + t] : 0;
+    const int n = t < CQ ? qc[t] : 0;
+    const int nt = (n + TA_QT - 1) / TA_QT, nw = (n + 31) / 32;
+    int tot;
+    const int q0 = block_scan(n, &tot);
+    if (t < CQ && t < PLAN_SORT_MAX) {
+      sk[t] = qrun + q0;
+      // the cluster's sort key: (largest task rows) x kv_len, ties by the lower
+      // index (a thread per cluster: the divisions cost a wave as much as 64)
+      const int big = nt > 0 ? 32 * ((nw + nt - 1) / nt) : 0;
+      unsigned long long work = (unsigned long long)big * skey[t];
+      if (work > 0xFFFFFFFFull) work = 0xFFFFFFFFull;
+      skey[t] = (work << 32) | (unsigned long long)(0x7FFFFFFF - t);
+    }
+    qrun += tot;
+    int ntot;
+    block_scan(nt, &ntot);
+    nT += ntot;
+  }
+  if (tid == 0) ntask[h] = nT;
+  int P2 = 64;
+  while (P2 < CQ) P2 <<= 1;
+  for (int i = CQ + tid; i < P2 && i < PLAN_SORT_MAX; i += 1024) skey[i] = 0ull;
+  __syncthreads();
+  // LPT order: descending work, so the tasks of one query cluster, which
+  // stream the same key/value union, stay next to each other and run on one
+  // XCD (lists past PLAN_SORT_MAX tasks keep cluster order)
+  const bool sorted = nT <= PLAN_SORT_MAX && nT >= 2 && P2 <= PLAN_SORT_MAX;
+  if (sorted) {
+    // steps of strides j .. 1 of bitonic block size k on 64 consecutive keys
+    auto in_wave = [&](unsigned long long x, int i, int k, int j) {
+      for (; j > 0; j >>= 1) {
+        const unsigned long long y = __shfl_xor(x, j, 64);
+        const bool keep_max = ((i & j) == 0) == ((i & k) == 0);
+        x = keep_max == (x > y) ? x : y;
+      }
+      return x;
+    };
+    for (int i = tid; i < P2; i += 1024) {
+      unsigned long long x = skey[i];
+      for (int k = 2; k <= 64; k <<= 1) x = in_wave(x, i, k, k >> 1);
+      skey[i] = x;
+    }
+    __syncthreads();
+    for (int k = 128; k <= P2; k <<= 1) {
+      for (int j = k >> 1; j >= 64; j >>= 1) {
+        for (int i = tid; i < P2; i += 1024) {
+          const int ixj = i ^ j;
+          if (ixj > i) {
+            const unsigned long long x = skey[i], y = skey[ixj];
+            const bool desc = (i & k) == 0;
+            if (desc ? (x < y) : (x > y)) {
+              skey[i] = y;
+              skey[ixj] = x;
+            }
+          }
+        }
+        __syncthreads();
+      }
+      for (int i = tid; i < P2; i += 1024) skey[i] = in_wave(skey[i], i, k, 32);
+      __syncthreads();
+    }
+  }
+  // task list: cluster t splits into ceil(n / QT) tasks of whole waves
+  int32_t* th = tasks + (size_t)h * maxT * 4;
+  int trun = 0, qrun2 = 0;
+  for (int b0 = 0; b0 < CQ; b0 += 1024) {
+    const int i = b0 + tid;
+    const int t = i >= CQ ? -1 : (sorted ? 0x7FFFFFFF - (int)(skey[i] & 0xFFFFFFFFull) : i);
+    const int n = t >= 0 ? qc[t] : 0;
     const int nt = (n + TA_QT - 1) / TA_QT;
-    int ti = wave_incl_scan(nt);
-    int qi = wave_incl_scan(n);
-    __syncthreads();
-    if (lane == 63) wsum[w] = ti;
-    __syncthreads();
-    int tex = ti - nt + carry;
-    for (int i = 0; i < w; ++i) tex += wsum[i];
-    const int tot_t = [&] { int s = 0; for (int i = 0; i < 16; ++i) s += wsum[i]; return s; }();
-    __syncthreads();
-    if (lane == 63) wsum[w] = qi;
-    __syncthreads();
-    int qex = qi - n + qcarry;
-    for (int i = 0; i < w; ++i) qex += wsum[i];
-    const int tot_q = [&] { int s = 0; for (int i = 0; i < 16; ++i) s += wsum[i]; return s; }();
-    if (t < CQ && nt > 0) {
+    int tot;
+    const int tex = trun + block_scan(nt, &tot);
+    trun += tot;
+    int q0 = 0;
+    if (!sorted) {  // cluster order: the starts are this pass's own scan
+      q0 = qrun2 + block_scan(n, &tot);
+      qrun2 += tot;
+    } else if (nt > 0) {
+      q0 = sk[t];
+    }
+    if (nt > 0) {
       // the cluster's ceil(n / 32) waves of 32 queries are dealt evenly over
       // its tasks; only the last task holds a partial wave, so the tasks pad
       // no more query rows than the cluster needs (an even split of the rows
       // would pad every task's last wave)
       const int nw = (n + 31) / 32;
       const int base = nw / nt, rem = nw % nt;
-      int s = qex;
-      for (int i = 0; i < nt; ++i) {
-        const int rows = min(32 * (base + (i < rem ? 1 : 0)), qex + n - s);
-        int32_t* tk = th + (size_t)(tex + i) * 4;
-        tk[0] = t;
-        tk[1] = s;
-        tk[2] = rows;
-        tk[3] = 32 * (base + (rem > 0 ? 1 : 0));  // the cluster's largest task
+      int s = q0;
+      for (int j = 0; j < nt; ++j) {
+        const int rows = min(32 * (base + (j < rem ? 1 : 0)), q0 + n - s);
+        // the last entry: rows of the cluster's largest task
+        *(int4*)(th + (size_t)(tex + j) * 4) = make_int4(t, s, rows, 32 * (base + (rem > 0 ? 1 : 0)));
         s += rows;
       }
     }
-    __syncthreads();
-    if (tid == 0) {
-      carry += tot_t;
-      qcarry += tot_q;
-    }
-    __syncthreads();
   }
-  const int nT = carry;
-  if (tid == 0) ntask[h] = nT;
-  __syncthreads();
-  if (nT > PLAN_SORT_MAX || nT < 2) return;
-  // LPT order: descending (largest task rows of the cluster) x kv_len, ties
-  // by lower task index, so the tasks of one query cluster, which stream the
-  // same key/value union, stay next to each other and run on one XCD
-  int P2 = 2;
-  while (P2 < nT) P2 <<= 1;
-  for (int i = tid; i < P2; i += 1024) {
-    unsigned long long key = 0ull;
-    if (i < nT) {
-      const int32_t* tk = th + (size_t)i * 4;
-      unsigned long long work =
-          (unsigned long long)tk[3] * (unsigned long long)kvlen[(size_t)h * CQ + tk[0]];
-      if (work > 0xFFFFFFFFull) work = 0xFFFFFFFFull;
-      key = (work << 32) | (unsigned long long)(0x7FFFFFFF - i);
-    }
-    skey[i] = key;
-  }
-  __syncthreads();
-  for (int k = 2; k <= P2; k <<= 1) {
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      for (int i = tid; i < P2; i += 1024) {
-        const int ixj = i ^ j;
-        if (ixj > i) {
-          const unsigned long long x = skey[i], y = skey[ixj];
-          const bool desc = (i & k) == 0;
-          if (desc ? (x < y) : (x > y)) {
-            skey[i] = y;
-            skey[ixj] = x;
-          }
-        }
-      }
-      __syncthreads();
-    }
-  }
-  // permute in place through registers (<= 4 tasks per thread)
-  int4 mine[PLAN_SORT_MAX / 1024];
-  int nm = 0;
-  for (int i = tid; i < nT; i += 1024) {
-    const int src = 0x7FFFFFFF - (int)(skey[i] & 0xFFFFFFFFull);
-    mine[nm++] = *(const int4*)(th + (size_t)src * 4);
-  }
-  __syncthreads();
-  nm = 0;
-  for (int i = tid; i < nT; i += 1024) *(int4*)(th + (size_t)i * 4) = mine[nm++];
 }
 
 extern "C" int t2t_tile_plan(const int32_t* qcounts, const int32_t* kcounts, const int32_t* unip,
@@ -244,11 +307,15 @@ __host__ __device__ inline int split_parts(int kvlen, int S) {
   const int n = (kvlen + TA_KT - 1) / TA_KT / TA_SPLIT_TILES;
   return n < 1 ? 1 : (n < S ? n : S);
 }
-// Most parts per task (1: the call is not split): about three work-groups per
+// Most parts per task (1: the call is not split): about two work-groups per
 // slot, counting a task per 128 queries and half a task more per query cluster.
+// us unsplit / at 1, 2, 3, 4 work-groups per slot: 2 x 4096 92 / 53, 51, 50,
+// 50; 10 x 2351 60 / 59, 61, 83, 68; 2 x 16384 269 / 255, 151, 150, 157; 5 x
+// 16384 530 / 525, 399, 391, 415; 1 x 32760 345 / 189, 161, 168, 180; 5 x 32760
+// 990 unsplit, 1056 in halves.
 static int split_max(int H, int N, int CQ) {
   const long long tasks = (long long)H * (cdiv(N, TA_QT) + CQ / 2) + 1;
-  const long long S = (3 * 512 + tasks - 1) / tasks;
+  const long long S = (2 * 512 + tasks - 1) / tasks;
   return (int)(S < 1 ? 1 : (S > TA_SPLIT_MAX ? TA_SPLIT_MAX : S));
 }
 
@@ -1008,16 +1075,23 @@ __global__ __launch_bounds__(256) void centroid_tiles_kernel(const uint16_t* __r
 // its own cluster's union, so all waves carry real rows.  The exact part is
 // read from attn_out (sorted order, SRC_SORTED) or from the original rows of
 // out, and the merged result is written to the original rows of out.
-template <typename T, bool SRC_SORTED>
-__global__ __launch_bounds__(256, 3) void resid_kernel(
+//
+// G groups of four waves share the queries, each walking its share of the 32
+// centroid tiles; the first group adds the others' sums through LDS.  G = 2
+// where the work-groups do not outnumber the CUs (launch_resid): a tile's fetch,
+// scores, exponentials and products follow one another, so the launch lasts
+// for the chain of tiles (64 work-groups: 39 us in one chain, 33 in two; 256: 41.5,
+// 40).
+template <typename T, bool SRC_SORTED, int G>
+__global__ __launch_bounds__(256 * G, G == 1 ? 3 : 1) void resid_kernel(
     const uint16_t* __restrict__ exact, const float* __restrict__ lse2v,
     const uint16_t* __restrict__ QU, const uint16_t* __restrict__ tiles,
     const int32_t* __restrict__ kcounts, const uint32_t* __restrict__ unip,
     const int32_t* __restrict__ qlab, const int32_t* __restrict__ qperm,
     const float* __restrict__ lam, const float* __restrict__ tailw, uint16_t* __restrict__ out,
     int N, int CQ, long long soh, long long son) {
-  __shared__ __attribute__((aligned(1024))) uint16_t sT0[RT_HALVES];
-  __shared__ __attribute__((aligned(1024))) uint16_t sT1[RT_HALVES];
+  __shared__ __attribute__((aligned(1024))) uint16_t sT0[G * RT_HALVES];
+  __shared__ __attribute__((aligned(1024))) uint16_t sT1[G * RT_HALVES];
   // counts as fp16, ordered so that the 16 a lane weights in one 32-centroid
   // half are contiguous: centroid 64 t + 32 kb + 8 j + 4 hh + e sits at
   // 64 t + 32 kb + 16 hh + 4 j + e
@@ -1026,12 +1100,17 @@ __global__ __launch_bounds__(256, 3) void resid_kernel(
   // four consecutive centroids)
   __shared__ __attribute__((aligned(16))) float sMask[16 * 4];
   const int h = blockIdx.y;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3;
+  const int grp = G > 1 ? __builtin_amdgcn_readfirstlane(tid >> 8) : 0;
+  constexpr int TILES = RT_TILES / G;  // per group
+  static_assert(TILES % 2 == 0, "tiles go two at a time");
+  const int tc0 = grp * TILES;
   const int jl = lane & 31, hh = lane >> 5;
   const int row = blockIdx.x * 128 + wave * 32 + jl;  // sorted position
   const bool ok = row < N;
   const int orig = qperm[(size_t)h * N + (ok ? row : 0)];
-  const uint32_t* ur = unip + ((size_t)h * CQ + qlab[(size_t)h * N + orig]) * (TA_CK / 32);
+  const uint32_t* ur = unip + ((size_t)h * CQ + qlab[(size_t)h * N + orig]) * (TA_CK / 32) + 2 * tc0;
   u32x4 qu0, qu1;
   {
     const uint16_t* qr = QU + ((size_t)h * N + orig) * 32 + 8 * hh;
@@ -1040,9 +1119,9 @@ __global__ __launch_bounds__(256, 3) void resid_kernel(
   }
   const char* th = (const char*)(tiles + (size_t)h * RT_TILES * RT_HALVES) + wave * 1024 + lane * 16;
   auto issue = [&](int tc, auto BUF) {
-    uint16_t* sb = decltype(BUF)::value ? sT1 : sT0;
+    uint16_t* sb = (decltype(BUF)::value ? sT1 : sT0) + grp * RT_HALVES;
     // 1 KB per wave and instruction; the image's last 2 KB go to waves 0 and 1
-    const char* src = th + (size_t)tc * RT_BYTES;
+    const char* src = th + (size_t)(tc0 + tc) * RT_BYTES;
 #pragma unroll
     for (int i = 0; i < RT_BYTES / 4096; ++i)
       __builtin_amdgcn_global_load_lds((const glb_void_t*)(src + i * 4096),
@@ -1056,8 +1135,8 @@ __global__ __launch_bounds__(256, 3) void resid_kernel(
   using B1 = std::integral_constant<int, 1>;
   issue(0, B0{});
 #pragma unroll
-  for (int i = 0; i < TA_CK / 256; ++i) {
-    const int c = tid + 256 * i;
+  for (int i = 0; i < TA_CK / (256 * G); ++i) {
+    const int c = tid + 256 * G * i;
     const int pos = (c & ~31) + 16 * ((c >> 2) & 1) + 4 * ((c >> 3) & 3) + (c & 3);
     sCnt[pos] = F16T::from_f((float)kcounts[(size_t)h * TA_CK + c]);
   }
@@ -1088,10 +1167,10 @@ __global__ __launch_bounds__(256, 3) void resid_kernel(
   f32x16 Snext = mask_init(uw0);
   auto body = [&](int tc, auto BUF) {
     constexpr int buf = decltype(BUF)::value;
-    const uint16_t* sb = buf ? sT1 : sT0;
-    if (tc + 1 < RT_TILES) issue(tc + 1, std::integral_constant<int, buf ^ 1>{});
+    const uint16_t* sb = (buf ? sT1 : sT0) + grp * RT_HALVES;
+    if (tc + 1 < TILES) issue(tc + 1, std::integral_constant<int, buf ^ 1>{});
     uint32_t nw0 = 0, nw1 = 0;
-    if (tc + 1 < RT_TILES) {
+    if (tc + 1 < TILES) {
       nw0 = ur[2 * tc + 2];
       nw1 = ur[2 * tc + 3];
     }
@@ -1127,7 +1206,7 @@ __global__ __launch_bounds__(256, 3) void resid_kernel(
       // rescaled.  An empty cluster's weight can pass unseen only while finite.
       // The exponent argument reads the fp16 halves directly (v_fma_mix_f32).
       u32x4 pb[2];
-      const u32x4* cw = (const u32x4*)(sCnt + TL_CT * tc + 32 * kb + 16 * hh);
+      const u32x4* cw = (const u32x4*)(sCnt + TL_CT * (tc0 + tc) + 32 * kb + 16 * hh);
       const u32x4 cn0 = cw[0], cn1 = cw[1];
       auto expo = [&](float nm) {
         float ph = 0.f;
@@ -1184,9 +1263,55 @@ __global__ __launch_bounds__(256, 3) void resid_kernel(
     __builtin_amdgcn_s_waitcnt(0);  // tile tc + 1 landed
     __syncthreads();
   };
-  for (int tc = 0; tc < RT_TILES; tc += 2) {
+  for (int tc = 0; tc < TILES; tc += 2) {
     body(tc, B0{});
     body(tc + 1, B1{});
+  }
+  if constexpr (G > 1) {
+    // the second group's sums, half of the dims at a time, in the LDS of the
+    // first tiles (every wave is past its last tile): rows padded to 68 floats
+    static_assert(G == 2 && 128 * 68 * 4 <= G * RT_BYTES, "the sums fit");
+    float* sO = (float*)sT0 + (wave * 32 + jl) * 68 + 4 * hh;
+    float* sMP = (float*)sT1 + 4 * (wave * 64 + lane);
+    float sa = 1.f, sb = 1.f;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      if (grp == 1) {
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const f32x16& o = O[2 * half + nb];
+            *(f32x4*)(sO + 32 * nb + 8 * g) =
+                f32x4{o[4 * g], o[4 * g + 1], o[4 * g + 2], o[4 * g + 3]};
+          }
+        if (half == 0) {
+          sMP[0] = m2;
+          sMP[1] = phi;
+        }
+      }
+      __syncthreads();
+      if (grp == 0) {
+        if (half == 0) {
+          const float mb = sMP[0], M = fmaxf(m2, mb);
+          sa = __builtin_amdgcn_exp2f((m2 - M) * L2E);
+          sb = __builtin_amdgcn_exp2f((mb - M) * L2E);
+          phi = fmaf(sb, sMP[1], sa * phi);
+          m2 = M;
+        }
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const f32x4 v = *(const f32x4*)(sO + 32 * nb + 8 * g);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              O[2 * half + nb][4 * g + e] = fmaf(sb, v[e], sa * O[2 * half + nb][4 * g + e]);
+          }
+      }
+      if (half == 0) __syncthreads();
+    }
+    if (grp > 0) return;
   }
   if (!ok) return;
   // ---- merge under one softmax
@@ -1265,16 +1390,17 @@ static void launch_resid(int dtype, const void* exact, const float* lse, const v
                          long long soh = -1, long long son = TA_D) {
   const dim3 grid(cdiv(N, 128), H);
   if (soh < 0) soh = (long long)N * TA_D;
-  if (dtype == T2T_F16)
-    hipLaunchKernelGGL((resid_kernel<F16T, SRC_SORTED>), grid, dim3(256), 0, st,
-                       (const uint16_t*)exact, lse, (const uint16_t*)QU, (const uint16_t*)tiles,
-                       kcounts, (const uint32_t*)unip, qlab, qperm, lam, tailw, (uint16_t*)out, N,
-                       CQ, soh, son);
-  else
-    hipLaunchKernelGGL((resid_kernel<BF16T, SRC_SORTED>), grid, dim3(256), 0, st,
-                       (const uint16_t*)exact, lse, (const uint16_t*)QU, (const uint16_t*)tiles,
-                       kcounts, (const uint32_t*)unip, qlab, qperm, lam, tailw, (uint16_t*)out, N,
-                       CQ, soh, son);
+#define RS_LAUNCH(T, G)                                                                            \
+  hipLaunchKernelGGL((resid_kernel<T, SRC_SORTED, G>), grid, dim3(256 * G), 0, st,                 \
+                     (const uint16_t*)exact, lse, (const uint16_t*)QU, (const uint16_t*)tiles,     \
+                     kcounts, (const uint32_t*)unip, qlab, qperm, lam, tailw, (uint16_t*)out, N,   \
+                     CQ, soh, son)
+  if ((long long)grid.x * H <= 256) {
+    if (dtype == T2T_F16) RS_LAUNCH(F16T, 2); else RS_LAUNCH(BF16T, 2);
+  } else {
+    if (dtype == T2T_F16) RS_LAUNCH(F16T, 1); else RS_LAUNCH(BF16T, 1);
+  }
+#undef RS_LAUNCH
 }
 
 extern "C" size_t t2t_tail_merge_ws_bytes(int H) { return t2t_centroid_tiles_bytes(H); }
