@@ -223,8 +223,8 @@ def test_exact_split_matches_whole_tasks(dev, H, N, CQ, dtype):
 
 
 def test_step_stages_and_streams(dev):
-    """One call's stages in one library call, launched stage by stage
-    (stage_events) and from another stream: same bits."""
+    """One call's stages in one library call (sharing kernels), launched stage by
+    stage (stage_events) and from another stream: same bits."""
     from token2tile_amd.deploy_step import MaskedStepDeploy
     from token2tile_amd.synth import generate
     H, N, CQ = 2, 3000, 40
@@ -244,7 +244,7 @@ def test_step_stages_and_streams(dev):
     staged = call(4), call(5)
     names = [n for n, _, _ in op.stage_events]
     assert names == ["project", "kmeans", "score", "select", "plan", "attention_exact",
-                     "attention_prep", "attention_residual", "attention_exact", "attention_prep",
+                     "attention_prep", "attention_residual", "attention_exact",
                      "attention_residual"]
     op.stage_events = None
     side = torch.cuda.Stream(device=dev)

@@ -92,11 +92,20 @@ __global__ __launch_bounds__(256) void project_kernel(const uint16_t* __restrict
 #define PJ_VMCNT(n) (((n) & 0xf) | (0x7 << 4) | (0xf << 8) | ((((n) >> 4) & 0x3) << 14))
 typedef __attribute__((address_space(3))) void pj_lds_t;
 typedef __attribute__((address_space(1))) void pj_glb_t;
+// A launch takes one or two tensors (blockIdx.z): a call's q and k.
+struct ProjArgs {
+  const uint16_t* x;
+  const uint16_t* U;
+  uint16_t* out;
+  long long sxh, sxn;
+};
 template <typename T>
-__global__ __launch_bounds__(256, 2) void project_lds_kernel(const uint16_t* __restrict__ x,
-                                                             const uint16_t* __restrict__ U,
-                                                             uint16_t* __restrict__ out, int N,
-                                                             long long sxh, long long sxn) {
+__global__ __launch_bounds__(256, 2) void project_lds_kernel(ProjArgs g0, ProjArgs g1, int N) {
+  const ProjArgs& ga = blockIdx.z ? g1 : g0;
+  const uint16_t* __restrict__ x = ga.x;
+  const uint16_t* __restrict__ U = ga.U;
+  uint16_t* __restrict__ out = ga.out;
+  const long long sxh = ga.sxh, sxn = ga.sxn;
   constexpr int D = 128, KS = D / 16;
   __shared__ __attribute__((aligned(1024))) uint16_t sX0[4][32 * D];
   __shared__ __attribute__((aligned(1024))) uint16_t sX1[4][32 * D];
@@ -227,9 +236,11 @@ static int launch_project(const void* x, const void* U, void* out, int H, int N,
   dim3 grid(gx, H);
   switch (D) {
     case 128:
-      hipLaunchKernelGGL((project_lds_kernel<T>), grid, dim3(256), 0, st, (const uint16_t*)x,
-                         (const uint16_t*)U, (uint16_t*)out, N, sxh, sxn);
+    {
+      const ProjArgs g{(const uint16_t*)x, (const uint16_t*)U, (uint16_t*)out, sxh, sxn};
+      hipLaunchKernelGGL((project_lds_kernel<T>), grid, dim3(256), 0, st, g, g, N);
       break;
+    }
     case 64:
       hipLaunchKernelGGL((project_kernel<T, 64>), grid, dim3(256), 0, st, (const uint16_t*)x,
                          (const uint16_t*)U, (uint16_t*)out, N, sxh, sxn);
@@ -242,6 +253,29 @@ static int launch_project(const void* x, const void* U, void* out, int H, int N,
       t2t_set_error("project: D=%d not in {32, 64, 128}", D);
       return T2T_ERR_UNSUPPORTED;
   }
+  T2T_LAUNCH_CHECK("project");
+  return T2T_OK;
+}
+
+int t2t_project_pair(const void* q, long long sqh, long long sqn, const void* Uq, void* QU,
+                     const void* k, long long skh, long long skn, const void* Uk, void* KU, int dtype,
+                     int H, int N, void* stream) {
+  T2T_REQUIRE(q && k && Uq && Uk && QU && KU, "project: null pointer");
+  T2T_REQUIRE(H > 0 && N > 0, "project: H=%d N=%d", H, N);
+  T2T_REQUIRE(dtype == T2T_F16 || dtype == T2T_BF16, "project: dtype %d", dtype);
+  for (long long s : {sqn, skn}) T2T_REQUIRE(s >= 128 && s % 8 == 0, "project: row stride %lld", s);
+  for (long long s : {sqh, skh}) T2T_REQUIRE(s >= 0 && s % 8 == 0, "project: head stride %lld", s);
+  int gx = cdiv(N, 128);
+  const int cap = (T2T_PROJ_WGS + H - 1) / H;
+  if (gx > cap) gx = cap;
+  const ProjArgs g0{(const uint16_t*)q, (const uint16_t*)Uq, (uint16_t*)QU, sqh, sqn};
+  const ProjArgs g1{(const uint16_t*)k, (const uint16_t*)Uk, (uint16_t*)KU, skh, skn};
+  if (dtype == T2T_F16)
+    hipLaunchKernelGGL(project_lds_kernel<F16T>, dim3(gx, H, 2), dim3(256), 0, (hipStream_t)stream, g0,
+                       g1, N);
+  else
+    hipLaunchKernelGGL(project_lds_kernel<BF16T>, dim3(gx, H, 2), dim3(256), 0, (hipStream_t)stream, g0,
+                       g1, N);
   T2T_LAUNCH_CHECK("project");
   return T2T_OK;
 }

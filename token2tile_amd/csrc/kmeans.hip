@@ -808,7 +808,8 @@ __global__ __launch_bounds__(256) void key_gather_kernel(
     const int32_t* __restrict__ perm, const int32_t* __restrict__ counts,
     const int32_t* __restrict__ cbase, const uint16_t* __restrict__ ck0, float* __restrict__ ck2,
     uint16_t* __restrict__ V_sorted, float* __restrict__ vsum, float* __restrict__ cmax, int N,
-    int C, long long svh, long long svn) {
+    int C, long long svh, long long svn, uint16_t* __restrict__ ck16, uint16_t* __restrict__ cks,
+    float scale) {
   const int h = blockIdx.y;
   const int l = threadIdx.x & 63;
   const int c = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -888,8 +889,15 @@ __global__ __launch_bounds__(256) void key_gather_kernel(
   }
   if (ck2 && l < 16) {
     const size_t o = ((size_t)h * C + c) * KM_R + 2 * l;
-    ck2[o] = n ? ax0 / (float)n : h2f(ck0[o]);
-    ck2[o + 1] = n ? ax1 / (float)n : h2f(ck0[o + 1]);
+    const float m0 = opaque(n ? ax0 / (float)n : h2f(ck0[o]));
+    const float m1 = opaque(n ? ax1 / (float)n : h2f(ck0[o + 1]));
+    ck2[o] = m0;
+    ck2[o + 1] = m1;
+    if (ck16) {  // the finalised centroids as well (centroid_finalize_kernel)
+      *(uint32_t*)(ck16 + o) = (uint32_t)f2h(m0) | ((uint32_t)f2h(m1) << 16);
+      *(uint32_t*)(cks + o) =
+          (uint32_t)f2h(opaque(m0 * scale)) | ((uint32_t)f2h(opaque(m1 * scale)) << 16);
+    }
   }
 }
 
@@ -931,7 +939,11 @@ __global__ __launch_bounds__(1024) void vstats_kernel(const float* __restrict__ 
   }
 }
 static void launch_vstats(const float* vsum, const float* cmax, void* sumv, float* lam, int H,
-                          int C, hipStream_t st) {
+                          int C, const T2tCentroidOut& co, hipStream_t st) {
+  if (co.tiles) {  // with the tile image that holds the same sums
+    t2t_launch_vstats_tiles(vsum, cmax, co.cks, sumv, lam, co.tiles, H, st);
+    return;
+  }
   hipLaunchKernelGGL(vstats_kernel, dim3(cdiv(C * 128, 1024 * VS_PER), H), dim3(1024), 0, st,
                      vsum, cmax, (uint16_t*)sumv, lam, C);
 }
@@ -1031,10 +1043,12 @@ template <typename T>
 static void launch_key_gather(const void* KU, const void* V, const int32_t* perm,
                               const int32_t* counts, const int32_t* cbase, const void* ck0,
                               float* ck2, void* V_sorted, float* vsum, float* cmax, int H, int N,
-                              int C, long long svh, long long svn, hipStream_t st) {
+                              int C, long long svh, long long svn, const T2tCentroidOut& co,
+                              hipStream_t st) {
   hipLaunchKernelGGL((key_gather_kernel<T, false>), dim3(cdiv(C, 4), H), dim3(256), 0, st,
                      (const uint16_t*)KU, (const uint16_t*)V, perm, counts, cbase,
-                     (const uint16_t*)ck0, ck2, (uint16_t*)V_sorted, vsum, cmax, N, C, svh, svn);
+                     (const uint16_t*)ck0, ck2, (uint16_t*)V_sorted, vsum, cmax, N, C, svh, svn,
+                     (uint16_t*)co.ck16, (uint16_t*)co.cks, co.scale);
 }
 
 #define KM_CHECK(x)            \
@@ -1048,7 +1062,8 @@ static int kmm_impl(const void* QU, const void* KU, const void* V, int v_dtype,
                     float* ck2, int32_t* qcounts, int32_t* qperm, int32_t* kcounts,
                     int32_t* kperm, void* V_sorted, void* sumv, float* lam, int H, int N, int CQ,
                     int CK, int pin_tail, void* ws, size_t ws_bytes, long long svh,
-                    long long svn, void* stream) {
+                    long long svn, const T2tCentroidOut& co, void* stream) {
+  T2T_REQUIRE(!co.tiles || CK == 2048, "kmm_run: the tile image holds 2048 clusters, not %d", CK);
   T2T_REQUIRE(QU && KU && V && cq0 && ck0 && qlab && cq2 && klab && ck2 && qcounts && qperm &&
                   kcounts && kperm && sumv && lam,
               "kmm_run: null pointer");  // V_sorted may be NULL: not written
@@ -1093,12 +1108,12 @@ static int kmm_impl(const void* QU, const void* KU, const void* V, int v_dtype,
   // key sums and value statistics
   if (v_dtype == T2T_F16)
     launch_key_gather<F16T>(KU, V, kperm, kcounts, w.cbasek, ck0, ck2, V_sorted, w.vsum, w.cmax, H, N, CK,
-                            svh, svn, st);
+                            svh, svn, co, st);
   else
     launch_key_gather<BF16T>(KU, V, kperm, kcounts, w.cbasek, ck0, ck2, V_sorted, w.vsum, w.cmax, H, N, CK,
-                             svh, svn, st);
+                             svh, svn, co, st);
   T2T_LAUNCH_CHECK("key gather");
-  launch_vstats(w.vsum, w.cmax, sumv, lam, H, CK, st);
+  launch_vstats(w.vsum, w.cmax, sumv, lam, H, CK, co, st);
   T2T_LAUNCH_CHECK("vstats");
   return T2T_OK;
 }
@@ -1111,7 +1126,7 @@ extern "C" int t2t_kmm_run(const void* QU, const void* KU, const void* V, int v_
                            size_t ws_bytes, void* stream) {
   return kmm_impl(QU, KU, V, v_dtype, cq0, ck0, qlab, cq2, klab, ck2, qcounts, qperm, kcounts,
                   kperm, V_sorted, sumv, lam, H, N, CQ, CK, pin_tail, ws, ws_bytes,
-                  (long long)N * 128, 128, stream);
+                  (long long)N * 128, 128, T2tCentroidOut{}, stream);
 }
 
 extern "C" int t2t_kmm_run_strided(const void* QU, const void* KU, const void* V, int v_dtype,
@@ -1123,7 +1138,16 @@ extern "C" int t2t_kmm_run_strided(const void* QU, const void* KU, const void* V
                                    void* ws, size_t ws_bytes, void* stream) {
   return kmm_impl(QU, KU, V, v_dtype, cq0, ck0, qlab, cq2, klab, ck2, qcounts, qperm, kcounts,
                   kperm, V_sorted, sumv, lam, H, N, CQ, CK, pin_tail, ws, ws_bytes, v_head_stride,
-                  v_row_stride, stream);
+                  v_row_stride, T2tCentroidOut{}, stream);
+}
+
+int t2t_kmm_run_out(const void* QU, const void* KU, const void* V, int v_dtype, long long svh,
+                    long long svn, const void* cq0, const void* ck0, int32_t* qlab, void* cq2,
+                    int32_t* klab, float* ck2, int32_t* qcounts, int32_t* qperm, int32_t* kcounts,
+                    int32_t* kperm, void* V_sorted, void* sumv, float* lam, int H, int N, int CQ, int CK,
+                    int pin_tail, void* ws, size_t ws_bytes, const T2tCentroidOut& co, void* stream) {
+  return kmm_impl(QU, KU, V, v_dtype, cq0, ck0, qlab, cq2, klab, ck2, qcounts, qperm, kcounts, kperm,
+                  V_sorted, sumv, lam, H, N, CQ, CK, pin_tail, ws, ws_bytes, svh, svn, co, stream);
 }
 
 // ---- value statistics of a reuse call ----
@@ -1150,7 +1174,9 @@ extern "C" size_t t2t_vstats_ws_bytes(int H, int N, int CK) {
 
 static int vstats_common(const void* V, int v_dtype, const int32_t* kperm, const int32_t* kcounts,
                          void* V_sorted, void* sumv, float* lam, int H, int N, int CK, void* ws,
-                         size_t ws_bytes, long long svh, long long svn, hipStream_t st) {
+                         size_t ws_bytes, long long svh, long long svn, const T2tCentroidOut& co,
+                         hipStream_t st) {
+  T2T_REQUIRE(!co.tiles || (CK == 2048 && co.cks), "vstats: the tile image holds 2048 clusters");
   T2T_REQUIRE(V && kcounts && sumv && lam, "vstats: null pointer");
   T2T_REQUIRE(v_dtype == T2T_F16 || v_dtype == T2T_BF16, "vstats: dtype %d", v_dtype);
   T2T_REQUIRE(H > 0 && N > 0 && CK >= 1 && CK <= KM_MAXC, "vstats: H=%d N=%d CK=%d", H, N, CK);
@@ -1165,11 +1191,11 @@ static int vstats_common(const void* V, int v_dtype, const int32_t* kperm, const
   hipLaunchKernelGGL(cbase_kernel, dim3(H), dim3(1024), 0, st, kcounts, w.cbase, CK);
   if (v_dtype == T2T_F16)
     launch_key_gather<F16T>(nullptr, V, kperm, kcounts, w.cbase, nullptr, nullptr, V_sorted,
-                            w.vsum, w.cmax, H, N, CK, svh, svn, st);
+                            w.vsum, w.cmax, H, N, CK, svh, svn, T2tCentroidOut{}, st);
   else
     launch_key_gather<BF16T>(nullptr, V, kperm, kcounts, w.cbase, nullptr, nullptr, V_sorted,
-                             w.vsum, w.cmax, H, N, CK, svh, svn, st);
-  launch_vstats(w.vsum, w.cmax, sumv, lam, H, CK, st);
+                             w.vsum, w.cmax, H, N, CK, svh, svn, T2tCentroidOut{}, st);
+  launch_vstats(w.vsum, w.cmax, sumv, lam, H, CK, co, st);
   T2T_LAUNCH_CHECK("vstats");
   return T2T_OK;
 }
@@ -1180,7 +1206,7 @@ extern "C" int t2t_kmm_run_vstats_gather(const void* V, int v_dtype, const int32
                                          size_t ws_bytes, void* stream) {
   T2T_REQUIRE(kperm, "vstats_gather: null kperm");  // V_sorted may be NULL: not written
   return vstats_common(V, v_dtype, kperm, kcounts, V_sorted, sumv, lam, H, N, CK, ws, ws_bytes,
-                       (long long)N * 128, 128, (hipStream_t)stream);
+                       (long long)N * 128, 128, T2tCentroidOut{}, (hipStream_t)stream);
 }
 
 extern "C" int t2t_kmm_run_vstats_gather_strided(const void* V, int v_dtype,
@@ -1191,14 +1217,23 @@ extern "C" int t2t_kmm_run_vstats_gather_strided(const void* V, int v_dtype,
                                                  void* stream) {
   T2T_REQUIRE(kperm, "vstats_gather: null kperm");  // V_sorted may be NULL: not written
   return vstats_common(V, v_dtype, kperm, kcounts, V_sorted, sumv, lam, H, N, CK, ws, ws_bytes,
-                       v_head_stride, v_row_stride, (hipStream_t)stream);
+                       v_head_stride, v_row_stride, T2tCentroidOut{}, (hipStream_t)stream);
+}
+
+int t2t_vstats_gather_out(const void* V, int v_dtype, long long svh, long long svn,
+                          const int32_t* kperm, const int32_t* kcounts, void* V_sorted, void* sumv,
+                          float* lam, int H, int N, int CK, void* ws, size_t ws_bytes,
+                          const T2tCentroidOut& co, void* stream) {
+  T2T_REQUIRE(kperm, "vstats_gather: null kperm");
+  return vstats_common(V, v_dtype, kperm, kcounts, V_sorted, sumv, lam, H, N, CK, ws, ws_bytes, svh, svn,
+                       co, (hipStream_t)stream);
 }
 
 extern "C" int t2t_kmm_run_vstats(const void* V_sorted, int v_dtype, const int32_t* kcounts,
                                   void* sumv, float* lam, int H, int N, int CK, void* ws,
                                   size_t ws_bytes, void* stream) {
   return vstats_common(V_sorted, v_dtype, nullptr, kcounts, nullptr, sumv, lam, H, N, CK, ws,
-                       ws_bytes, (long long)N * 128, 128, (hipStream_t)stream);
+                       ws_bytes, (long long)N * 128, 128, T2tCentroidOut{}, (hipStream_t)stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -1322,11 +1357,13 @@ extern "C" int t2t_fused_update_vstats(const void* x, const int32_t* labels, con
   else if (v_dtype == T2T_BF16)
     hipLaunchKernelGGL((key_gather_kernel<BF16T, true>), g, dim3(256), 0, st, (const uint16_t*)x,
                        (const uint16_t*)v, w.perm, counts, w.cbase, (const uint16_t*)old, cent,
-                       (uint16_t*)nullptr, vmean, (float*)nullptr, N, C, vs, 128ll);
+                       (uint16_t*)nullptr, vmean, (float*)nullptr, N, C, vs, 128ll,
+                       (uint16_t*)nullptr, (uint16_t*)nullptr, 0.f);
   else
     hipLaunchKernelGGL((key_gather_kernel<F16T, true>), g, dim3(256), 0, st, (const uint16_t*)x,
                        (const uint16_t*)v, w.perm, counts, w.cbase, (const uint16_t*)old, cent,
-                       (uint16_t*)nullptr, vmean, (float*)nullptr, N, C, vs, 128ll);
+                       (uint16_t*)nullptr, vmean, (float*)nullptr, N, C, vs, 128ll,
+                       (uint16_t*)nullptr, (uint16_t*)nullptr, 0.f);
   T2T_LAUNCH_CHECK("fused_update_vstats");
   return T2T_OK;
 }

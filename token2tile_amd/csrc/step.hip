@@ -17,22 +17,35 @@ extern "C" int t2t_step(const t2t_step_args* a, unsigned stages, void* stream) {
               a ? a->struct_bytes : (size_t)0, sizeof(t2t_step_args));
   const int H = a->H, N = a->N, CQ = a->CQ, CK = a->CK, dt = a->dtype;
   const long long hs = (long long)N * 128;
-  if (stages & T2T_STEP_PROJECT_Q)
+  // Stages asked for together share kernels where their results allow: both
+  // projections one launch; the finalised centroids come from the key sums
+  // and the tile image from the value statistics (2 x 4096 tokens: three
+  // launches of 3-5 us less)
+  const unsigned pair = T2T_STEP_PROJECT_Q | T2T_STEP_PROJECT_K;
+  const bool fin = (stages & T2T_STEP_KMEANS) && (stages & T2T_STEP_FINALIZE) && a->ck16 && a->cks;
+  const bool tiles = (stages & T2T_STEP_TILES) && (fin || (stages & T2T_STEP_VSTATS)) && CK == 2048 &&
+                     a->cks && a->tiles;
+  if ((stages & pair) == pair)
+    ST_CHECK(t2t_project_pair(a->q, a->q_head_stride, a->q_row_stride, a->Uq, a->QU, a->k,
+                              a->k_head_stride, a->k_row_stride, a->Uk, a->KU, dt, H, N, stream));
+  else if (stages & T2T_STEP_PROJECT_Q)
     ST_CHECK(t2t_project_strided(a->q, dt, a->Uq, a->QU, H, N, 128, 32, a->q_head_stride,
                                  a->q_row_stride, stream));
-  if (stages & T2T_STEP_PROJECT_K)
+  else if (stages & T2T_STEP_PROJECT_K)
     ST_CHECK(t2t_project_strided(a->k, dt, a->Uk, a->KU, H, N, 128, 32, a->k_head_stride,
                                  a->k_row_stride, stream));
+  const T2tCentroidOut co{fin ? a->ck16 : nullptr, fin || tiles ? a->cks : nullptr, a->scale,
+                          tiles ? a->tiles : nullptr};
   if (stages & T2T_STEP_KMEANS)
-    ST_CHECK(t2t_kmm_run_strided(a->QU, a->KU, a->v, dt, a->v_head_stride, a->v_row_stride, a->cq0,
-                                 a->ck0, a->qlab, a->cq2, a->klab, a->ck2, a->qcounts, a->qperm,
-                                 a->kcounts, a->kperm, a->vp, a->sumv, a->lam, H, N, CQ, CK,
-                                 a->pin_tail, a->ws_kmm, a->ws_kmm_bytes, stream));
+    ST_CHECK(t2t_kmm_run_out(a->QU, a->KU, a->v, dt, a->v_head_stride, a->v_row_stride, a->cq0, a->ck0,
+                             a->qlab, a->cq2, a->klab, a->ck2, a->qcounts, a->qperm, a->kcounts,
+                             a->kperm, a->vp, a->sumv, a->lam, H, N, CQ, CK, a->pin_tail, a->ws_kmm,
+                             a->ws_kmm_bytes, co, stream));
   if (stages & T2T_STEP_VSTATS)
-    ST_CHECK(t2t_kmm_run_vstats_gather_strided(a->v, dt, a->v_head_stride, a->v_row_stride, a->kperm,
-                                               a->kcounts, a->vp, a->sumv, a->lam, H, N, CK, a->ws_vst,
-                                               a->ws_vst_bytes, stream));
-  if (stages & T2T_STEP_FINALIZE)
+    ST_CHECK(t2t_vstats_gather_out(a->v, dt, a->v_head_stride, a->v_row_stride, a->kperm, a->kcounts,
+                                   a->vp, a->sumv, a->lam, H, N, CK, a->ws_vst, a->ws_vst_bytes, co,
+                                   stream));
+  if ((stages & T2T_STEP_FINALIZE) && !fin)
     ST_CHECK(t2t_centroid_finalize(a->ck2, a->ck16, a->cks, a->scale, H, CK, 32, stream));
   if (stages & T2T_STEP_SELECT) {
     ST_CHECK(t2t_score_select_packed(a->QU, a->cks, a->kcounts, a->qperm, a->qcounts, a->ns, a->unip,
@@ -53,7 +66,7 @@ extern "C" int t2t_step(const t2t_step_args* a, unsigned stages, void* stream) {
         a->vp ? 128 : a->v_row_stride, a->kperm, a->kp ? 0 : (a->vp ? 1 : 2), dt, a->kcounts, a->unip,
         a->qlab, a->qperm, a->plan, a->out, a->out_head_stride, a->out_row_stride, a->lse, H, N, CQ,
         a->ws_split, a->ws_split_bytes, stream));
-  if (stages & T2T_STEP_TILES) ST_CHECK(t2t_centroid_tiles(a->cks, a->sumv, a->tiles, H, stream));
+  if ((stages & T2T_STEP_TILES) && !tiles) ST_CHECK(t2t_centroid_tiles(a->cks, a->sumv, a->tiles, H, stream));
   if (stages & T2T_STEP_RESIDUAL)
     ST_CHECK(t2t_resid_merge_inplace_strided(a->out, a->out_head_stride, a->out_row_stride, a->lse, a->QU,
                                              a->tiles, a->kcounts, a->unip, a->qlab, a->qperm, a->lam,

@@ -202,6 +202,32 @@ int t2t_check_launch(const char* what);
 static inline size_t t2t_align256(size_t x) { return (x + 255) & ~(size_t)255; }
 static inline int cdiv(long long a, long long b) { return (int)((a + b - 1) / b); }
 
+// ---- forms of the entry points that one call's stages share (step.hip) ----
+// both projections in one launch (D = 128, r = 32)
+int t2t_project_pair(const void* q, long long sqh, long long sqn, const void* Uq, void* QU,
+                     const void* k, long long skh, long long skn, const void* Uk, void* KU, int dtype,
+                     int H, int N, void* stream);
+// outputs that the k-means or value-statistics kernels can write themselves:
+// the finalised centroids (t2t_centroid_finalize) and the centroid tile image
+// (t2t_centroid_tiles, from cks; 2048 clusters)
+struct T2tCentroidOut {
+  void* ck16;
+  void* cks;
+  float scale;
+  void* tiles;
+};
+int t2t_kmm_run_out(const void* QU, const void* KU, const void* V, int v_dtype, long long svh,
+                    long long svn, const void* cq0, const void* ck0, int32_t* qlab, void* cq2,
+                    int32_t* klab, float* ck2, int32_t* qcounts, int32_t* qperm, int32_t* kcounts,
+                    int32_t* kperm, void* V_sorted, void* sumv, float* lam, int H, int N, int CQ, int CK,
+                    int pin_tail, void* ws, size_t ws_bytes, const T2tCentroidOut& co, void* stream);
+int t2t_vstats_gather_out(const void* V, int v_dtype, long long svh, long long svn,
+                          const int32_t* kperm, const int32_t* kcounts, void* V_sorted, void* sumv,
+                          float* lam, int H, int N, int CK, void* ws, size_t ws_bytes,
+                          const T2tCentroidOut& co, void* stream);
+void t2t_launch_vstats_tiles(const float* vsum, const float* cmax, const void* cks, void* sumv,
+                             float* lam, void* tiles, int H, hipStream_t st);
+
 // Carves aligned sub-buffers out of a caller-owned workspace (base may be
 // NULL to measure the size).
 struct WsCarver {

@@ -1070,6 +1070,69 @@ __global__ __launch_bounds__(256) void centroid_tiles_kernel(const uint16_t* __r
   }
 }
 
+// vstats_kernel and centroid_tiles_kernel in one: lam = max(1, max|vsum| / 32768),
+// sumv = fp16(vsum (1 / lam)) and the tile image of cks and sumv.  Each
+// work-group (64 centroids) reduces the head's 2048 per-cluster maxima itself.
+__global__ __launch_bounds__(256) void vstats_tiles_kernel(const float* __restrict__ vsum,
+                                                           const float* __restrict__ cmax,
+                                                           const uint16_t* __restrict__ cks,
+                                                           uint16_t* __restrict__ sumv,
+                                                           float* __restrict__ lam,
+                                                           uint16_t* __restrict__ tiles) {
+  __shared__ float red[4];
+  const int tc = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+  // thread: 4 centroids (kq) x 8 dims (dseg)
+  const int kq = tid >> 4, dseg = tid & 15;
+  const float* vh = vsum + ((size_t)h * TA_CK + tc * TL_CT) * TA_D;
+  f32x4 x[4][2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      x[i][j] = *(const f32x4*)(vh + (size_t)(4 * kq + i) * TA_D + 8 * dseg + 4 * j);
+  float mx = 0.f;
+#pragma unroll
+  for (int i = 0; i < TA_CK / 256; ++i) mx = fmaxf(mx, cmax[(size_t)h * TA_CK + tid + 256 * i]);
+  mx = wave_max(mx);
+  if ((tid & 63) == 0) red[tid >> 6] = mx;
+  __syncthreads();
+  mx = fmaxf(fmaxf(fmaxf(fmaxf(0.f, red[0]), red[1]), red[2]), red[3]);
+  const float lm = fmaxf(1.0f, mx / 32768.0f);
+  const float inv = 1.0f / lm;
+  if (tc == 0 && tid == 0) lam[h] = lm;
+  uint16_t* dst = tiles + ((size_t)h * RT_TILES + tc) * RT_HALVES;
+  {
+    const uint16_t* ch = cks + ((size_t)h * TA_CK + tc * TL_CT) * 32;
+    const int r = tid >> 2, c = tid & 3;
+    *(u32x4*)(dst + rc_off(r, c)) = *(const u32x4*)(ch + r * 32 + 8 * c);
+  }
+  uint16_t* sh = sumv + ((size_t)h * TA_CK + tc * TL_CT) * TA_D;
+  u32x4 v[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const f32x4& a = x[i][w >> 1];
+      v[i][w] = (uint32_t)f2h(opaque(a[2 * (w & 1)] * inv)) |
+                ((uint32_t)f2h(opaque(a[2 * (w & 1) + 1] * inv)) << 16);
+    }
+    *(u32x4*)(sh + (size_t)(4 * kq + i) * TA_D + 8 * dseg) = v[i];
+  }
+  uint16_t* vt = dst + 2048;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const u32x2 lo = {pack_lo(v[0][w], v[1][w]), pack_lo(v[2][w], v[3][w])};
+    const u32x2 hi = {pack_hi(v[0][w], v[1][w]), pack_hi(v[2][w], v[3][w])};
+    *(u32x2*)(vt + vt_gran_off(8 * dseg + 2 * w, kq)) = lo;
+    *(u32x2*)(vt + vt_gran_off(8 * dseg + 2 * w + 1, kq)) = hi;
+  }
+}
+void t2t_launch_vstats_tiles(const float* vsum, const float* cmax, const void* cks, void* sumv,
+                             float* lam, void* tiles, int H, hipStream_t st) {
+  hipLaunchKernelGGL(vstats_tiles_kernel, dim3(RT_TILES, H), dim3(256), 0, st, vsum, cmax,
+                     (const uint16_t*)cks, (uint16_t*)sumv, lam, (uint16_t*)tiles);
+}
+
 // One work-group per 128 consecutive sorted queries (4 waves x 32, queries of
 // several query clusters side by side): every lane masks the centroids of
 // its own cluster's union, so all waves carry real rows.  The exact part is

@@ -474,13 +474,13 @@ class MaskedStepDeploy:
             a.Uq = st["Uq"].data_ptr()
             # reuse: project with the snapshot's Uq, group K and V through the
             # stored kperm, fresh value statistics from this call's V.  Only
-            # the residual reads QU, sumv and lam: with the fused gathers the
-            # projection and the value statistics run on the side stream,
-            # under the exact attention.
+            # the residual reads QU, lam and the tile image of cks and sumv: with
+            # the fused gathers the projection and the value statistics run on
+            # the side stream, under the exact attention.
             after(s1, 1, s0)
             side = (("", _lib.STEP_PROJECT_Q),)
             if self._fused_kv:
-                side += (("", _lib.STEP_VSTATS),)
+                side += (("", _lib.STEP_VSTATS | _lib.STEP_TILES),)
             self._launch(a, side, s1)
             joined = torch.cuda.Event() if capturing else self._ev[2]
             joined.record(s1)
@@ -491,6 +491,8 @@ class MaskedStepDeploy:
                 main += (("vstats", _lib.STEP_VSTATS),)
             self._launch(a, main + (("attention_exact", _lib.STEP_EXACT),), s0)
             s0.wait_event(joined)
+            tail = () if self._fused_kv else (("attention_prep", _lib.STEP_TILES),)
+            self._launch(a, tail + (("attention_residual", _lib.STEP_RESIDUAL),), s0)
         else:
             for name in ("Uq", "Uk", "ck", "cq"):
                 if not state[name].is_contiguous():
@@ -521,7 +523,9 @@ class MaskedStepDeploy:
                 self._launch(a, (("project", _lib.STEP_PROJECT_Q | _lib.STEP_PROJECT_K),
                                  ("kmeans", _lib.STEP_KMEANS), ("score", _lib.STEP_FINALIZE),
                                  ("select", _lib.STEP_SELECT), *gather, ("plan", _lib.STEP_PLAN),
-                                 ("attention_exact", _lib.STEP_EXACT)), s0)
+                                 ("attention_exact", _lib.STEP_EXACT),
+                                 ("attention_prep", _lib.STEP_TILES),
+                                 ("attention_residual", _lib.STEP_RESIDUAL)), s0)
                 state["ck"], state["cq"] = ck16, cq2
                 if self._cfg_on:
                     if recycle:
@@ -529,10 +533,6 @@ class MaskedStepDeploy:
                     else:  # qlab, klab and counts are this object's own: copied
                         own = dict(st, **{n: st[n].clone() for n in ("qlab", "klab", "counts")})
                     self._cfg_hold[self._cfg_key] = dict(own, Uq=state["Uq"], step=self._cfg_step)
-        # the centroid tile image (after the side stream's value statistics on
-        # reuse calls), residual over the other clusters and the merge
-        self._launch(a, (("attention_prep", _lib.STEP_TILES),
-                         ("attention_residual", _lib.STEP_RESIDUAL)), s0)
         if capturing:
             s1.wait_stream(s0)
             caller.wait_stream(s1)
