@@ -510,6 +510,7 @@ __global__ __launch_bounds__(SEL_WAVES * 64) void select_main_kernel(
 #define SF_ROWS 32
 #define SF_BATCHES 16    // most batches a work-group takes (sf_batches)
 #define SF_CUS 256       // compute units: one work-group each
+#define SF_SPREAD 0.3    // how much longer the slowest work-group of one round takes
 #define SF_START 0.8     // a work-group's start (sizes, first rows by radix passes), in batches
 #define SF_PITCH SEL_NC  // halves per LDS key row (chunks swizzled by row, no padding)
 #define SF_TILES 6       // most 32-centroid score tiles a wave holds (64 tiles over 12 waves)
@@ -735,11 +736,14 @@ static int select_common(const void* gl, const int32_t* kcounts, const int32_t* 
 // Batches per work-group.  One work-group fills a CU, so a launch runs in
 // rounds of SF_CUS work-groups of batches + SF_START batch times each (the
 // start: cluster sizes, and each wave's first row by the radix passes, having
-// no previous crossing); the fewest batch times win.  Fixed at 16 batches, a
+// no previous crossing); the slowest work-group of a lone round takes about a
+// third longer than the mean, which averages out over rounds (SF_SPREAD); the
+// fewest batch times win.  Fixed at 16 batches, a
 // call of few rows left most CUs idle (2 heads x 4096 rows: 16 work-groups,
 // 223 us against 30 at one batch) and one of slightly over a whole number of
 // rounds ran the last one nearly empty (5 x 32760: 402 us against 289 at 7
-// batches; 7 x 98304: 940 against 872 at 12).  Past eight rounds work-groups
+// batches, 293 at 4; 7 x 98304: 940 against 872 at 12; 3 x 20011: 206, 125 at
+// the one round of 8 and 112 at 4).  Past eight rounds work-groups
 // drift apart and the last round fills up by itself: 16 (40 x 75600: 3930 us
 // against 3970 at the model's 15).
 static int sf_batches(int H, int N) {
@@ -748,7 +752,8 @@ static int sf_batches(int H, int N) {
   double bc = 1e30;
   for (int nb = SF_BATCHES; nb >= 1; --nb) {
     const long long wgs = (long long)H * cdiv(N, SF_ROWS * nb);
-    const double cost = (double)((wgs + SF_CUS - 1) / SF_CUS) * (nb + SF_START);
+    const double rounds = (double)((wgs + SF_CUS - 1) / SF_CUS);
+    const double cost = rounds * (nb + SF_START) * (1.0 + SF_SPREAD / rounds);
     if (cost < bc) {
       bc = cost;
       best = nb;
