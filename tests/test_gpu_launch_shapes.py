@@ -140,10 +140,11 @@ def test_projection_fit_forms(dev, D):
     assert torch.equal(Uq, Eq.float()) and torch.equal(Uk, Ek.float())
 
 
-# row blocks per wave 4, 2 and 1 (rows in whole, partial and single chunks), the
-# key pass sharing the first query pass's launches with more and fewer clusters
+# row blocks per wave 4, 2 and 1 (rows in whole, partial and single chunks; a head
+# alone and the last shape with two centroid groups), the key pass sharing the first query pass's launches with more and fewer clusters
 @pytest.mark.parametrize("H,N,CQ,CK,pin", [(8, 131100, 200, 2048, 0), (16, 16450, 33, 500, 77),
-                                           (3, 4097, 4096, 64, 0), (2, 255, 7, 31, 255)])
+                                           (3, 4097, 4096, 64, 0), (40, 1030, 65, 600, 0),
+                                           (2, 255, 7, 31, 255)])
 def test_kmeans_of_many_heads_equals_each_head_alone(dev, H, N, CQ, CK, pin):
     """A head's clustering does not depend on how many heads share the launch,
     so the launch shapes that follow H N agree bit for bit with the smallest;

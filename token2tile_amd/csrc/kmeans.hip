@@ -326,9 +326,12 @@ struct AssignArgs {
   int32_t* chist;          // [H, chunks, C]
   int C, pin_begin, pin_label;
 };
-template <int RB>
-__global__ __launch_bounds__(AK_WAVES * 64) void assign_km_kernel(AssignArgs g0, AssignArgs g1,
-                                                                  int N) {
+// CS groups of AK_WAVES waves take the centroid blocks of the same rows in turn
+// (two where the launch leaves CUs idle: 2 x 4096 rows, 64 work-groups, 26 us in
+// one group, 21 in two).
+template <int RB, int CS>
+__global__ __launch_bounds__(AK_WAVES * 64 * CS) void assign_km_kernel(AssignArgs g0, AssignArgs g1,
+                                                                       int N) {
   constexpr int CMAX = AK_CHUNK, AK_RB = RB;
   const AssignArgs& ga = blockIdx.z ? g1 : g0;
   const uint16_t* __restrict__ X = ga.X;
@@ -342,7 +345,8 @@ __global__ __launch_bounds__(AK_WAVES * 64) void assign_km_kernel(AssignArgs g0,
   __shared__ __attribute__((aligned(16))) float sN[CMAX];
   const int h = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) % AK_WAVES;
+  const int cg = CS > 1 ? __builtin_amdgcn_readfirstlane(tid >> 6) / AK_WAVES : 0;
   const int jl = lane & 31, hh = lane >> 5;
   const int Cp = (C + 31) & ~31;
   const uint16_t* xh = X + (size_t)h * N * D;
@@ -396,16 +400,16 @@ __global__ __launch_bounds__(AK_WAVES * 64) void assign_km_kernel(AssignArgs g0,
   for (int c0 = 0; c0 < Cp; c0 += CMAX) {
   const int nc = Cp - c0 < CMAX ? Cp - c0 : CMAX;
   if (c0 > 0) __syncthreads();  // every wave is done with the previous chunk
-  for (int i = tid; i < nc * 4; i += AK_WAVES * 64) {
+  for (int i = tid; i < nc * 4; i += AK_WAVES * 64 * CS) {
     const int r = i >> 2, c = i & 3;
     u32x4 v = {0u, 0u, 0u, 0u};
     if (c0 + r < C) v = cph[(size_t)c0 * 4 + i];
     ((u32x4*)sC)[r * 4 + (c ^ ((r >> 2) & 3))] = v;
   }
-  for (int i = tid; i < nc; i += AK_WAVES * 64)
+  for (int i = tid; i < nc; i += AK_WAVES * 64 * CS)
     sN[i] = c0 + i < C ? cnorm[(size_t)h * C + c0 + i] : __builtin_inff();
   __syncthreads();
-  for (int cb = 0; cb < nc / 32; ++cb) {
+  for (int cb = cg; cb < nc / 32; cb += CS) {
     const int r = cb * 32 + jl;
     const u32x4* crow = (const u32x4*)sC + r * 4;
     const u32x4 a0 = crow[(0 + hh) ^ ((r >> 2) & 3)];
@@ -445,23 +449,50 @@ __global__ __launch_bounds__(AK_WAVES * 64) void assign_km_kernel(AssignArgs g0,
     const float ob = __builtin_bit_cast(float, half_partner(__builtin_bit_cast(uint32_t, best[k])));
     const int oi = (int)half_partner((uint32_t)bidx[k]);
     lab[k] = bidx[k];
-    if (ob < best[k] || (ob == best[k] && oi < bidx[k])) lab[k] = oi;
+    if (ob < best[k] || (ob == best[k] && oi < bidx[k])) {
+      lab[k] = oi;
+      best[k] = ob;
+    }
+  }
+  if constexpr (CS > 1) {
+    // the other group's best of each row, ties to the lower index
+    static_assert(CS == 2 && CMAX * 4 >= AK_WAVES * 32 * AK_RB * 4, "the values fit");
+    int* sI = (int*)sC;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < AK_RB; ++k)
+      if (cg == 1 && hh == 0) {
+        sN[(wave * AK_RB + k) * 32 + jl] = best[k];
+        sI[(wave * AK_RB + k) * 32 + jl] = lab[k];
+      }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < AK_RB; ++k)
+      if (cg == 0) {
+        const float ob = sN[(wave * AK_RB + k) * 32 + jl];
+        const int oi = sI[(wave * AK_RB + k) * 32 + jl];
+        if (ob < best[k] || (ob == best[k] && oi < lab[k])) lab[k] = oi;
+      }
+  }
+  const bool owner = cg == 0 && hh == 0;
+#pragma unroll
+  for (int k = 0; k < AK_RB; ++k) {
     const int row = rbase + 32 * k;
     lab[k] = row >= pin_begin ? pin_label : lab[k];
-    if (row < N && hh == 0) labels[(size_t)h * N + row] = lab[k];
+    if (row < N && owner) labels[(size_t)h * N + row] = lab[k];
   }
   // the chunk's label histogram, in the LDS of the centroids
   static_assert(CMAX * D * 2 >= KM_MAXC * 4, "the histogram fits the centroid chunk");
   int* hist = (int*)sC;
   __syncthreads();
-  for (int i = tid; i < C; i += AK_WAVES * 64) hist[i] = 0;
+  for (int i = tid; i < C; i += AK_WAVES * 64 * CS) hist[i] = 0;
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < AK_RB; ++k)
-    if (rbase + 32 * k < N && hh == 0) atomicAdd(&hist[lab[k]], 1);
+    if (rbase + 32 * k < N && owner) atomicAdd(&hist[lab[k]], 1);
   __syncthreads();
   int32_t* ho = ga.chist + ((size_t)h * gridDim.x + blockIdx.x) * C;
-  for (int i = tid; i < C; i += AK_WAVES * 64) ho[i] = hist[i];
+  for (int i = tid; i < C; i += AK_WAVES * 64 * CS) ho[i] = hist[i];
 }
 
 // ---------------------------------------------------------------------------
@@ -1032,9 +1063,13 @@ static int launch_assign_km(const AssignArgs& a, const AssignArgs& b, int sets, 
                             hipStream_t st) {
   const dim3 g(km_chunks(H, N), H, sets);
   switch (km_rb(H, N)) {
-    case 4: hipLaunchKernelGGL(assign_km_kernel<4>, g, dim3(AK_WAVES * 64), 0, st, a, b, N); break;
-    case 2: hipLaunchKernelGGL(assign_km_kernel<2>, g, dim3(AK_WAVES * 64), 0, st, a, b, N); break;
-    default: hipLaunchKernelGGL(assign_km_kernel<1>, g, dim3(AK_WAVES * 64), 0, st, a, b, N);
+    case 4: hipLaunchKernelGGL((assign_km_kernel<4, 1>), g, dim3(AK_WAVES * 64), 0, st, a, b, N); break;
+    case 2: hipLaunchKernelGGL((assign_km_kernel<2, 1>), g, dim3(AK_WAVES * 64), 0, st, a, b, N); break;
+    default:
+      if ((long long)g.x * H * sets <= 256)
+        hipLaunchKernelGGL((assign_km_kernel<1, 2>), g, dim3(AK_WAVES * 128), 0, st, a, b, N);
+      else
+        hipLaunchKernelGGL((assign_km_kernel<1, 1>), g, dim3(AK_WAVES * 64), 0, st, a, b, N);
   }
   return t2t_check_launch("assign");
 }
