@@ -325,7 +325,8 @@ int t2t_tile_attn_run_planned(const void* q, const void* kp, const void* vp, int
  * VSTATS, a reuse call PROJECT_Q | VSTATS (on any stream the RESIDUAL waits
  * for; TILES may join them) and EXACT | TILES | RESIDUAL.  Each stage is the
  * entry point named, with its argument checks and results; stages of one call
- * share kernels where they can. */
+ * share kernels where they can, and EXACT may leave the rows of split tasks in
+ * parts in ws_split, which RESIDUAL adds. */
 #define T2T_STEP_PROJECT_Q 1u  /* t2t_project_strided: q, Uq -> QU             */
 #define T2T_STEP_PROJECT_K 2u  /* t2t_project_strided: k, Uk -> KU             */
 #define T2T_STEP_KMEANS    4u  /* t2t_kmm_run_strided                          */

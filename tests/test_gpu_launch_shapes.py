@@ -330,3 +330,31 @@ def test_residual_groups(dev, dtype):
     u = 2.0 ** -11
     bound = 4 * u * 1.01 * mean.float() + 2.0 ** (-10 if dtype == torch.float16 else -7) * a.float().abs() + 1e-6
     assert not a.isnan().any() and bool(((a - b).float().abs() <= bound).all())
+
+
+# parts added by the combine (fewer than 256 row blocks) and by the residual
+# (from 256 on, with two wave groups and with one)
+@pytest.mark.parametrize("H,N,CQ", [(1, 4100, 16), (2, 16384, 100), (3, 20011, 201)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_split_call_equals_its_stages(dev, H, N, CQ, dtype):
+    """run_planned, which may leave the parts to the residual, against the split
+    exact attention (always combined) and the residual one by one: same bits."""
+    from token2tile_amd import ops
+    rng = np.random.default_rng(N)
+    qlab, klab, qperm, qcounts, kperm, kcounts = structure(rng, H, N, CQ)
+    density = rng.choice([0.0, 0.01, 0.3, 1.0], (H, CQ, 1))
+    sel = (rng.random((H, CQ, 2048)) < density).astype(np.uint8)
+    unip = np.packbits(sel, axis=2, bitorder="little").view(np.int32)
+    gen = torch.Generator(device=dev).manual_seed(N)
+    r = lambda *s: torch.randn(*s, generator=gen, device=dev)  # noqa: E731
+    q, kp, vp = (r(H, N, 128).to(dtype) for _ in range(3))
+    QU, cks, sumv = r(H, N, 32).half(), (0.1 * r(H, 2048, 32)).half(), r(H, 2048, 128).half()
+    lam, tw = torch.linspace(1, 2, H, device=dev), torch.tensor(1.0, device=dev)
+    tq, tk, tu, tqp, tql = (g(a, dev) for a in (qcounts, kcounts, unip, qperm, qlab))
+    plan = ops.tile_plan(tq, tk, tu, N)
+    a, b = torch.full_like(q, float("nan")), torch.full_like(q, float("nan"))
+    lse = torch.empty(H, N, device=dev)
+    ops.tile_attn_exact_split(q, kp, vp, None, tk, tu, tql, tqp, plan, a, lse, gather=0)
+    ops.resid_merge_inplace(a, lse, QU, ops.centroid_tiles(cks, sumv), tk, tu, tql, tqp, lam, tw)
+    ops.tile_attn_run_planned(q, kp, vp, tq, tk, tu, QU, cks, sumv, lam, tql, tqp, tw, b, plan, False)
+    assert not a.isnan().any() and torch.equal(a, b)

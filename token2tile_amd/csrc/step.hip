@@ -60,7 +60,7 @@ extern "C" int t2t_step(const t2t_step_args* a, unsigned stages, void* stream) {
   if (stages & T2T_STEP_PLAN)
     ST_CHECK(t2t_tile_plan(a->qcounts, a->kcounts, a->unip, a->plan, H, N, CQ, stream));
   if (stages & T2T_STEP_EXACT)
-    ST_CHECK(t2t_tile_attn_exact_split(
+    ST_CHECK(t2t_exact_split_parts(
         a->q, a->q_head_stride, a->q_row_stride, a->kp ? a->kp : a->k, a->kp ? hs : a->k_head_stride,
         a->kp ? 128 : a->k_row_stride, a->vp ? a->vp : a->v, a->vp ? hs : a->v_head_stride,
         a->vp ? 128 : a->v_row_stride, a->kperm, a->kp ? 0 : (a->vp ? 1 : 2), dt, a->kcounts, a->unip,
@@ -68,8 +68,8 @@ extern "C" int t2t_step(const t2t_step_args* a, unsigned stages, void* stream) {
         a->ws_split, a->ws_split_bytes, stream));
   if ((stages & T2T_STEP_TILES) && !tiles) ST_CHECK(t2t_centroid_tiles(a->cks, a->sumv, a->tiles, H, stream));
   if (stages & T2T_STEP_RESIDUAL)
-    ST_CHECK(t2t_resid_merge_inplace_strided(a->out, a->out_head_stride, a->out_row_stride, a->lse, a->QU,
-                                             a->tiles, a->kcounts, a->unip, a->qlab, a->qperm, a->lam,
-                                             a->tailw, dt, H, N, CQ, stream));
+    ST_CHECK(t2t_resid_merge_parts(a->out, a->out_head_stride, a->out_row_stride, a->lse, a->QU,
+                                   a->tiles, a->kcounts, a->unip, a->qlab, a->qperm, a->plan, a->lam,
+                                   a->tailw, dt, H, N, CQ, a->ws_split, a->ws_split_bytes, stream));
   return T2T_OK;
 }

@@ -225,6 +225,20 @@ int t2t_vstats_gather_out(const void* V, int v_dtype, long long svh, long long s
                           const int32_t* kperm, const int32_t* kcounts, void* V_sorted, void* sumv,
                           float* lam, int H, int N, int CK, void* ws, size_t ws_bytes,
                           const T2tCentroidOut& co, void* stream);
+// t2t_tile_attn_exact_split whose split rows may stay in parts in ws, and the
+// residual that then adds them (t2t_resid_merge_inplace_strided otherwise)
+int t2t_exact_split_parts(
+    const void* q, long long q_head_stride, long long q_row_stride, const void* k,
+    long long k_head_stride, long long k_row_stride, const void* v, long long v_head_stride,
+    long long v_row_stride, const int32_t* kperm, int gather, int dtype, const int32_t* kcounts,
+    const int32_t* unip, const int32_t* qlab, const int32_t* qperm, const int32_t* plan, void* out,
+    long long out_head_stride, long long out_row_stride, float* lse, int H, int N, int CQ, void* ws,
+    size_t ws_bytes, void* stream);
+int t2t_resid_merge_parts(void* out, long long soh, long long son, const float* lse, const void* QU,
+                          const void* tiles, const int32_t* kcounts, const int32_t* unip,
+                          const int32_t* qlab, const int32_t* qperm, const int32_t* plan,
+                          const float* lam, const float* tailw_dev, int dtype, int H, int N, int CQ,
+                          void* ws, size_t ws_bytes, void* stream);
 void t2t_launch_vstats_tiles(const float* vsum, const float* cmax, const void* cks, void* sumv,
                              float* lam, void* tiles, int H, hipStream_t st);
 

@@ -307,6 +307,12 @@ __host__ __device__ inline int split_parts(int kvlen, int S) {
   const int n = (kvlen + TA_KT - 1) / TA_KT / TA_SPLIT_TILES;
   return n < 1 ? 1 : (n < S ? n : S);
 }
+// Whether the residual adds the parts of a split call (else combine_kernel): a
+// lane of it reads its whole row's parts, which pays from one work-group per CU
+// on (2 x 16384: 214 us a reuse call with the combine, 208 without; 3 x 20011
+// 514, 505); 64 work-groups take longer over it than a launch (2 x 4096: 232,
+// 251).
+static bool split_in_resid(int H, int N) { return (long long)H * cdiv(N, 128) >= 256; }
 // Most parts per task (1: the call is not split): about two work-groups per
 // slot, counting a task per 128 queries and half a task more per query cluster.
 // us unsplit / at 1, 2, 3, 4 work-groups per slot: 2 x 4096 92 / 53, 51, 50,
@@ -957,6 +963,44 @@ static void launch_attn(const void* q, const void* kp, const void* vp, const int
                      skh, skn, soh, son, svh, svn, 1, (float*)nullptr, (float*)nullptr);
 }
 
+// A sorted row's parts: the weight of each (0 past P), the log2-sum of the row.
+// opart and mlpart rows sit H N apart.
+struct PartSum {
+  float a[TA_SPLIT_MAX];  // exp2(m_i - M) / sum
+  float lse2;
+  __device__ void load(const float* mlpart, size_t row, size_t HN, int P) {
+    float l[TA_SPLIT_MAX];
+    float M = -__builtin_inff(), lt = 0.f;
+#pragma unroll
+    for (int i = 0; i < TA_SPLIT_MAX; ++i) {
+      a[i] = i < P ? mlpart[2 * (row + i * HN)] : -__builtin_inff();
+      l[i] = i < P ? mlpart[2 * (row + i * HN) + 1] : 0.f;
+      if (i < P) M = vmax(M, a[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < TA_SPLIT_MAX; ++i) {
+      a[i] = i < P ? __builtin_amdgcn_exp2f(a[i] - M) : 0.f;
+      lt = i < P ? fmaf(a[i], l[i], lt) : lt;
+    }
+    const float inv = 1.0f / lt;
+#pragma unroll
+    for (int i = 0; i < TA_SPLIT_MAX; ++i) a[i] *= inv;
+    lse2 = M + __log2f(lt);
+  }
+  // four dims of the row, from column d
+  __device__ f32x4 sum(const float* opart, size_t row, size_t HN, int P, int d) const {
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < TA_SPLIT_MAX; ++i)
+      if (i < P) {
+        const f32x4 v = *(const f32x4*)(opart + (row + i * HN) * TA_D + d);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = fmaf(a[i], v[e], o[e]);
+      }
+    return o;
+  }
+};
+
 // adds the parts of the split tasks: 32 lanes per sorted row, four dims each
 template <typename T>
 __global__ __launch_bounds__(256) void combine_kernel(
@@ -970,32 +1014,13 @@ __global__ __launch_bounds__(256) void combine_kernel(
   const int orig = qperm[(size_t)h * N + j];
   const int P = split_parts(kvlen[(size_t)h * CQ + qlab[(size_t)h * N + orig]], S);
   if (P < 2) return;  // the task wrote its rows itself
-  float mi[TA_SPLIT_MAX], li[TA_SPLIT_MAX];
-  f32x4 oi[TA_SPLIT_MAX];
-  float M = -__builtin_inff();
-#pragma unroll
-  for (int i = 0; i < TA_SPLIT_MAX; ++i)
-    if (i < P) {
-      const size_t pr = (size_t)i * H * N + (size_t)h * N + j;
-      mi[i] = mlpart[2 * pr];
-      li[i] = mlpart[2 * pr + 1];
-      oi[i] = *(const f32x4*)(opart + pr * TA_D + 4 * l);
-      M = vmax(M, mi[i]);
-    }
-  float lt = 0.f;
-  f32x4 o = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int i = 0; i < TA_SPLIT_MAX; ++i)
-    if (i < P) {
-      const float a = __builtin_amdgcn_exp2f(mi[i] - M);
-      lt = fmaf(a, li[i], lt);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) o[e] = fmaf(a, oi[i][e], o[e]);
-    }
-  const float inv = 1.0f / lt;
+  const size_t row = (size_t)h * N + j, HN = (size_t)H * N;
+  PartSum ps;
+  ps.load(mlpart, row, HN, P);
+  const f32x4 o = ps.sum(opart, row, HN, P, 4 * l);
   *(u32x2*)(out + (size_t)h * soh + (size_t)orig * son + 4 * l) =
-      u32x2{Pk<T>::pack(o[0] * inv, o[1] * inv), Pk<T>::pack(o[2] * inv, o[3] * inv)};
-  if (l == 0) lse[(size_t)h * N + j] = M + __log2f(lt);
+      u32x2{Pk<T>::pack(o[0], o[1]), Pk<T>::pack(o[2], o[3])};
+  if (l == 0) lse[row] = ps.lse2;
 }
 
 struct SplitWs {
@@ -1017,13 +1042,14 @@ static void launch_attn_split(const void* q, const void* k, const void* v, const
                               const int32_t* qlab, const int32_t* qperm, const int32_t* kcounts,
                               const PlanView& p, float* lse, void* out, int H, int N, int CQ, int S,
                               const SplitWs& w, const int32_t* kperm, const long long (&sd)[8],
-                              hipStream_t st) {
+                              bool combine, hipStream_t st) {
   const int grid = ((H * p.maxT * S + 63) / 64) * 64;
   hipLaunchKernelGGL((attn_kernel<T, MODE, true>), dim3(grid), dim3(TA_WAVES * 64), 0, st,
                      (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v,
                      (const uint32_t*)unip, qperm, kcounts, p.k_off, p.ntask, p.tasks,
                      (uint16_t*)nullptr, lse, (uint16_t*)out, kperm, H, N, CQ, p.maxT, sd[0], sd[1],
                      sd[2], sd[3], sd[6], sd[7], sd[4], sd[5], S, w.opart, w.mlpart);
+  if (!combine) return;  // the residual adds the parts
   hipLaunchKernelGGL(combine_kernel<T>, dim3(cdiv(N, 8), H), dim3(256), 0, st, w.opart, w.mlpart,
                      p.kvlen, qlab, qperm, (uint16_t*)out, lse, H, N, CQ, S, sd[6], sd[7]);
 }
@@ -1069,6 +1095,13 @@ __global__ __launch_bounds__(256) void centroid_tiles_kernel(const uint16_t* __r
     *(u32x2*)(vt + vt_gran_off(8 * dseg + 2 * w + 1, kq)) = hi;
   }
 }
+
+struct SplitIn {
+  const float* opart;
+  const float* mlpart;
+  const int32_t* kvlen;
+  int S;
+};
 
 // vstats_kernel and centroid_tiles_kernel in one: lam = max(1, max|vsum| / 32768),
 // sumv = fp16(vsum (1 / lam)) and the tile image of cks and sumv.  Each
@@ -1139,20 +1172,23 @@ void t2t_launch_vstats_tiles(const float* vsum, const float* cmax, const void* c
 // read from attn_out (sorted order, SRC_SORTED) or from the original rows of
 // out, and the merged result is written to the original rows of out.
 //
+// SPLIT: rows of split tasks are added from their parts here (as combine_kernel
+// would, rounded to T like the exact part it stores), not read from out.
+//
 // G groups of four waves share the queries, each walking its share of the 32
 // centroid tiles; the first group adds the others' sums through LDS.  G = 2
 // where the work-groups do not outnumber the CUs (launch_resid): a tile's fetch,
 // scores, exponentials and products follow one another, so the launch lasts
 // for the chain of tiles (64 work-groups: 39 us in one chain, 33 in two; 256: 41.5,
 // 40).
-template <typename T, bool SRC_SORTED, int G>
+template <typename T, bool SRC_SORTED, int G, bool SPLIT>
 __global__ __launch_bounds__(256 * G, G == 1 ? 3 : 1) void resid_kernel(
     const uint16_t* __restrict__ exact, const float* __restrict__ lse2v,
     const uint16_t* __restrict__ QU, const uint16_t* __restrict__ tiles,
     const int32_t* __restrict__ kcounts, const uint32_t* __restrict__ unip,
     const int32_t* __restrict__ qlab, const int32_t* __restrict__ qperm,
     const float* __restrict__ lam, const float* __restrict__ tailw, uint16_t* __restrict__ out,
-    int N, int CQ, long long soh, long long son) {
+    int N, int CQ, long long soh, long long son, SplitIn sp) {
   __shared__ __attribute__((aligned(1024))) uint16_t sT0[G * RT_HALVES];
   __shared__ __attribute__((aligned(1024))) uint16_t sT1[G * RT_HALVES];
   // counts as fp16, ordered so that the 16 a lane weights in one 32-centroid
@@ -1381,7 +1417,15 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : 1) void resid_kernel(
   phi = half_sum(phi);
   const float tw = *tailw;
   const float lm = lam[h];
-  const float le = lse2v[(size_t)h * N + row] * 0.6931471805599453f;
+  // SPLIT: the exact part of a split task's row is still in parts
+  const size_t srow = (size_t)h * N + row, HN = (size_t)gridDim.y * N;
+  int P = 1;
+  PartSum ps;
+  if constexpr (SPLIT) {
+    P = split_parts(sp.kvlen[(size_t)h * CQ + qlab[(size_t)h * N + orig]], sp.S);
+    if (P > 1) ps.load(sp.mlpart, srow, HN, P);
+  }
+  const float le = (SPLIT && P > 1 ? ps.lse2 : lse2v[srow]) * 0.6931471805599453f;
   float ex, st;
   if (le >= m2) {
     ex = 1.0f;
@@ -1397,13 +1441,19 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : 1) void resid_kernel(
   // out row n of head h at out + h soh + n son (elements)
   uint16_t* orow = out + (size_t)h * soh + (size_t)orig * son;
   const uint16_t* er = SRC_SORTED ? exact + ((size_t)h * N + row) * TA_D : orow;
-  if (bad && !SRC_SORTED) return;  // the exact part in out is the output
+  if (bad && !SRC_SORTED && P == 1) return;  // the exact part in out is the output
 #pragma unroll
   for (int nb = 0; nb < 4; ++nb)
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const int d0 = 32 * nb + 8 * g + 4 * hh;
-      u32x2 v = *(const u32x2*)(er + d0);
+      u32x2 v;
+      if (SPLIT && P > 1) {
+        const f32x4 o = ps.sum(sp.opart, srow, HN, P, d0);
+        v = u32x2{Pk<T>::pack(o[0], o[1]), Pk<T>::pack(o[2], o[3])};
+      } else {
+        v = *(const u32x2*)(er + d0);
+      }
       if (!bad) {
         const float x0 = T::to_f((uint16_t)(v[0] & 0xffff)), x1 = T::to_f((uint16_t)(v[0] >> 16));
         const float x2 = T::to_f((uint16_t)(v[1] & 0xffff)), x3 = T::to_f((uint16_t)(v[1] >> 16));
@@ -1450,19 +1500,29 @@ static void launch_resid(int dtype, const void* exact, const float* lse, const v
                          const void* tiles, const int32_t* kcounts, const int32_t* unip,
                          const int32_t* qlab, const int32_t* qperm, const float* lam,
                          const float* tailw, void* out, int H, int N, int CQ, hipStream_t st,
-                         long long soh = -1, long long son = TA_D) {
+                         long long soh = -1, long long son = TA_D,
+                         const SplitIn& sp = SplitIn{nullptr, nullptr, nullptr, 1}) {
   const dim3 grid(cdiv(N, 128), H);
   if (soh < 0) soh = (long long)N * TA_D;
-#define RS_LAUNCH(T, G)                                                                            \
-  hipLaunchKernelGGL((resid_kernel<T, SRC_SORTED, G>), grid, dim3(256 * G), 0, st,                 \
+  // (SRC_SORTED rows are never in parts)
+#define RS_LAUNCH(T, G, SP)                                                                        \
+  hipLaunchKernelGGL((resid_kernel<T, SRC_SORTED, G, SP>), grid, dim3(256 * G), 0, st,             \
                      (const uint16_t*)exact, lse, (const uint16_t*)QU, (const uint16_t*)tiles,     \
                      kcounts, (const uint32_t*)unip, qlab, qperm, lam, tailw, (uint16_t*)out, N,   \
-                     CQ, soh, son)
-  if ((long long)grid.x * H <= 256) {
-    if (dtype == T2T_F16) RS_LAUNCH(F16T, 2); else RS_LAUNCH(BF16T, 2);
-  } else {
-    if (dtype == T2T_F16) RS_LAUNCH(F16T, 1); else RS_LAUNCH(BF16T, 1);
+                     CQ, soh, son, sp)
+#define RS_LAUNCH_T(T)                                               \
+  if (sp.S > 1) {                                                    \
+    if (two) RS_LAUNCH(T, 2, !SRC_SORTED); else RS_LAUNCH(T, 1, !SRC_SORTED); \
+  } else {                                                           \
+    if (two) RS_LAUNCH(T, 2, false); else RS_LAUNCH(T, 1, false);    \
   }
+  const bool two = (long long)grid.x * H <= 256;
+  if (dtype == T2T_F16) {
+    RS_LAUNCH_T(F16T)
+  } else {
+    RS_LAUNCH_T(BF16T)
+  }
+#undef RS_LAUNCH_T
 #undef RS_LAUNCH
 }
 
@@ -1555,11 +1615,12 @@ template <typename T>
 static void exact_launch(int mode, const void* q, const void* k, const void* v, const long long (&sd)[8],
                          const int32_t* kperm, const int32_t* kcounts, const int32_t* unip,
                          const int32_t* qlab, const int32_t* qperm, const PlanView& p, void* out,
-                         float* lse, int H, int N, int CQ, int S, const SplitWs& w, hipStream_t st) {
+                         float* lse, int H, int N, int CQ, int S, const SplitWs& w, bool combine,
+                         hipStream_t st) {
 #define EX_LAUNCH(M)                                                                                \
   if (S > 1)                                                                                        \
     launch_attn_split<T, M>(q, k, v, unip, qlab, qperm, kcounts, p, lse, out, H, N, CQ, S, w, kperm, \
-                            sd, st);                                                                \
+                            sd, combine, st);                                                       \
   else                                                                                              \
     launch_attn<T, M>(q, k, v, unip, qperm, kcounts, p, nullptr, lse, out, H, N, CQ, st, kperm,     \
                       sd[0], sd[1], sd[2], sd[3], sd[6], sd[7], sd[4], sd[5])
@@ -1577,7 +1638,8 @@ static void exact_launch(int mode, const void* q, const void* k, const void* v, 
 static int exact_impl(int mode, const void* q, const void* k, const void* v, const long long (&sd)[8],
                       const int32_t* kperm, int dtype, const int32_t* kcounts, const int32_t* unip,
                       const int32_t* qlab, const int32_t* qperm, const int32_t* plan, void* out,
-                      float* lse, int H, int N, int CQ, void* ws, size_t ws_bytes, void* stream) {
+                      float* lse, int H, int N, int CQ, void* ws, size_t ws_bytes, bool combine,
+                      void* stream) {
   T2T_REQUIRE(q && k && v && (kperm || mode < 2) && kcounts && unip && qperm && plan && out && lse,
               "tile_attn_exact_orig_gather_kv: null pointer");
   T2T_REQUIRE(check_dtype(dtype), "tile_attn_exact_orig_gather_kv: dtype %d", dtype);
@@ -1601,10 +1663,10 @@ static int exact_impl(int mode, const void* q, const void* k, const void* v, con
   }
   if (dtype == T2T_F16)
     exact_launch<F16T>(mode, q, k, v, sd, kperm, kcounts, unip, qlab, qperm, p, out, lse, H, N, CQ, S,
-                       w, st);
+                       w, combine, st);
   else
     exact_launch<BF16T>(mode, q, k, v, sd, kperm, kcounts, unip, qlab, qperm, p, out, lse, H, N, CQ, S,
-                        w, st);
+                        w, combine, st);
   T2T_LAUNCH_CHECK("tile_attn_exact_orig_gather_kv");
   return T2T_OK;
 }
@@ -1619,7 +1681,7 @@ extern "C" int t2t_tile_attn_exact_orig_gather_kv_strided(
   const long long sd[8] = {q_head_stride, q_row_stride, k_head_stride, k_row_stride,
                            v_head_stride, v_row_stride, out_head_stride, out_row_stride};
   return exact_impl(3, q, k, v, sd, kperm, dtype, kcounts, unip, nullptr, qperm, plan, out, lse, H, N,
-                    CQ, nullptr, 0, stream);
+                    CQ, nullptr, 0, true, stream);
 }
 
 extern "C" size_t t2t_tile_attn_split_ws_bytes(int H, int N, int CQ) {
@@ -1628,13 +1690,13 @@ extern "C" size_t t2t_tile_attn_split_ws_bytes(int H, int N, int CQ) {
   return S > 1 ? split_layout(H, N, S, nullptr).total : 0;
 }
 
-extern "C" int t2t_tile_attn_exact_split(
+static int exact_split(
     const void* q, long long q_head_stride, long long q_row_stride, const void* k,
     long long k_head_stride, long long k_row_stride, const void* v, long long v_head_stride,
     long long v_row_stride, const int32_t* kperm, int gather, int dtype, const int32_t* kcounts,
     const int32_t* unip, const int32_t* qlab, const int32_t* qperm, const int32_t* plan, void* out,
     long long out_head_stride, long long out_row_stride, float* lse, int H, int N, int CQ, void* ws,
-    size_t ws_bytes, void* stream) {
+    size_t ws_bytes, bool combine, void* stream) {
   T2T_REQUIRE(qlab, "tile_attn_exact_split: null qlab");
   T2T_REQUIRE(gather >= 0 && gather <= 2, "tile_attn_exact_split: gather=%d not in [0, 2]", gather);
   // cluster-ordered rows are read from contiguous [H, N, 128] buffers
@@ -1646,7 +1708,31 @@ extern "C" int t2t_tile_attn_exact_split(
   const long long sd[8] = {q_head_stride, q_row_stride, k_head_stride, k_row_stride,
                            v_head_stride, v_row_stride, out_head_stride, out_row_stride};
   return exact_impl(1 + gather, q, k, v, sd, kperm, dtype, kcounts, unip, qlab, qperm, plan, out, lse,
-                    H, N, CQ, ws, ws_bytes, stream);
+                    H, N, CQ, ws, ws_bytes, combine, stream);
+}
+
+extern "C" int t2t_tile_attn_exact_split(
+    const void* q, long long q_head_stride, long long q_row_stride, const void* k,
+    long long k_head_stride, long long k_row_stride, const void* v, long long v_head_stride,
+    long long v_row_stride, const int32_t* kperm, int gather, int dtype, const int32_t* kcounts,
+    const int32_t* unip, const int32_t* qlab, const int32_t* qperm, const int32_t* plan, void* out,
+    long long out_head_stride, long long out_row_stride, float* lse, int H, int N, int CQ, void* ws,
+    size_t ws_bytes, void* stream) {
+  return exact_split(q, q_head_stride, q_row_stride, k, k_head_stride, k_row_stride, v, v_head_stride, v_row_stride,
+                     kperm, gather, dtype, kcounts, unip, qlab, qperm, plan, out, out_head_stride,
+                     out_row_stride, lse, H, N, CQ, ws, ws_bytes, true, stream);
+}
+
+int t2t_exact_split_parts(
+    const void* q, long long q_head_stride, long long q_row_stride, const void* k,
+    long long k_head_stride, long long k_row_stride, const void* v, long long v_head_stride,
+    long long v_row_stride, const int32_t* kperm, int gather, int dtype, const int32_t* kcounts,
+    const int32_t* unip, const int32_t* qlab, const int32_t* qperm, const int32_t* plan, void* out,
+    long long out_head_stride, long long out_row_stride, float* lse, int H, int N, int CQ, void* ws,
+    size_t ws_bytes, void* stream) {
+  return exact_split(q, q_head_stride, q_row_stride, k, k_head_stride, k_row_stride, v, v_head_stride, v_row_stride,
+                     kperm, gather, dtype, kcounts, unip, qlab, qperm, plan, out, out_head_stride,
+                     out_row_stride, lse, H, N, CQ, ws, ws_bytes, !split_in_resid(H, N), stream);
 }
 
 extern "C" int t2t_tile_attn_exact_orig(const void* q, const void* kp, const void* vp, int dtype,
@@ -1672,7 +1758,8 @@ static int resid_inplace_impl(void* out, long long soh, long long son, const flo
                               const void* QU, const void* tiles, const int32_t* kcounts,
                               const int32_t* unip, const int32_t* qlab, const int32_t* qperm,
                               const float* lam, const float* tailw_dev, int dtype, int H, int N,
-                              int CQ, void* stream) {
+                              int CQ, void* stream,
+                              const SplitIn& sp = SplitIn{nullptr, nullptr, nullptr, 1}) {
   T2T_REQUIRE(out && lse && QU && tiles && kcounts && unip && qlab && qperm && lam && tailw_dev,
               "resid_merge_inplace: null pointer");
   T2T_REQUIRE(check_dtype(dtype), "resid_merge_inplace: dtype %d", dtype);
@@ -1680,9 +1767,26 @@ static int resid_inplace_impl(void* out, long long soh, long long son, const flo
   T2T_REQUIRE(son >= TA_D && son % 8 == 0 && soh >= 0 && soh % 8 == 0,
               "resid_merge_inplace: out strides (%lld, %lld)", soh, son);
   launch_resid<false>(dtype, nullptr, lse, QU, tiles, kcounts, unip, qlab, qperm, lam, tailw_dev,
-                      out, H, N, CQ, (hipStream_t)stream, soh, son);
+                      out, H, N, CQ, (hipStream_t)stream, soh, son, sp);
   T2T_LAUNCH_CHECK("resid_merge_inplace");
   return T2T_OK;
+}
+
+int t2t_resid_merge_parts(void* out, long long soh, long long son, const float* lse, const void* QU,
+                          const void* tiles, const int32_t* kcounts, const int32_t* unip,
+                          const int32_t* qlab, const int32_t* qperm, const int32_t* plan,
+                          const float* lam, const float* tailw_dev, int dtype, int H, int N, int CQ,
+                          void* ws, size_t ws_bytes, void* stream) {
+  T2T_REQUIRE(H > 0 && N > 0 && CQ > 0 && plan, "resid_merge_parts: H=%d N=%d CQ=%d", H, N, CQ);
+  const int S = split_max(H, N, CQ);
+  const SplitWs w = split_layout(H, N, S, ws);
+  if (S > 1 && (!ws || ws_bytes < w.total)) {
+    t2t_set_error("resid_merge_parts: workspace %zu < %zu bytes", ws_bytes, w.total);
+    return T2T_ERR_WORKSPACE;
+  }
+  const PlanView p = plan_view((int32_t*)plan, H, N, CQ);
+  return resid_inplace_impl(out, soh, son, lse, QU, tiles, kcounts, unip, qlab, qperm, lam, tailw_dev,
+                            dtype, H, N, CQ, stream, SplitIn{w.opart, w.mlpart, p.kvlen, split_in_resid(H, N) ? S : 1});
 }
 
 extern "C" int t2t_resid_merge_inplace(void* out, const float* lse, const void* QU,
@@ -1746,14 +1850,15 @@ extern "C" int t2t_tile_attn_run_planned(const void* q, const void* kp, const vo
   const long long sd[8] = {hs, TA_D, hs, TA_D, hs, TA_D, hs, TA_D};
   const int S = split_max(H, N, CQ);
   const SplitWs sw = split_layout(H, N, S, (char*)ws + w.off);
+  const bool late = split_in_resid(H, N);
   if (dtype == T2T_F16)
     exact_launch<F16T>(1, q, kp, vp, sd, nullptr, kcounts, unip, qlab, qperm, p, out, lse, H, N, CQ, S,
-                       sw, st);
+                       sw, !late, st);
   else
     exact_launch<BF16T>(1, q, kp, vp, sd, nullptr, kcounts, unip, qlab, qperm, p, out, lse, H, N, CQ, S,
-                        sw, st);
+                        sw, !late, st);
   launch_resid<false>(dtype, nullptr, lse, QU, tiles, kcounts, unip, qlab, qperm, lam, tailw_dev,
-                      out, H, N, CQ, st);
+                      out, H, N, CQ, st, -1, TA_D, SplitIn{sw.opart, sw.mlpart, p.kvlen, late ? S : 1});
   T2T_LAUNCH_CHECK("tile_attn_run_planned");
   return T2T_OK;
 }
