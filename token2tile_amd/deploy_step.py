@@ -275,10 +275,13 @@ class MaskedStepDeploy:
         self.s_main = torch.cuda.Stream(device=dev)
         self.s_side = torch.cuda.Stream(device=dev)
         self._lock = threading.Lock()
-        # caller, fork, join, done (recorded once: torch creates the event then)
+        # caller, fork, join, done.  Used once here: an event and a stream's queue
+        # are made at their first use (200 us on the first reuse call otherwise)
         self._ev = [torch.cuda.Event() for _ in range(4)]
         for ev in self._ev:
             ev.record(self.s_main)
+        self.s_side.wait_event(self._ev[1])
+        self._ev[2].record(self.s_side)
         self.last_call_full = None
         # optional list: (stage name, start event, end event) per launch group
         # recorded on s_main, for the benchmark's per-kernel timing
