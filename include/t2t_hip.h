@@ -390,6 +390,12 @@ int t2t_fused_update_vstats(const void* x, const int32_t* labels, const void* ol
                             const void* v, int v_dtype, float* cent, int32_t* counts,
                             float* vmean, int H, int N, int C, int D, void* ws,
                             size_t ws_bytes, void* stream);
+/* t2t_fused_update_vstats with its fp32 means rounded to 16 bits: cent16 fp16,
+ * vmean16 in v_dtype.  (Rows whose label is not in [0, C) are in no cluster;
+ * the counts then sum to less than N.) */
+int t2t_fused_update_vstats16(const void* x, const int32_t* labels, const void* old, const void* v,
+                              int v_dtype, void* cent16, int32_t* counts, void* vmean16, int H, int N,
+                              int C, int D, void* ws, size_t ws_bytes, void* stream);
 /* Warm Lloyd iterations in place on cen [H, C, D] fp16: `iters` times
  * t2t_fast_assign and the fp32 means of t2t_fused_update_vstats (without v)
  * rounded to fp16; empty clusters keep theirs.  D == 32; ws >=

@@ -358,3 +358,27 @@ def test_split_call_equals_its_stages(dev, H, N, CQ, dtype):
     ops.resid_merge_inplace(a, lse, QU, ops.centroid_tiles(cks, sumv), tk, tu, tql, tqp, lam, tw)
     ops.tile_attn_run_planned(q, kp, vp, tq, tk, tu, QU, cks, sumv, lam, tql, tqp, tw, b, plan, False)
     assert not a.isnan().any() and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("H,N,C", [(2, 1000, 33), (1, 300, 2048)])
+def test_update_leaves_foreign_labels_out(dev, H, N, C):
+    """Rows labelled outside [0, C) belong to no cluster (the checked call raises
+    from the counts' sum): means and counts are those of the other rows."""
+    from token2tile_amd import ops
+    gen = torch.Generator(device=dev).manual_seed(N)
+    x = torch.randn(H, N, 32, generator=gen, device=dev).half()
+    v = torch.randn(H, N, 128, generator=gen, device=dev).bfloat16()
+    old = torch.randn(H, C, 32, generator=gen, device=dev).half()
+    lab = torch.randint(0, C, (H, N), generator=gen, device=dev, dtype=torch.int32)
+    bad = lab.clone()
+    bad[:, 5::7], bad[:, 6::70], bad[:, 8::90] = -1, C, 2 ** 31 - 1
+    for h in range(H):
+        ok = ((bad[h] >= 0) & (bad[h] < C)).nonzero().flatten()
+        args = (x[h:h + 1], bad[h:h + 1], old[h:h + 1], v[h:h + 1])
+        part = (x[h:h + 1, ok], bad[h:h + 1, ok], old[h:h + 1], v[h:h + 1, ok])
+        for half in (False, True):
+            got = ops.fused_update_vstats(*args, check_labels=False, half=half)
+            want = ops.fused_update_vstats(*(t.contiguous() for t in part), half=half)
+            assert all(torch.equal(a, b) for a, b in zip(got, want))
+        with pytest.raises(ValueError, match="labels"):
+            ops.fused_update_vstats(*args)

@@ -113,6 +113,8 @@ SIGNATURES = {
                                         c_size_t, _P]),
     "t2t_fused_update_vstats": (c_int, [_P, _P, _P, _P, c_int, _P, _P, _P, c_int, c_int, c_int,
                                         c_int, _P, c_size_t, _P]),
+    "t2t_fused_update_vstats16": (c_int, [_P, _P, _P, _P, c_int, _P, _P, _P, c_int, c_int, c_int,
+                                          c_int, _P, c_size_t, _P]),
     "t2t_lloyd_ws_bytes": (c_size_t, [c_int, c_int, c_int]),
     "t2t_lloyd": (c_int, [_P, _P, c_int, c_int, c_int, c_int, c_int, _P, c_size_t, _P]),
     "t2t_gram_ws_bytes": (c_size_t, [c_int, c_int, c_int]),

@@ -1,13 +1,13 @@
 // S2: warm-started k-means maintenance, and the init_state helpers
-// (fast_assign, deterministic centroid update), for gfx950.
+// (fast_assign, Lloyd iterations, centroid updates), for gfx950.
 //
 // Pipeline of one maintenance call (all deterministic):
-//   prep centroids -> assign (MFMA distances + argmin) -> stable counting
-//   sort of the labels (chunk histograms, column scans, ballot-ranked
-//   scatter; the chunk histograms come with the labels) -> per-cluster sums by one owner wave per cluster, in sorted
-//   row order (exact int64 fixed point for query clusters; sequential fp32
-//   for key clusters, which also writes the cluster-ordered V) -> value
-//   statistics (lam, sumv).
+//   prep centroids -> assign (MFMA distances + argmin, and the label histogram
+//   of the work-group's rows) -> stable counting sort of the labels (column
+//   scans, ballot-ranked scatter) -> per-cluster sums in sorted row order
+//   (exact int64 fixed point for query clusters; sequential fp32 for key
+//   clusters, which also writes the cluster-ordered V) -> value statistics
+//   (lam, sumv).
 #include "t2t_common.h"
 
 #define KM_R 32            // rank of the projected space
@@ -17,7 +17,7 @@
 static inline int pad32(int c) { return (c + 31) & ~31; }
 
 // ---------------------------------------------------------------------------
-// fast_assign (init_state).  Transposed MFMA product: centroids on the row
+// fast_assign, general form (D = 64 and 128).  Transposed MFMA product: centroids on the row
 // axis (A), tokens on the column axis (B), so a lane owns one token and 16
 // centroids per 32-centroid block, visited in ascending index order:
 // d2 = |x|^2 + (cn2 - 2 x.c); key = (bits(d2) & ~m) | c, the smallest key wins.
@@ -498,7 +498,8 @@ __global__ __launch_bounds__(AK_WAVES * 64 * CS) void assign_km_kernel(AssignArg
 // ---------------------------------------------------------------------------
 // stable counting sort of labels -> counts, cbase (exclusive scan), perm, over
 // chunks of 256 RB rows.  Like the assignment, each kernel takes up to two
-// label sets in one launch (blockIdx.z).
+// label sets in one launch (blockIdx.z).  Rows whose label is not in [0, C) are
+// in no cluster: not counted, and perm ends before them.
 // ---------------------------------------------------------------------------
 struct SortArgs {
   const int32_t* lab;  // [H, N]
@@ -518,7 +519,10 @@ __global__ __launch_bounds__(256) void sort_hist_kernel(const int32_t* __restric
   __syncthreads();
   const int r0 = k * rows;
   const int r1 = (r0 + rows) < N ? (r0 + rows) : N;
-  for (int r = r0 + tid; r < r1; r += 256) atomicAdd(&hist[lab[(size_t)h * N + r]], 1);
+  for (int r = r0 + tid; r < r1; r += 256) {
+    const int c = lab[(size_t)h * N + r];
+    if ((unsigned)c < (unsigned)C) atomicAdd(&hist[c], 1);
+  }
   __syncthreads();
   int32_t* out = chist + ((size_t)h * gridDim.x + k) * C;
   for (int i = tid; i < C; i += 256) out[i] = hist[i];
@@ -592,13 +596,14 @@ __global__ __launch_bounds__(256) void sort_scatter_kernel(SortArgs g0, SortArgs
 #pragma unroll
   for (int i = 0; i < RB; ++i) {
     const int row = r0 + 64 * i + l;
-    labs[i] = row < N ? g.lab[(size_t)h * N + row] : 0;
+    labs[i] = row < N ? g.lab[(size_t)h * N + row] : -1;
+    if ((unsigned)labs[i] >= (unsigned)C) labs[i] = -1;  // in no cluster
   }
   for (int c = l; c < C; c += 64) mine[c] = 0;
   wave_sync_km();
 #pragma unroll
   for (int i = 0; i < RB; ++i)
-    if (r0 + 64 * i + l < N) atomicAdd(&mine[labs[i]], 1);
+    if (labs[i] >= 0) atomicAdd(&mine[labs[i]], 1);
   // exclusive scan of the head's counts: thread tid owns clusters per tid ..
   const int per = (C + 255) / 256;
   const int32_t* cnt = g.counts + (size_t)h * C;
@@ -633,8 +638,8 @@ __global__ __launch_bounds__(256) void sort_scatter_kernel(SortArgs g0, SortArgs
   for (int i = 0; i < RB; ++i) {
     const int row = r0 + 64 * i + l;
     if (r0 + 64 * i >= N) break;  // wave-uniform
-    const bool valid = row < N;
     const int c = labs[i];
+    const bool valid = c >= 0;
     unsigned long long peers = __ballot(valid);
     for (int b = 0; b < lbits; ++b) {
       const unsigned long long bb = __ballot((c >> b) & 1);
@@ -831,7 +836,8 @@ static void launch_fixed_mean(const void* X, const int32_t* perm, const int32_t*
 // perm == nullptr: rows are already cluster ordered (V_sorted input).
 // ---------------------------------------------------------------------------
 // MEAN: vsum and ck2 hold the cluster's means of V (over max(n, 1)) and KU (the
-// fused_update_vstats outputs), and cmax is not written.
+// fused_update_vstats outputs), and cmax is not written; or, where ck16 is given,
+// ck16 and V_sorted hold those means in 16 bits (fp16, and V's type).
 #define KG_UNR 16
 template <typename T, bool MEAN>
 __global__ __launch_bounds__(256) void key_gather_kernel(
@@ -852,7 +858,7 @@ __global__ __launch_bounds__(256) void key_gather_kernel(
   // V row n of head h at V + h svh + n svn (elements; svn even)
   const uint32_t* vh = (const uint32_t*)(V + (size_t)h * svh);
   const size_t vrow = (size_t)(svn >> 1);
-  uint32_t* vsh = V_sorted ? (uint32_t*)(V_sorted + (size_t)h * N * 128) : nullptr;
+  uint32_t* vsh = !MEAN && V_sorted ? (uint32_t*)(V_sorted + (size_t)h * N * 128) : nullptr;
   // lanes 0..15 also sum the projected key rows, dims 2 l and 2 l + 1 (one
   // 4-byte load per row; each dim still sums its rows in order)
   float ax0 = 0.f, ax1 = 0.f, v0 = 0.f, v1 = 0.f;
@@ -906,28 +912,37 @@ __global__ __launch_bounds__(256) void key_gather_kernel(
     run(std::true_type{});
   else
     run(std::false_type{});
-  float* vo = vsum + ((size_t)h * C + c) * 128 + 2 * l;
+  const size_t vi = ((size_t)h * C + c) * 128 + 2 * l;
   if constexpr (MEAN) {
     const float d = n ? (float)n : 1.0f;
-    vo[0] = v0 / d;
-    vo[1] = v1 / d;
+    const float w0 = opaque(v0 / d), w1 = opaque(v1 / d);
+    if (ck16) {
+      *(uint32_t*)(V_sorted + vi) = (uint32_t)T::from_f(w0) | ((uint32_t)T::from_f(w1) << 16);
+    } else {
+      vsum[vi] = w0;
+      vsum[vi + 1] = w1;
+    }
   } else {
+    float* vo = vsum + vi;
     vo[0] = v0;
     vo[1] = v1;
     // the cluster's largest |value sum|, for the per-head scale lam
     const float mx = wave_max(fmaxf(fabsf(v0), fabsf(v1)));
     if (l == 0) cmax[(size_t)h * C + c] = mx;
   }
-  if (ck2 && l < 16) {
+  if ((ck2 || (MEAN && ck16)) && l < 16) {
     const size_t o = ((size_t)h * C + c) * KM_R + 2 * l;
     const float m0 = opaque(n ? ax0 / (float)n : h2f(ck0[o]));
     const float m1 = opaque(n ? ax1 / (float)n : h2f(ck0[o + 1]));
-    ck2[o] = m0;
-    ck2[o + 1] = m1;
+    if (ck2) {
+      ck2[o] = m0;
+      ck2[o + 1] = m1;
+    }
     if (ck16) {  // the finalised centroids as well (centroid_finalize_kernel)
       *(uint32_t*)(ck16 + o) = (uint32_t)f2h(m0) | ((uint32_t)f2h(m1) << 16);
-      *(uint32_t*)(cks + o) =
-          (uint32_t)f2h(opaque(m0 * scale)) | ((uint32_t)f2h(opaque(m1 * scale)) << 16);
+      if constexpr (!MEAN)
+        *(uint32_t*)(cks + o) =
+            (uint32_t)f2h(opaque(m0 * scale)) | ((uint32_t)f2h(opaque(m1 * scale)) << 16);
     }
   }
 }
@@ -1365,12 +1380,13 @@ __global__ __launch_bounds__(256) void seg_mean_kernel(
   }
 }
 
-extern "C" int t2t_fused_update_vstats(const void* x, const int32_t* labels, const void* old,
-                                       const void* v, int v_dtype, float* cent, int32_t* counts,
-                                       float* vmean, int H, int N, int C, int D, void* ws,
-                                       size_t ws_bytes, void* stream) {
-  T2T_REQUIRE(x && labels && old && cent && counts, "fused_update_vstats: null pointer");
-  T2T_REQUIRE(!v || vmean, "fused_update_vstats: v given without vmean");
+// cent / vmean in fp32, or cent16 / vmean16 in fp16 and v's type
+static int update_impl(const void* x, const int32_t* labels, const void* old, const void* v,
+                       int v_dtype, float* cent, void* cent16, int32_t* counts, float* vmean,
+                       void* vmean16, int H, int N, int C, int D, void* ws, size_t ws_bytes,
+                       void* stream) {
+  T2T_REQUIRE(x && labels && old && (cent || cent16) && counts, "fused_update_vstats: null pointer");
+  T2T_REQUIRE(!v || vmean || vmean16, "fused_update_vstats: v given without vmean");
   T2T_REQUIRE(!v || v_dtype == T2T_F16 || v_dtype == T2T_BF16, "fused_update_vstats: dtype %d",
               v_dtype);
   T2T_REQUIRE(H > 0 && N > 0 && C >= 1 && C <= KM_MAXC, "fused_update_vstats: H=%d N=%d C=%d", H,
@@ -1385,22 +1401,37 @@ extern "C" int t2t_fused_update_vstats(const void* x, const int32_t* labels, con
   DetWs w = det_layout(H, N, C, ws);
   KM_CHECK(run_sort(labels, counts, w.cbase, w.perm, w.chist, H, N, C, st));
   const long long vs = (long long)N * 128;
-  const dim3 g(cdiv(C, 4), H);
+#define UP_LAUNCH(T)                                                                              \
+  hipLaunchKernelGGL((key_gather_kernel<T, true>), dim3(cdiv(C, 4), H), dim3(256), 0, st,         \
+                     (const uint16_t*)x, (const uint16_t*)v, w.perm, counts, w.cbase,             \
+                     (const uint16_t*)old, cent, (uint16_t*)vmean16, vmean, (float*)nullptr, N, C, \
+                     vs, 128ll, (uint16_t*)cent16, (uint16_t*)nullptr, 0.f)
   if (!v)
     hipLaunchKernelGGL(seg_mean_kernel, dim3(cdiv(C, 16), H), dim3(256), 0, st, (const uint16_t*)x,
-                       w.perm, counts, w.cbase, (const uint16_t*)old, cent, (uint16_t*)nullptr, N, C);
+                       w.perm, counts, w.cbase, (const uint16_t*)old, cent, (uint16_t*)cent16, N, C);
   else if (v_dtype == T2T_BF16)
-    hipLaunchKernelGGL((key_gather_kernel<BF16T, true>), g, dim3(256), 0, st, (const uint16_t*)x,
-                       (const uint16_t*)v, w.perm, counts, w.cbase, (const uint16_t*)old, cent,
-                       (uint16_t*)nullptr, vmean, (float*)nullptr, N, C, vs, 128ll,
-                       (uint16_t*)nullptr, (uint16_t*)nullptr, 0.f);
+    UP_LAUNCH(BF16T);
   else
-    hipLaunchKernelGGL((key_gather_kernel<F16T, true>), g, dim3(256), 0, st, (const uint16_t*)x,
-                       (const uint16_t*)v, w.perm, counts, w.cbase, (const uint16_t*)old, cent,
-                       (uint16_t*)nullptr, vmean, (float*)nullptr, N, C, vs, 128ll,
-                       (uint16_t*)nullptr, (uint16_t*)nullptr, 0.f);
+    UP_LAUNCH(F16T);
+#undef UP_LAUNCH
   T2T_LAUNCH_CHECK("fused_update_vstats");
   return T2T_OK;
+}
+
+extern "C" int t2t_fused_update_vstats(const void* x, const int32_t* labels, const void* old,
+                                       const void* v, int v_dtype, float* cent, int32_t* counts,
+                                       float* vmean, int H, int N, int C, int D, void* ws,
+                                       size_t ws_bytes, void* stream) {
+  return update_impl(x, labels, old, v, v_dtype, cent, nullptr, counts, vmean, nullptr, H, N, C, D, ws,
+                     ws_bytes, stream);
+}
+
+extern "C" int t2t_fused_update_vstats16(const void* x, const int32_t* labels, const void* old,
+                                         const void* v, int v_dtype, void* cent16, int32_t* counts,
+                                         void* vmean16, int H, int N, int C, int D, void* ws,
+                                         size_t ws_bytes, void* stream) {
+  return update_impl(x, labels, old, v, v_dtype, nullptr, cent16, counts, nullptr, vmean16, H, N, C, D,
+                     ws, ws_bytes, stream);
 }
 
 // ---- warm Lloyd iterations (init_state) ----

@@ -165,11 +165,7 @@ def fused_update_vstats(ku, labels, old_centroids, v=None, *, BLOCK_N=32, num_wa
                          f"{tuple(ku.shape)}, got {tuple(v.shape)}")
     cent, counts, vmean = ops.fused_update_vstats(
         ku.contiguous(), labels.to(torch.int32).contiguous(), old_centroids.contiguous(),
-        None if v is None else v.contiguous())
-    if not return_fp32:
-        cent = cent.to(ku.dtype)
-        if vmean is not None:
-            vmean = vmean.to(v.dtype)
+        None if v is None else v.contiguous(), half=not return_fp32)
     return cent, counts, vmean
 
 

@@ -8,6 +8,7 @@ library and CUDA (ROCm) tensors.
 from __future__ import annotations
 
 import math
+from contextlib import nullcontext
 
 import torch
 
@@ -600,12 +601,14 @@ def det_centroid_update(x, labels, old, stream=None):
     return new, counts
 
 
-def fused_update_vstats(x, labels, old, v=None, stream=None, check_labels=True):
+def fused_update_vstats(x, labels, old, v=None, stream=None, check_labels=True, half=False):
     """fp32 centroid means (empty clusters keep ``old``), counts, and the
     fp32 per-cluster means of v when given -> (cent fp32 [H, C, D], counts
-    int32 [H, C], vmean fp32 [H, C, 128] or None).  ``check_labels`` reads
-    the label range back to the host (a synchronisation); callers whose
-    labels come from an assignment kernel pass False."""
+    int32 [H, C], vmean fp32 [H, C, 128] or None); with ``half`` the means are
+    rounded to x's and v's types.  ``check_labels`` raises ValueError for labels
+    outside [0, C), which the kernels leave out of every cluster (it reads the
+    counts' sum back, a synchronisation); callers whose labels come from an
+    assignment kernel pass False."""
     H, N, D = x.shape
     C = old.shape[1]
     dev = _dev(x)
@@ -614,16 +617,21 @@ def fused_update_vstats(x, labels, old, v=None, stream=None, check_labels=True):
     _check(old, (H, C, D), _f16, "old", dev)
     if v is not None:
         _check(v, (H, N, HEAD_DIM), _HALF, "v", dev)
-    if check_labels:
-        lo, hi = (int(t) for t in torch.aminmax(labels))
-        if lo < 0 or hi >= C:
-            raise ValueError(f"t2t: labels must lie in [0, {C}), got [{lo}, {hi}]")
-    cent = torch.empty(H, C, D, dtype=_f32, device=dev)
+    cent = torch.empty(H, C, D, dtype=_f16 if half else _f32, device=dev)
     counts = torch.empty(H, C, dtype=_i32, device=dev)
-    vmean = None if v is None else torch.empty(H, C, HEAD_DIM, dtype=_f32, device=dev)
+    vmean = None
+    if v is not None:
+        vmean = torch.empty(H, C, HEAD_DIM, dtype=v.dtype if half else _f32, device=dev)
     ws = _ws(size_query("t2t_det_update_ws_bytes", H, N, C), dev)
-    call("t2t_fused_update_vstats", x, labels, old, v, dtype_code(v.dtype) if v is not None else 0,
-         cent, counts, vmean, H, N, C, D, ws, ws.numel(), stream_handle(stream))
+    call("t2t_fused_update_vstats16" if half else "t2t_fused_update_vstats", x, labels, old, v,
+         dtype_code(v.dtype) if v is not None else 0, cent, counts, vmean, H, N, C, D, ws, ws.numel(),
+         stream_handle(stream))
+    if check_labels:
+        with torch.cuda.stream(stream) if stream is not None else nullcontext():
+            rows = int(counts.sum())
+        if rows != H * N:
+            lo, hi = (int(t) for t in torch.aminmax(labels))
+            raise ValueError(f"t2t: labels must lie in [0, {C}), got [{lo}, {hi}]")
     return cent, counts, vmean
 
 
