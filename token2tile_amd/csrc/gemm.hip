@@ -398,7 +398,7 @@ extern "C" int t2t_score(const void* QU, const void* cks, void* gl, int H, int N
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 #define GR_ROWS 64      // rows staged per step
 #define GR_PITCH 144    // floats per staged row: the four rows of a fragment read start 16 banks apart
-#define GR_MAXSPLIT 64  // row splits per head (partial Grams in the workspace)
+#define GR_MAXSPLIT 128 // row splits per head (partial Grams in the workspace)
 
 // the 36 blocks (i <= j) of the upper triangle of 8 x 8 blocks of 16 columns,
 // nine per wave
@@ -420,7 +420,7 @@ __device__ constexpr GrPairs GR_PAIR = gr_pairs();
 // Partial Gram products on fp64 MFMA (v_mfma_f64_16x16x4_f64).  Block (s, h)
 // sums rows [s R, s R + R) of head h; the result is symmetric, so only the
 // 36 blocks on and above the diagonal are formed, nine per wave (40 x 75600 x
-// 128: 2.83 ms with all 64 blocks, 1.16 with these, 48 TFLOP/s where a large
+// 128: 2.83 ms with all 64 blocks, 0.97 with these, 57 TFLOP/s where a large
 // fp64 matrix product reaches 61).  Rows are staged through LDS as fp32 (exact for fp16 values; bf16 is
 // rounded to fp16 first, as the reference's backend casts to fp16), the next
 // rows' loads in flight meanwhile.  For a k-step of four rows, lane l holds
@@ -545,8 +545,13 @@ __global__ __launch_bounds__(256) void gram_reduce_kernel(const double* __restri
   if (gi / 16 < gj / 16) G[(size_t)h * D * D + (size_t)gj * D + gi] = acc;
 }
 
+// Row splits per head: 512 work-groups run at once (two per CU by their
+// registers), so the grid stays just under one round of them, or two where that
+// still leaves a head 64 splits or fewer.  (Rounded up to 1040, 40 heads x 75600
+// ran a third round of 16 work-groups: 1.14 ms against 0.97; 5 heads at 64
+// splits, 1.25 work-groups a CU: 212 us against 154 at 102.)
 static int gram_splits(int H, int N) {
-  int S = (1024 + H - 1) / H;  // about 1024 work-groups
+  int S = 1024 / H <= 64 ? 1024 / H : 512 / H;
   const int maxS = (N + 4 * GR_ROWS - 1) / (4 * GR_ROWS);  // >= 4 staging steps per split
   if (S > maxS) S = maxS;
   if (S > GR_MAXSPLIT) S = GR_MAXSPLIT;
