@@ -34,3 +34,32 @@ def test_eigh_robust_matches_eigh_on_host():
     m = a @ a.transpose(1, 2)
     e, v = DS._eigh_robust(m)
     assert torch.allclose(v @ torch.diag_embed(e) @ v.transpose(1, 2), m, atol=1e-10)
+
+
+# a full-rank Gram, and few effective dimensions beside one large channel, every
+# Gram eigenvalue far above the floor of 1e-8
+@pytest.mark.parametrize("rank,channel,rest", [(128, 0.0, 0.5), (2, 1000.0, 0.01),
+                                               (1, 30000.0, 0.01)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_projection_fit_of_graded_inputs(rank, channel, rest, dtype):
+    """However the singular values are graded, the Cholesky form's score products
+    are as near to the scores as the square-root form's, and fp16 holds its
+    projections and the projected rows.  (Both take V from an eigensolution of
+    M^T M, which resolves singular values down to sqrt(eps) = 1.5e-8 of the
+    largest: that much is allowed beside the truncation.)"""
+    gen = torch.Generator().manual_seed(rank)
+    r = lambda *s: torch.randn(*s, generator=gen)  # noqa: E731
+    basis = 0.5 * r(rank, 128)
+    x = [r(2000, rank) @ basis + rest * r(2000, 128) for _ in range(2)]
+    for t in x:
+        t[:, 7] += channel
+    q, k = (t.to(dtype).half().double().unsqueeze(0) for t in x)
+    Mq, Mk = (t.transpose(1, 2) @ t / 2000 for t in (q, k))
+    assert min(float(torch.linalg.eigvalsh(M).min()) for M in (Mq, Mk)) > 1e-5
+    Uq, Uk = DS._fit_chol(Mq, Mk, torch.linalg.cholesky(Mk), 32)
+    for t, U in ((q, Uq), (k, Uk)):
+        assert bool(U.half().isfinite().all())
+        assert bool((t @ U.half().double()).half().isfinite().all())
+    S = q @ k.transpose(1, 2)
+    err = lambda a, b: float(((q @ a) @ (k @ b).transpose(1, 2) - S).norm() / S.norm())  # noqa: E731
+    assert err(Uq, Uk) <= 1.1 * err(*DS._fit_eigh(Mq, Mk, 32)) + 1.5e-8

@@ -91,13 +91,15 @@ def _fit_chol(Mq, Mk, L, r):
     """The same fit where every Gram eigenvalue is above the floor.  Any factor
     of a Gram serves as its root: with Mk = L L^T and Mq = F F^T, M = F^T L has
     the singular values of Rq Rk and M^T M = L^T Mq L, so one eigensolution is
-    left.  The inverses cancel: Uq = F^-T U S^1/2 = L V S^-1/2 and
-    Uk = L^-T V S^1/2 = Mq Uq S^-1."""
-    MqL = torch.bmm(Mq, L)
-    w, V = _eigh_robust(torch.bmm(L.transpose(1, 2).contiguous(), MqL))
+    left: Uq = F^-T U S^1/2 = L V S^-1/2 and Uk = L^-T V S^1/2.  (Uk also equals
+    Mq L V S^-3/2, but the eigensolver's absolute noise in V, about the machine
+    epsilon of the largest S, grows without bound there where S is small: inputs
+    of few effective dimensions beside one large channel left fp16's range.)"""
+    w, V = _eigh_robust(torch.bmm(L.transpose(1, 2).contiguous(), torch.bmm(Mq, L)))
     Vr = V[:, :, -r:].flip(-1).contiguous()
     sr = w[:, -r:].flip(-1).clamp_min(1e-30).sqrt().unsqueeze(1)
-    return torch.bmm(L, Vr) * sr.rsqrt(), torch.bmm(MqL, Vr) * sr.pow(-1.5)
+    Uk = torch.linalg.solve_triangular(L.transpose(1, 2), Vr, upper=True) * sr.sqrt()
+    return torch.bmm(L, Vr) * sr.rsqrt(), Uk
 
 
 def online_u(qf, kf, r=32):
