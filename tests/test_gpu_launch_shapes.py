@@ -140,6 +140,22 @@ def test_projection_fit_forms(dev, D):
     assert torch.equal(Uq, Eq.float()) and torch.equal(Uk, Ek.float())
 
 
+def test_projection_fit_of_a_head_ignores_its_neighbours(dev):
+    """A head with a dead channel takes the square-root form alone: the heads
+    beside it get, bit for bit, what they get without it."""
+    from token2tile_amd import deploy_step as DS, ops
+    gen = torch.Generator(device=dev).manual_seed(7)
+    q, k = (torch.randn(5, 3000, 128, generator=gen, device=dev).half() for _ in range(2))
+    qz, kz = q.clone(), k.clone()
+    qz[1, :, 9] = 0
+    kz[4, :, 100] = 0
+    plain, mixed = DS.online_u(q, k), DS.online_u(qz, kz)
+    same, low = [0, 2, 3], [1, 4]
+    E = DS._fit_eigh(*(ops.gram_strided(t)[low] for t in (qz, kz)), 32)
+    for a, b, e in zip(plain, mixed, E):
+        assert torch.equal(a[same], b[same]) and torch.equal(b[low], e.float())
+
+
 # row blocks per wave 4, 2 and 1 (rows in whole, partial and single chunks; a head
 # alone and the last shape with two centroid groups), the key pass sharing the first query pass's launches with more and fewer clusters
 @pytest.mark.parametrize("H,N,CQ,CK,pin", [(8, 131100, 200, 2048, 0), (16, 16450, 33, 500, 77),

@@ -102,6 +102,20 @@ def _fit_chol(Mq, Mk, L, r):
     return torch.bmm(L, Vr) * sr.rsqrt(), Uk
 
 
+def _fit_heads(Mq, Mk, L, low, r):
+    """_fit_chol, and _fit_eigh for the heads ``low`` whose Grams have eigenvalues
+    at the floor.  Those heads' places in the batch hold unit matrices, so what
+    the others get does not depend on them."""
+    if len(low) == Mq.shape[0]:
+        return _fit_eigh(Mq, Mk, r)
+    if not low:
+        return _fit_chol(Mq, Mk, L, r)
+    idx = torch.tensor(low, device=Mq.device)
+    unit = torch.eye(Mq.shape[1], dtype=Mq.dtype, device=Mq.device).expand(len(low), -1, -1)
+    fits = _fit_chol(*(M.index_copy(0, idx, unit) for M in (Mq, Mk, L)), r)
+    return tuple(U.index_copy(0, idx, E) for U, E in zip(fits, _fit_eigh(Mq[idx], Mk[idx], r)))
+
+
 def online_u(qf, kf, r=32):
     """Matched rank-r projections Uq, Uk [H, D, r] (fp32) minimising
     ||Q K^T - (Q Uq)(K Uk)^T||_F (deploy_step.py:122-149).
@@ -109,8 +123,8 @@ def online_u(qf, kf, r=32):
     The Gram matrices come from the HIP fp64 Gram kernel (16-bit inputs, read
     in place) or from fp64 matmul for fp32 inputs; the 128 x 128 problems run
     batched in fp64 on the GPU: a Cholesky factor and one symmetric
-    eigensolution (_fit_chol), or three eigensolutions where a Gram has
-    eigenvalues at the floor (_fit_eigh).  The reference backend's fast
+    eigensolution (_fit_chol), or three eigensolutions for the heads where a
+    Gram has eigenvalues at the floor (_fit_eigh).  The reference backend's fast
     initialisation eigensolves in the same way (t2t_attn.py:211-239): a
     batched symmetric eigensolver is two orders of magnitude faster here than
     a batched SVD.  Raises RuntimeError on non-finite input."""
@@ -136,10 +150,10 @@ def online_u(qf, kf, r=32):
     Mq = ops.gram_strided(rows(qf), flags[0])
     Mk = ops.gram_strided(rows(kf), flags[1])
     L = ops.fit_chol(Mq, Mk, _EIG_FLOOR, flags[2:])
-    bad_q, bad_k, *small = (any(f) for f in flags.tolist())
-    if bad_q or bad_k:
+    bad_q, bad_k, small_q, small_k = flags.tolist()
+    if any(bad_q) or any(bad_k):
         _require_finite(q=qf, k=kf)
-    Uq, Uk = _fit_eigh(Mq, Mk, r) if any(small) else _fit_chol(Mq, Mk, L, r)
+    Uq, Uk = _fit_heads(Mq, Mk, L, [h for h in range(H) if small_q[h] or small_k[h]], r)
     return Uq.float().contiguous(), Uk.float().contiguous()
 
 
