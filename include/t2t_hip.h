@@ -246,7 +246,8 @@ int t2t_tile_attn_exact_orig_gather_kv_strided(
     void* stream);
 /* The three calls above with a workspace (t2t_tile_attn_split_ws_bytes; 0 where
  * the sizes fill the GPU and nothing is split): a small call's tasks are split
- * along the keys and their parts added in fp32.  gather 0: k and v are the
+ * along the keys and their parts added in fp32; with less (or NULL) they are
+ * not split.  gather 0: k and v are the
  * cluster-ordered kp and vp (contiguous; kperm unused); 1: k in the original
  * order through kperm; 2: k and v.  qlab: the query labels that qperm sorts.
  * The results do not depend on gather.  No counterpart in the reference. */
@@ -301,7 +302,9 @@ int t2t_resid_merge_inplace(void* out, const float* lse, const void* QU, const v
                             const int32_t* qperm, const float* lam, const float* tailw_dev,
                             int dtype, int H, int N, int CQ, void* stream);
 /* Workspace bytes of t2t_tile_attn_run_planned: lse [H, N] fp32, the centroid
- * tile image and the parts of a small call's split tasks. */
+ * tile image (t2t_centroid_tiles_bytes) and the parts of a small call's split
+ * tasks.  The parts are optional: a workspace that holds only the first two
+ * (256-byte aligned) serves, with nothing split. */
 size_t t2t_tile_attn_ws_bytes(int H, int N, int dtype);
 /* Plan (when rebuild_plan != 0), exact attention, residual and merge in
  * one call: the exact part is written to the original rows of out and the

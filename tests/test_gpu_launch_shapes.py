@@ -376,6 +376,48 @@ def test_split_call_equals_its_stages(dev, H, N, CQ, dtype):
     assert not a.isnan().any() and torch.equal(a, b)
 
 
+# parts added by the combine, and by the residual
+@pytest.mark.parametrize("H,N,CQ", [(1, 4100, 16), (3, 12000, 60)])
+def test_attention_without_room_for_parts(dev, H, N, CQ):
+    """A workspace of lse and the tile image alone, as one sized for a longer
+    sequence may be, serves a small call unsplit: the bits of the whole-task
+    kernel and the residual after it."""
+    from token2tile_amd import _lib, ops
+    rng = np.random.default_rng(N)
+    qlab, klab, qperm, qcounts, kperm, kcounts = structure(rng, H, N, CQ)
+    sel = (rng.random((H, CQ, 2048)) < 0.3).astype(np.uint8)
+    unip = np.packbits(sel, axis=2, bitorder="little").view(np.int32)
+    gen = torch.Generator(device=dev).manual_seed(N)
+    r = lambda *s: torch.randn(*s, generator=gen, device=dev)  # noqa: E731
+    q, kp, vp = (r(H, N, 128).half() for _ in range(3))
+    QU, cks, sumv = r(H, N, 32).half(), (0.1 * r(H, 2048, 32)).half(), r(H, 2048, 128).half()
+    lam, tw = torch.linspace(1, 2, H, device=dev), torch.tensor(1.0, device=dev)
+    tq, tk, tu, tqp, tql = (g(a, dev) for a in (qcounts, kcounts, unip, qperm, qlab))
+    plan = ops.tile_plan(tq, tk, tu, N)
+    a, lse = torch.full_like(q, float("nan")), torch.empty(H, N, device=dev)
+    ops.tile_attn_exact_orig(q, kp, vp, tk, tu, tqp, plan, a, lse)
+    one = torch.full_like(q, float("nan"))
+    lse1 = torch.empty_like(lse)
+    assert ops.attn_split_ws_bytes(H, N, CQ) > 0
+    hs = N * 128
+    for ws, size in ((None, 0), (torch.empty(256, dtype=torch.uint8, device=dev), 256)):
+        one.fill_(float("nan"))
+        _lib.call("t2t_tile_attn_exact_split", q, hs, 128, kp, hs, 128, vp, hs, 128, None, 0, 0, tk, tu,
+                  tql, tqp, plan, one, hs, 128, lse1, H, N, CQ, ws, size, _lib.stream_handle())
+        assert torch.equal(one, a) and torch.equal(lse1, lse)
+    ops.resid_merge_inplace(a, lse, QU, ops.centroid_tiles(cks, sumv), tk, tu, tql, tqp, lam, tw)
+    size = -(-H * N * 4 // 256) * 256 + ops.size_query("t2t_centroid_tiles_bytes", H)
+    assert size < ops.attn_ws_bytes(H, N, q.dtype)
+    ws = torch.empty(size + 512, dtype=torch.uint8, device=dev)
+    ws[size:] = 77
+    for rebuild in (True, False):
+        b = torch.full_like(q, float("nan"))
+        ops.tile_attn_run_planned(q, kp, vp, tq, tk, tu, QU, cks, sumv, lam, tql, tqp, tw, b, plan,
+                                  rebuild, ws=ws[:size])
+        assert not a.isnan().any() and torch.equal(a, b)
+    assert bool((ws[size:] == 77).all())
+
+
 @pytest.mark.parametrize("H,N,C", [(2, 1000, 33), (1, 300, 2048)])
 def test_update_leaves_foreign_labels_out(dev, H, N, C):
     """Rows labelled outside [0, C) belong to no cluster (the checked call raises

@@ -1037,6 +1037,14 @@ static SplitWs split_layout(int H, int N, int S, void* base) {
   return v;
 }
 
+// Most parts per task with the workspace at hand (1, unsplit, where the parts
+// do not fit it): the exact attention and the residual of a call ask with the
+// same workspace.
+static int split_with(int H, int N, int CQ, const void* ws, size_t ws_bytes) {
+  const int S = split_max(H, N, CQ);
+  return ws && ws_bytes >= split_layout(H, N, S, nullptr).total ? S : 1;
+}
+
 template <typename T, int MODE>
 static void launch_attn_split(const void* q, const void* k, const void* v, const int32_t* unip,
                               const int32_t* qlab, const int32_t* qperm, const int32_t* kcounts,
@@ -1655,12 +1663,8 @@ static int exact_impl(int mode, const void* q, const void* k, const void* v, con
                 "elements, more than 4 GiB", rs);
   PlanView p = plan_view((int32_t*)plan, H, N, CQ);
   hipStream_t st = (hipStream_t)stream;
-  const int S = qlab ? split_max(H, N, CQ) : 1;
+  const int S = qlab ? split_with(H, N, CQ, ws, ws_bytes) : 1;
   const SplitWs w = split_layout(H, N, S, ws);
-  if (S > 1 && (!ws || ws_bytes < w.total)) {
-    t2t_set_error("tile_attn_exact_split: workspace %zu < %zu bytes", ws_bytes, w.total);
-    return T2T_ERR_WORKSPACE;
-  }
   if (dtype == T2T_F16)
     exact_launch<F16T>(mode, q, k, v, sd, kperm, kcounts, unip, qlab, qperm, p, out, lse, H, N, CQ, S,
                        w, combine, st);
@@ -1778,12 +1782,8 @@ int t2t_resid_merge_parts(void* out, long long soh, long long son, const float* 
                           const float* lam, const float* tailw_dev, int dtype, int H, int N, int CQ,
                           void* ws, size_t ws_bytes, void* stream) {
   T2T_REQUIRE(H > 0 && N > 0 && CQ > 0 && plan, "resid_merge_parts: H=%d N=%d CQ=%d", H, N, CQ);
-  const int S = split_max(H, N, CQ);
+  const int S = split_with(H, N, CQ, ws, ws_bytes);
   const SplitWs w = split_layout(H, N, S, ws);
-  if (S > 1 && (!ws || ws_bytes < w.total)) {
-    t2t_set_error("resid_merge_parts: workspace %zu < %zu bytes", ws_bytes, w.total);
-    return T2T_ERR_WORKSPACE;
-  }
   const PlanView p = plan_view((int32_t*)plan, H, N, CQ);
   return resid_inplace_impl(out, soh, son, lse, QU, tiles, kcounts, unip, qlab, qperm, lam, tailw_dev,
                             dtype, H, N, CQ, stream, SplitIn{w.opart, w.mlpart, p.kvlen, split_in_resid(H, N) ? S : 1});
@@ -1811,7 +1811,9 @@ extern "C" int t2t_resid_merge_inplace_strided(void* out, long long out_head_str
 }
 
 // lse, the centroid tile image, and the parts of a split call at the fewest
-// query clusters (the most parts)
+// query clusters (the most parts).  The parts are optional, and their bytes
+// fall where a longer call is split less: a workspace sized for the longest
+// sequence serves the shorter ones too, unsplit where the parts do not fit.
 extern "C" size_t t2t_tile_attn_ws_bytes(int H, int N, int dtype) {
   (void)dtype;
   if (H <= 0 || N <= 0) return 0;
@@ -1836,7 +1838,7 @@ extern "C" int t2t_tile_attn_run_planned(const void* q, const void* kp, const vo
     const int rc = t2t_tile_plan(qcounts, kcounts, unip, plan, H, N, CQ, stream);
     if (rc) return rc;
   }
-  const size_t need = t2t_tile_attn_ws_bytes(H, N, dtype);
+  const size_t need = t2t_align256((size_t)H * N * sizeof(float)) + t2t_centroid_tiles_bytes(H);
   if (!ws || ws_bytes < need) {
     t2t_set_error("tile_attn_run_planned: workspace of %zu bytes, need %zu", ws_bytes, need);
     return T2T_ERR_WORKSPACE;
@@ -1848,8 +1850,9 @@ extern "C" int t2t_tile_attn_run_planned(const void* q, const void* kp, const vo
   launch_centroid_tiles(cks, sumv, tiles, H, st);
   const long long hs = (long long)N * TA_D;
   const long long sd[8] = {hs, TA_D, hs, TA_D, hs, TA_D, hs, TA_D};
-  const int S = split_max(H, N, CQ);
-  const SplitWs sw = split_layout(H, N, S, (char*)ws + w.off);
+  char* pws = (char*)ws + w.off;  // what is left holds the parts
+  const int S = split_with(H, N, CQ, pws, ws_bytes > w.off ? ws_bytes - w.off : 0);
+  const SplitWs sw = split_layout(H, N, S, pws);
   const bool late = split_in_resid(H, N);
   if (dtype == T2T_F16)
     exact_launch<F16T>(1, q, kp, vp, sd, nullptr, kcounts, unip, qlab, qperm, p, out, lse, H, N, CQ, S,

@@ -566,6 +566,8 @@ def tile_attn_run_planned(q, kp, vp, qcounts, kcounts, unip, QU, cks, sumv, lam,
                 QU=QU, cks=cks, sumv=sumv, lam=lam, qlab=qlab, qperm=qperm, tailw_t=tailw_t,
                 out=out, plan=plan, dt=q.dtype)
     need = attn_ws_bytes(H, N, q.dtype)
+    if ws is not None:  # lse and the tile image suffice: nothing is split then
+        need = min(need, -(-H * N * 4 // 256) * 256 + size_query("t2t_centroid_tiles_bytes", H))
     ws = _ws_for(ws, need, dev)
     call("t2t_tile_attn_run_planned", q, kp, vp, dtype_code(q.dtype), qcounts, kcounts, unip, QU,
          cks, sumv, lam, qlab, qperm, tailw_t, out, plan, int(bool(rebuild)), H, N, CQ, ws,
