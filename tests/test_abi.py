@@ -36,6 +36,29 @@ def test_workspace_queries():
     assert ops.vstats_ws_bytes(2, 16384) >= 2 * 2048 * 128 * 4
 
 
+@pytest.mark.parametrize("query", [
+    lambda L, H, N: L.t2t_kmm_ws_bytes(H, N, 256, 2048),
+    lambda L, H, N: L.t2t_det_update_ws_bytes(H, N, 2048),
+    lambda L, H, N: L.t2t_lloyd_ws_bytes(H, N, 512),
+    lambda L, H, N: L.t2t_vstats_ws_bytes(H, N, 2048),
+    lambda L, H, N: L.t2t_select_ws_bytes(H, N, 256),
+    lambda L, H, N: L.t2t_gram_ws_bytes(H, N, 128),
+])
+def test_a_workspace_serves_every_smaller_call(query):
+    """Launch shapes step with the sizes; the bytes they need must not fall, or
+    a workspace sized for the longest call is refused on a shorter one."""
+    from token2tile_amd import _lib
+    L = _lib.lib()
+    sizes = sorted({*range(1, 200, 13), *range(2048, 110000, 1021), 52000, 52224, 52225, 52500, 75600,
+                    131072, 131073, 262144, 262145, 500000})
+    last = [0] * len(sizes)
+    for H in range(1, 49):
+        row = [query(L, H, N) for N in sizes]
+        assert row == sorted(row)
+        assert all(a <= b for a, b in zip(last, row))
+        last = row
+
+
 @pytest.mark.parametrize("call", [
     lambda L: L.t2t_project(None, 0, None, None, 1, 1, 128, 32, None),
     lambda L: L.t2t_score(None, None, None, 1, 1, 2048, 32, None),

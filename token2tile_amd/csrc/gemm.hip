@@ -560,8 +560,11 @@ static int gram_splits(int H, int N) {
 
 extern "C" size_t t2t_gram_ws_bytes(int H, int N, int D) {
   if (H <= 0 || N <= 0 || D <= 0) return 0;
-  const size_t S = gram_splits(H, N);
-  return t2t_align256(S * H * D * D * sizeof(double)) + t2t_align256(S * H * sizeof(int32_t));
+  // the most splits of all heads at these sizes or smaller ones, so that a
+  // workspace serves every call up to those it was sized for
+  const size_t one = (size_t)H * gram_splits(1, N), most = H > 1024 ? H : 1024;
+  const size_t all = one < most ? one : most;
+  return t2t_align256(all * D * D * sizeof(double)) + t2t_align256(all * sizeof(int32_t));
 }
 
 static int gram_impl(const void* x, int x_dtype, long long sxh, long long sxn, double* G,

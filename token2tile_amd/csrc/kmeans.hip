@@ -693,6 +693,15 @@ static int km_rb(int H, int N) {
   return (long long)H * cdiv(N, 512) >= 512 ? 2 : 1;
 }
 static int km_chunks(int H, int N) { return cdiv(N, 256 * km_rb(H, N)); }
+// Chunks of all heads that a workspace holds.  H km_chunks falls where km_rb
+// steps up; a workspace sized for the longest call has to serve the shorter ones
+// (and fewer heads), so its size must not: one row block has at most 2 x 511
+// chunks, two at most 2 x 1023.
+static size_t km_chunk_cap(int H, int N) {
+  const size_t one = (size_t)H * cdiv(N, 256), four = (size_t)H * cdiv(N, 1024);
+  const size_t most = four > 2046 ? four : 2046;
+  return one < most ? one : most;
+}
 
 // the sort proper, from the chunk histograms; sets: 1 or 2
 static int run_scatter(const SortArgs& a, const SortArgs& b, int sets, int H, int N, hipStream_t st) {
@@ -1019,7 +1028,7 @@ struct KmmWs {
 static KmmWs kmm_layout(int H, int N, int CQ, int CK, void* base) {
   WsCarver w(base);
   KmmWs k;
-  const int nChunk = km_chunks(H, N);
+  const size_t chunks = km_chunk_cap(H, N);
   k.qlab1 = w.take<int32_t>((size_t)H * N);
   k.cq1 = w.take<uint16_t>((size_t)H * CQ * KM_R);
   k.perm1 = w.take<int32_t>((size_t)H * N);
@@ -1027,8 +1036,8 @@ static KmmWs kmm_layout(int H, int N, int CQ, int CK, void* base) {
   k.cbase1 = w.take<int32_t>((size_t)H * CQ);
   k.cbaseq = w.take<int32_t>((size_t)H * CQ);
   k.cbasek = w.take<int32_t>((size_t)H * CK);
-  k.chistq = w.take<int32_t>((size_t)H * nChunk * CQ);
-  k.chistk = w.take<int32_t>((size_t)H * nChunk * CK);
+  k.chistq = w.take<int32_t>(chunks * CQ);
+  k.chistk = w.take<int32_t>(chunks * CK);
   k.vsum = w.take<float>((size_t)H * CK * 128);
   k.cmax = w.take<float>((size_t)H * CK);
   k.cprepq = w.take<uint16_t>((size_t)H * CQ * KM_R);
@@ -1321,7 +1330,7 @@ static DetWs det_layout(int H, int N, int C, void* base) {
   DetWs d;
   d.perm = w.take<int32_t>((size_t)H * N);
   d.cbase = w.take<int32_t>((size_t)H * C);
-  d.chist = w.take<int32_t>((size_t)H * km_chunks(H, N) * C);
+  d.chist = w.take<int32_t>(km_chunk_cap(H, N) * C);
   d.total = w.off;
   return d;
 }
