@@ -440,3 +440,38 @@ def test_update_leaves_foreign_labels_out(dev, H, N, C):
             assert all(torch.equal(a, b) for a, b in zip(got, want))
         with pytest.raises(ValueError, match="labels"):
             ops.fused_update_vstats(*args)
+
+
+def test_calls_on_a_stream_allocate_there(dev, monkeypatch):
+    """Scratch and outputs of a call on another stream come from that stream's
+    memory: the current stream's may still be in use by its earlier work, and
+    would go back to it while the call runs."""
+    from token2tile_amd import ops
+    gen = torch.Generator(device=dev).manual_seed(1)
+    r = lambda *s: torch.randn(*s, generator=gen, device=dev).half()  # noqa: E731
+    H, N, CQ, rng = 2, 4096, 16, np.random.default_rng(1)
+    x, q, k, v, old = r(H, N, 32), r(H, N, 128), r(H, N, 128), r(H, N, 128), r(H, 64, 32)
+    qlab, _, qperm, qcounts, kperm, kcounts = structure(rng, H, N, CQ)
+    tq, tk, tp, tl, tkp = (g(a, dev) for a in (qcounts, kcounts, qperm, qlab, kperm))
+    unip = torch.full((H, CQ, 64), -1, dtype=torch.int32, device=dev)
+    plan = ops.tile_plan(tq, tk, unip, N)
+    M, small = ops.gram_strided(q), torch.empty(2, H, dtype=torch.int32, device=dev)
+    want = (ops.lloyd(x, old.clone(), 2), M, ops.fit_chol(M, M, 1e-8, small),
+            ops.tile_attn_exact_split(q, k, v, tkp, tk, unip, tl, tp, plan, torch.empty_like(q),
+                                      torch.empty(H, N, device=dev)))
+    cen, out, lse = old.clone(), torch.empty_like(q), torch.empty(H, N, device=dev)
+    side = torch.cuda.Stream(device=dev)
+    side.wait_stream(torch.cuda.current_stream())
+    made, empty = [], torch.empty
+
+    def recorded(*a, **kw):
+        made.append(torch.cuda.current_stream().cuda_stream)
+        return empty(*a, **kw)
+    monkeypatch.setattr(torch, "empty", recorded)
+    got = (ops.lloyd(x, cen, 2, stream=side), ops.gram_strided(q, stream=side),
+           ops.fit_chol(M, M, 1e-8, small, stream=side),
+           ops.tile_attn_exact_split(q, k, v, tkp, tk, unip, tl, tp, plan, out, lse, stream=side))
+    monkeypatch.undo()
+    torch.cuda.current_stream().wait_stream(side)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    assert len(made) >= 5 and set(made) == {side.cuda_stream}

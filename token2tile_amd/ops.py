@@ -28,11 +28,25 @@ def _dev(t):
     return t.device
 
 
-def _ws(nbytes, device):
-    return torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=device)
+def _new(stream, *shape, dtype, device):
+    """An output of a call on ``stream``: that stream's memory (kernels of the
+    current one may still use what it freed), not reused before the current
+    stream is done with it either."""
+    with torch.cuda.stream(stream):
+        t = torch.empty(*shape, dtype=dtype, device=device)
+    if stream is not None:
+        t.record_stream(torch.cuda.current_stream(device))
+    return t
 
 
-def _ws_for(ws, nbytes, device):
+def _ws(nbytes, device, stream=None):
+    """A call's scratch, of the stream that it runs on: released at return, the
+    memory goes to that stream's later work."""
+    with torch.cuda.stream(stream):
+        return torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=device)
+
+
+def _ws_for(ws, nbytes, device, stream=None):
     """A caller's workspace if it is a large enough uint8 buffer on ``device``,
     else a fresh one.  Its byte count is passed to the library, which checks it."""
     if ws is not None:
@@ -41,7 +55,7 @@ def _ws_for(ws, nbytes, device):
             raise ValueError(f"t2t: ws must be a contiguous uint8 tensor on {device}")
         if ws.numel() >= nbytes:
             return ws
-    return _ws(nbytes, device)
+    return _ws(nbytes, device, stream)
 
 
 _HALF = (torch.float16, torch.bfloat16)
@@ -159,7 +173,7 @@ def kmm_run(QU, KU, V, cq0, ck0, *, pin_tail=0, out=None, ws=None, stream=None,
         if o[name] is not None or name != "V_sorted":
             _check(o[name], shape, dt, name, dev)
     need = kmm_ws_bytes(H, N, CQ, CK)
-    ws = _ws_for(ws, need, dev)
+    ws = _ws_for(ws, need, dev, stream)
     if V.is_contiguous():
         call("t2t_kmm_run", QU, KU, V, dtype_code(V.dtype), cq0, ck0, o["qlab"], o["cq2"],
              o["klab"], o["ck2"], o["qcounts"], o["qperm"], o["kcounts"], o["kperm"],
@@ -199,7 +213,7 @@ def vstats_gather(V, kperm, kcounts, V_sorted=None, sumv=None, lam=None, ws=None
     _check(sumv, (H, CK, HEAD_DIM), _f16, "sumv", dev)
     _check(lam, (H,), _f32, "lam", dev)
     need = vstats_ws_bytes(H, N, CK)
-    ws = _ws_for(ws, need, dev)
+    ws = _ws_for(ws, need, dev, stream)
     if V.is_contiguous():
         call("t2t_kmm_run_vstats_gather", V, dtype_code(V.dtype), kperm, kcounts, V_sorted, sumv,
              lam, H, N, CK, ws, ws.numel(), stream_handle(stream))
@@ -221,7 +235,7 @@ def vstats(V_sorted, kcounts, sumv=None, lam=None, ws=None, stream=None):
     _check(sumv, (H, CK, HEAD_DIM), _f16, "sumv", dev)
     _check(lam, (H,), _f32, "lam", dev)
     need = vstats_ws_bytes(H, N, CK)
-    ws = _ws_for(ws, need, dev)
+    ws = _ws_for(ws, need, dev, stream)
     call("t2t_kmm_run_vstats", V_sorted, dtype_code(V_sorted.dtype), kcounts, sumv, lam, H, N, CK,
          ws, ws.numel(), stream_handle(stream))
     return sumv, lam
@@ -283,7 +297,7 @@ def select_union(gl, kcounts, qperm, qcounts, ns_t, unip=None, rowcnt=None, ws=N
                   unip=unip, rowcnt=rowcnt)
     _check_ns(ns_t, dev)
     need = select_ws_bytes(H, N, CQ)
-    ws = _ws_for(ws, need, dev)
+    ws = _ws_for(ws, need, dev, stream)
     if split_cap:
         call("t2t_select_run_split_packed", gl, kcounts, qperm, qcounts, int(split_cap), ns_t, unip,
              rowcnt, H, N, CQ, ws, ws.numel(), stream_handle(stream))
@@ -310,7 +324,7 @@ def score_select(QU, cks, kcounts, qperm, qcounts, ns_t, unip=None, rowcnt=None,
                   rowcnt=rowcnt)
     _check_ns(ns_t, dev)
     need = select_ws_bytes(H, N, CQ)
-    ws = _ws_for(ws, need, dev)
+    ws = _ws_for(ws, need, dev, stream)
     call("t2t_score_select_packed", QU, cks, kcounts, qperm, qcounts, ns_t, unip, rowcnt, H, N, CQ,
          ws, ws.numel(), stream_handle(stream))
     return unip, rowcnt
@@ -329,7 +343,7 @@ def select_union_bytes(gl, kcounts, qperm, qcounts, ns_t, uni=None, rowcnt=None,
                   rowcnt=rowcnt)
     _check_ns(ns_t, dev)
     need = select_ws_bytes(H, N, CQ)
-    ws = _ws_for(ws, need, dev)
+    ws = _ws_for(ws, need, dev, stream)
     call("t2t_select_run", gl, kcounts, qperm, qcounts, ns_t, uni, rowcnt, H, N, CQ, ws, ws.numel(),
          stream_handle(stream))
     return uni, rowcnt
@@ -430,7 +444,7 @@ def tail_merge(attn_out, lse, QU, cks, sumv, kcounts, unip, qlab, qperm, lam, ta
                 kcounts=kcounts, unip=unip, qlab=qlab, qperm=qperm, lam=lam, tailw_t=tailw_t,
                 dt=attn_out.dtype)
     need = size_query("t2t_tail_merge_ws_bytes", H)
-    ws = _ws_for(ws, need, dev)
+    ws = _ws_for(ws, need, dev, stream)
     call("t2t_tail_merge", attn_out, lse, QU, cks, sumv, kcounts, unip, qlab, qperm, lam, tailw_t,
          out, dtype_code(attn_out.dtype), H, N, CQ, ws, ws.numel(), stream_handle(stream))
     return out
@@ -526,7 +540,7 @@ def tile_attn_exact_split(q, k, v, kperm, kcounts, unip, qlab, qperm, plan, out,
                 lse=lse, dt=q.dtype)
     if gather:
         _check(kperm, (H, N), _i32, "kperm", dev)
-    ws = _ws_for(ws, attn_split_ws_bytes(H, N, CQ), dev)
+    ws = _ws_for(ws, attn_split_ws_bytes(H, N, CQ), dev, stream)
     call("t2t_tile_attn_exact_split", _lib.RowView(q), *sq, _lib.RowView(k), *sk, _lib.RowView(v),
          *sv, kperm if gather else None, int(gather), dtype_code(q.dtype), kcounts, unip, qlab,
          qperm, plan, _lib.RowView(out), *so, lse, H, N, CQ, ws, ws.numel(), stream_handle(stream))
@@ -568,7 +582,7 @@ def tile_attn_run_planned(q, kp, vp, qcounts, kcounts, unip, QU, cks, sumv, lam,
     need = attn_ws_bytes(H, N, q.dtype)
     if ws is not None:  # lse and the tile image suffice: nothing is split then
         need = min(need, -(-H * N * 4 // 256) * 256 + size_query("t2t_centroid_tiles_bytes", H))
-    ws = _ws_for(ws, need, dev)
+    ws = _ws_for(ws, need, dev, stream)
     call("t2t_tile_attn_run_planned", q, kp, vp, dtype_code(q.dtype), qcounts, kcounts, unip, QU,
          cks, sumv, lam, qlab, qperm, tailw_t, out, plan, int(bool(rebuild)), H, N, CQ, ws,
          ws.numel(), stream_handle(stream))
@@ -597,7 +611,7 @@ def det_centroid_update(x, labels, old, stream=None):
     _check(old, (H, C, D), _f16, "old", dev)
     new = torch.empty(H, C, D, dtype=_f16, device=dev)
     counts = torch.empty(H, C, dtype=_i32, device=dev)
-    ws = _ws(size_query("t2t_det_update_ws_bytes", H, N, C), dev)
+    ws = _ws(size_query("t2t_det_update_ws_bytes", H, N, C), dev, stream)
     call("t2t_det_centroid_update", x, labels, old, new, counts, H, N, C, D, ws, ws.numel(),
          stream_handle(stream))
     return new, counts
@@ -624,7 +638,7 @@ def fused_update_vstats(x, labels, old, v=None, stream=None, check_labels=True, 
     vmean = None
     if v is not None:
         vmean = torch.empty(H, C, HEAD_DIM, dtype=v.dtype if half else _f32, device=dev)
-    ws = _ws(size_query("t2t_det_update_ws_bytes", H, N, C), dev)
+    ws = _ws(size_query("t2t_det_update_ws_bytes", H, N, C), dev, stream)
     call("t2t_fused_update_vstats16" if half else "t2t_fused_update_vstats", x, labels, old, v,
          dtype_code(v.dtype) if v is not None else 0, cent, counts, vmean, H, N, C, D, ws, ws.numel(),
          stream_handle(stream))
@@ -645,7 +659,7 @@ def lloyd(x, cen, iters, stream=None):
     dev = _dev(x)
     _check(x, (H, N, D), _f16, "x", dev)
     _check(cen, (H, C, D), _f16, "cen", dev)
-    ws = _ws(size_query("t2t_lloyd_ws_bytes", H, N, C), dev)
+    ws = _ws(size_query("t2t_lloyd_ws_bytes", H, N, C), dev, stream)
     call("t2t_lloyd", x, cen, int(iters), H, N, C, D, ws, ws.numel(), stream_handle(stream))
     return cen
 
@@ -656,7 +670,7 @@ def gram(x, stream=None):
     _check(x, (H, N, D), _HALF, "x", _dev(x))
     G = torch.empty(H, D, D, dtype=torch.float64, device=_dev(x))
     nws = size_query("t2t_gram_ws_bytes", H, N, D)
-    ws = torch.empty(nws, dtype=torch.uint8, device=_dev(x))
+    ws = _ws(nws, _dev(x), stream)
     call("t2t_gram", x, dtype_code(x.dtype), G, H, N, D, ws, nws, stream_handle(stream))
     return G
 
@@ -671,9 +685,9 @@ def gram_strided(x, nonfinite=None, stream=None):
                          f"{tuple(x.shape)} strides {tuple(x.stride())}")
     if nonfinite is not None:
         _check(nonfinite, (H,), _i32, "nonfinite", dev)
-    G = torch.empty(H, D, D, dtype=torch.float64, device=dev)
+    G = _new(stream, H, D, D, dtype=torch.float64, device=dev)
     nws = size_query("t2t_gram_ws_bytes", H, N, D)
-    ws = torch.empty(nws, dtype=torch.uint8, device=dev)
+    ws = _ws(nws, dev, stream)
     call("t2t_gram_strided", _lib.RowView(x), dtype_code(x.dtype), x.stride(0), x.stride(1), G,
          nonfinite, H, N, D, ws, nws, stream_handle(stream))
     return G
@@ -687,6 +701,6 @@ def fit_chol(Mq, Mk, floor, small, stream=None):
     _check(Mq, (H, D, D), torch.float64, "Mq", dev)
     _check(Mk, (H, D, D), torch.float64, "Mk", dev)
     _check(small, (2, H), _i32, "small", dev)
-    L = torch.empty_like(Mk)
+    L = _new(stream, H, D, D, dtype=torch.float64, device=dev)
     call("t2t_fit_chol", Mq, Mk, L, small, H, D, float(floor), stream_handle(stream))
     return L
