@@ -1,5 +1,7 @@
 """Host-side argument checks of the operator surface that run before any
 device work (no GPU needed)."""
+import threading
+
 import pytest
 import torch
 
@@ -63,3 +65,25 @@ def test_projection_fit_of_graded_inputs(rank, channel, rest, dtype):
     S = q @ k.transpose(1, 2)
     err = lambda a, b: float(((q @ a) @ (k @ b).transpose(1, 2) - S).norm() / S.norm())  # noqa: E731
     assert err(Uq, Uk) <= 1.1 * err(*DS._fit_eigh(Mq, Mk, 32)) + 1.5e-8
+
+
+def test_a_call_runs_under_its_own_device(monkeypatch):
+    """Whatever form a call takes, all of it runs with the object's GPU current."""
+    inside = []
+
+    class Guard:
+        def __init__(self, device):
+            self.device = device
+
+        def __enter__(self):
+            inside.append(self.device)
+
+        def __exit__(self, *exc):
+            inside.pop()
+
+    monkeypatch.setattr(torch.cuda, "device", Guard)
+    op = DS.MaskedStepDeploy.__new__(DS.MaskedStepDeploy)
+    op.dev, op._lock = torch.device("cuda", 1), threading.Lock()
+    op._step = lambda *a: (list(inside), a)
+    seen, args = op.step("q", "k", "v", "state")
+    assert seen == [op.dev] and args == ("q", "k", "v", "state", None) and not inside

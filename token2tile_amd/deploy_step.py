@@ -415,7 +415,9 @@ class MaskedStepDeploy:
         holding the centroids that warm-start the next call.  Returns out
         [H, N, 128] in q's dtype: the given ``out`` view (written in place), or
         a buffer reused by the next call."""
-        with self._lock:  # the events and buffers serve one call at a time
+        # the events and buffers serve one call at a time; the launches, events
+        # and the capture query go to this object's GPU whichever is current
+        with self._lock, torch.cuda.device(self.dev):
             return self._step(q, k, v, state, out)
 
     def _step(self, q, k, v, state, out):
