@@ -265,3 +265,34 @@ def test_full_call_shape_sweep(dev, shape):
     eu, er = O.select_union(gl, last["counts"], last["qperm"], last["tile_sizes"], deploy.ns)
     assert np.array_equal(last["unip"], eu)
     assert np.array_equal(deploy.rowcnt.cpu().numpy(), er)
+
+
+def test_settings_and_buffers_replaced_after_construction(dev):
+    """A call takes the operator's settings and buffers as they stand: pin_tail,
+    scale, a replaced buffer, and less room than split tasks need."""
+    from token2tile_amd import ops
+    pinned, q, k, v = make(dev, pin_tail=300)
+    deploy, *_ = make(dev)
+    tq, tk, tv = (torch.from_numpy(a).to(dev) for a in (q, k, v))
+    state = deploy.init_state(tq, tk, seed=1)
+    want = pinned.step(tq, tk, tv, dict(state)).clone()
+    deploy.pin_tail = 300
+    old = deploy.QU, deploy.KU, deploy.qlab      # kept: nothing is freed here
+    deploy.QU, deploy.KU, deploy.qlab = (torch.zeros_like(t) for t in old)
+    for t in old:
+        t.fill_(7)
+    assert torch.equal(deploy.step(tq, tk, tv, dict(state)), want)
+    assert all(bool((t == 7).all()) for t in old)
+    assert torch.equal(deploy.QU, ops.project(tq, state["Uq"]))
+    assert torch.equal(deploy._last["qlab"], deploy.qlab)
+    assert deploy._ws_split.numel() > 256
+    deploy._ws_split = deploy._ws_split[:256]
+    whole = deploy.step(tq, tk, tv, dict(state)).clone()
+    # either form rounds its weights and output to fp16 (u = 2^-11 each)
+    assert float((whole.float() - want.float()).norm()) <= 4 * 2.0 ** -11 * float(want.float().norm())
+    deploy.scale = 0.05
+    deploy.step(tq, tk, tv, dict(state))
+    assert torch.equal(deploy._last["cks"], ops.centroid_finalize(deploy._kmm_ck2, 0.05)[1])
+    deploy.QU = deploy.QU[:, :100].contiguous()
+    with pytest.raises(ValueError, match="QU"):
+        deploy.step(tq, tk, tv, dict(state))

@@ -270,19 +270,6 @@ class MaskedStepDeploy:
         self._cfg_key = 0
         self._cfg_step = 0
 
-        # the fields of a call's arguments that never change: its own buffers
-        a = self._args = _lib.StepArgs()
-        a.struct_bytes = ctypes.sizeof(a)
-        a.H, a.N, a.CQ, a.CK, a.pin_tail, a.scale = H, N, CQ, C, self.pin_tail, self.scale
-        for name, t in (("QU", self.QU), ("KU", self.KU), ("rowcnt", self.rowcnt),
-                        ("ck2", self._kmm_ck2), ("sumv", self._kmm_sumv), ("lam", self._kmm_lam),
-                        ("tiles", self._ctiles), ("lse", self._lse)):
-            setattr(a, name, t.data_ptr())
-        for name, t in (("ws_kmm", self._ws_kmm), ("ws_vst", self._ws_vst),
-                        ("ws_sel", self._ws_sel), ("ws_split", self._ws_split)):
-            setattr(a, name, t.data_ptr())
-            setattr(a, name + "_bytes", t.numel())
-
         # default-priority streams (the two-stream schedule of the reference)
         self.s_main = torch.cuda.Stream(device=dev)
         self.s_side = torch.cuda.Stream(device=dev)
@@ -420,11 +407,35 @@ class MaskedStepDeploy:
         with self._lock, torch.cuda.device(self.dev):
             return self._step(q, k, v, state, out)
 
+    def _own_args(self):
+        """A call's arguments that name this object's own settings and buffers, as
+        they stand now."""
+        H, N = self.H, self.N
+        a = _lib.StepArgs()
+        a.struct_bytes = ctypes.sizeof(a)
+        a.H, a.N, a.CQ, a.CK = H, N, self.CQ, self.C
+        a.pin_tail, a.scale = int(self.pin_tail), float(self.scale)
+        for name, shape, dtype in (("QU", (H, N, self.r), torch.float16),
+                                   ("KU", (H, N, self.r), torch.float16),
+                                   ("rowcnt", (H, N), torch.int32), ("qlab", (H, N), torch.int32),
+                                   ("klab", (H, N), torch.int32)):
+            t = getattr(self, name)
+            ops._check(t, shape, dtype, name, self.dev)
+            setattr(a, name, t.data_ptr())
+        for name, t in (("ck2", self._kmm_ck2), ("sumv", self._kmm_sumv), ("lam", self._kmm_lam),
+                        ("tiles", self._ctiles), ("lse", self._lse)):
+            setattr(a, name, t.data_ptr())
+        for name in ("ws_kmm", "ws_vst", "ws_sel", "ws_split"):
+            t = getattr(self, "_" + name)
+            setattr(a, name, t.data_ptr())
+            setattr(a, name + "_bytes", t.numel())
+        return a
+
     def _step(self, q, k, v, state, out):
         H, N, C, CQ, D = self.H, self.N, self.C, self.CQ, self.D
         if not (q.dtype == k.dtype == v.dtype) or q.dtype not in (torch.float16, torch.bfloat16):
             raise TypeError("step: q, k, v must share dtype fp16 or bf16")
-        a = _lib.StepArgs.from_buffer_copy(self._args)
+        a = self._own_args()
         a.dtype = _lib.dtype_code(q.dtype)
         io = self._buffers(q.dtype)
         dst = io["out"] if out is None else out
