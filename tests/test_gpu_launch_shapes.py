@@ -273,6 +273,36 @@ def test_step_stages_and_streams(dev):
         assert all(torch.equal(x, y) for x, y in zip(full + reuse, a + b))
 
 
+@pytest.mark.parametrize("with_kmeans", [False, True])
+def test_step_stages_run_in_order(dev, with_kmeans):
+    """The tile image of a call that also finalises the centroids holds those,
+    not the ones that were there before."""
+    from token2tile_amd import _lib, ops
+    from token2tile_amd.deploy_step import MaskedStepDeploy
+    gen = torch.Generator(device=dev).manual_seed(2)
+    H, N, CQ = 2, 3000, 20
+    q, k, v = (torch.randn(H, N, 128, generator=gen, device=dev).half() for _ in range(3))
+    op = MaskedStepDeploy(H, N, CQ, device=dev)
+    state = op.init_state(q, k, seed=1)
+    first = dict(state)
+    op._ctiles.zero_()                       # (its rows are padded)
+    op.step(q, k, v, state)
+    want = op._ctiles.clone()
+    a, last = op._own_args(), op._last
+    cks, ck16 = torch.zeros_like(last["cks"]), torch.zeros_like(last["cks"])
+    cq2 = torch.empty_like(state["cq"])
+    kcounts, kperm, qcounts, qperm = (last[n].clone() for n in ("counts", "kperm", "tile_sizes", "qperm"))
+    a.v, a.v_head_stride, a.v_row_stride = v.data_ptr(), N * 128, 128
+    for name, t in (("kcounts", kcounts), ("kperm", kperm), ("qcounts", qcounts), ("qperm", qperm),
+                    ("cks", cks), ("ck16", ck16), ("cq2", cq2), ("cq0", first["cq"]), ("ck0", first["ck"])):
+        setattr(a, name, t.data_ptr())
+    op._ctiles.zero_()
+    stages = _lib.STEP_VSTATS | _lib.STEP_FINALIZE | _lib.STEP_TILES
+    assert _lib.lib().t2t_step(a, stages | (_lib.STEP_KMEANS if with_kmeans else 0),
+                               _lib.stream_handle()) == 0
+    assert torch.equal(cks, last["cks"]) and torch.equal(op._ctiles, want)
+
+
 # one wave's sort, strides across waves, several keys per thread, more clusters
 # than key clusters, and a list past the sort's limit (cluster order)
 @pytest.mark.parametrize("H,N,CQ,kind", [(2, 5000, 1, "mix"), (2, 9000, 65, "mix"),

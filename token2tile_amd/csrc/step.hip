@@ -20,11 +20,12 @@ extern "C" int t2t_step(const t2t_step_args* a, unsigned stages, void* stream) {
   // Stages asked for together share kernels where their results allow: both
   // projections one launch; the finalised centroids come from the key sums
   // and the tile image from the value statistics (2 x 4096 tokens: three
-  // launches of 3-5 us less)
+  // launches of 3-5 us less), unless a FINALIZE after them is still to write the
+  // centroids that the image holds
   const unsigned pair = T2T_STEP_PROJECT_Q | T2T_STEP_PROJECT_K;
   const bool fin = (stages & T2T_STEP_KMEANS) && (stages & T2T_STEP_FINALIZE) && a->ck16 && a->cks;
-  const bool tiles = (stages & T2T_STEP_TILES) && (fin || (stages & T2T_STEP_VSTATS)) && CK == 2048 &&
-                     a->cks && a->tiles;
+  const bool tiles = (stages & T2T_STEP_TILES) && CK == 2048 && a->cks && a->tiles &&
+                     (fin || ((stages & T2T_STEP_VSTATS) && !(stages & T2T_STEP_FINALIZE)));
   if ((stages & pair) == pair)
     ST_CHECK(t2t_project_pair(a->q, a->q_head_stride, a->q_row_stride, a->Uq, a->QU, a->k,
                               a->k_head_stride, a->k_row_stride, a->Uk, a->KU, dt, H, N, stream));
