@@ -406,6 +406,46 @@ def test_split_call_equals_its_stages(dev, H, N, CQ, dtype):
     assert not a.isnan().any() and torch.equal(a, b)
 
 
+# parts added by the combine and by the residual
+@pytest.mark.parametrize("H,N,CQ", [(1, 4100, 16), (3, 12000, 60)])
+def test_split_call_on_a_kept_plan(dev, H, N, CQ):
+    """A plan serves the query clusters it was built for whatever the union is
+    now (it orders and cuts the queries): lengths that grew, shrank to less than
+    a tile per part or to nothing.  Bounds as between split and whole tasks."""
+    from token2tile_amd import ops
+    rng = np.random.default_rng(N)
+    qlab, klab, qperm, qcounts, kperm, kcounts = structure(rng, H, N, CQ)
+    dens = rng.choice([0.0, 0.002, 0.3, 1.0], (2, H, CQ, 1))
+    dens[0, :, :4], dens[1, :, :4] = [[0.0], [1.0], [1.0], [1.0]], [[1.0], [0.0], [0.001], [0.05]]
+    dens[1, :, 2] = 0.0
+    sel = (rng.random((2, H, CQ, 2048)) < dens).astype(np.uint8)
+    sel[1, :, 2, 0] = 1                        # a single cluster, of at most a few keys
+    was, now = (g(np.packbits(x, axis=2, bitorder="little").view(np.int32), dev) for x in sel)
+    gen = torch.Generator(device=dev).manual_seed(N)
+    r = lambda *s: torch.randn(*s, generator=gen, device=dev)  # noqa: E731
+    q, kp, vp = (r(H, N, 128).half() for _ in range(3))
+    q *= 0.5
+    QU, cks, sumv = r(H, N, 32).half(), (0.1 * r(H, 2048, 32)).half(), r(H, 2048, 128).half()
+    lam, tw = torch.linspace(1, 2, H, device=dev), torch.tensor(1.0, device=dev)
+    tq, tk, tqp, tql = (g(a, dev) for a in (qcounts, kcounts, qperm, qlab))
+    plan = ops.tile_plan(tq, tk, was, N)
+    new = lambda: (torch.full_like(q, float("nan")), torch.full((H, N), float("nan"), device=dev))  # noqa: E731
+    (a, la), (b, lb), (m, lm) = new(), new(), new()
+    ops.tile_attn_exact_orig(q, kp, vp, tk, now, tqp, plan, a, la)
+    ops.tile_attn_exact_orig(q, kp, vp.abs(), tk, now, tqp, plan, m, lm)
+    ops.tile_attn_exact_split(q, kp, vp, None, tk, now, tql, tqp, plan, b, lb, gather=0)
+    u = 2.0 ** -11
+    assert not a.isnan().any() and not b.isnan().any()
+    assert bool(((a - b).float().abs() <= 4.04 * u * m.float() + 2 * u * a.float().abs() + 1e-6).all())
+    fin = la.isfinite()
+    assert not fin.all() and torch.equal(la[~fin], lb[~fin])
+    assert float((la - lb)[fin].abs().max()) <= 2 * u * 1.4427 * 1.01 + 2e-5
+    ops.resid_merge_inplace(b, lb, QU, ops.centroid_tiles(cks, sumv), tk, now, tql, tqp, lam, tw)
+    c2, _ = new()
+    ops.tile_attn_run_planned(q, kp, vp, tq, tk, now, QU, cks, sumv, lam, tql, tqp, tw, c2, plan, False)
+    assert torch.equal(c2, b)
+
+
 # parts added by the combine, and by the residual
 @pytest.mark.parametrize("H,N,CQ", [(1, 4100, 16), (3, 12000, 60)])
 def test_attention_without_room_for_parts(dev, H, N, CQ):

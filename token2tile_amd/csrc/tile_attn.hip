@@ -300,7 +300,10 @@ __device__ inline int xcd_remap(int bid, int total) {
 // unnormalised in fp32 and combine_kernel adds the parts.  P follows the
 // task's own length, at least TA_SPLIT_TILES tiles a part (below that a
 // part's start, the union runs and the first tile's fetch, costs more than
-// its tiles).
+// its tiles).  The length is the plan's kvlen on every side (the parts, the
+// combine and the residual), so they agree also where a kept plan is used with
+// another union than it was built from; the tiles that the parts share are
+// always the union's own.
 #define TA_SPLIT_MAX 8
 #define TA_SPLIT_TILES 6
 __host__ __device__ inline int split_parts(int kvlen, int S) {
@@ -397,7 +400,8 @@ __global__ __launch_bounds__(TA_WAVES * 64, 2) void attn_kernel(
     const int32_t* __restrict__ tasks, uint16_t* __restrict__ attn_out, float* __restrict__ lse,
     uint16_t* __restrict__ out, const int32_t* __restrict__ kperm, int H, int N, int CQ, int maxT,
     long long sqh, long long sqn, long long skh, long long skn, long long soh, long long son,
-    long long svh, long long svn, int S, float* __restrict__ opart, float* __restrict__ mlpart) {
+    long long svh, long long svn, int S, const int32_t* __restrict__ plan_kvlen,
+    float* __restrict__ opart, float* __restrict__ mlpart) {
   // row n of head h of q / k (MODE 2) / out (MODE 1, 2) sits at base + h s_h + n s_n
   // (elements): [H, N, 128] contiguous or a strided view such as token-major [N, H, 128]
   constexpr bool KG = MODE >= 2;
@@ -441,6 +445,8 @@ __global__ __launch_bounds__(TA_WAVES * 64, 2) void attn_kernel(
   if (ti >= ntask[h]) return;
   const int32_t* tk = tasks + ((size_t)h * maxT + ti) * 4;
   const int t = tk[0], qs = tk[1], qrows = tk[2];
+  const int nparts = SPLIT ? split_parts(plan_kvlen[(size_t)h * CQ + t], S) : 1;
+  if (SPLIT && part >= nparts) return;  // uniform
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int jl = lane & 31, hh = lane >> 5;
 
@@ -474,8 +480,6 @@ __global__ __launch_bounds__(TA_WAVES * 64, 2) void attn_kernel(
     nrun += wsc[i];
     kvlen += wsr[i];
   }
-  const int nparts = SPLIT ? split_parts(kvlen, S) : 1;
-  if (SPLIT && part >= nparts) return;  // uniform
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
     if (cnts[j] > 0) {
@@ -578,7 +582,12 @@ __global__ __launch_bounds__(TA_WAVES * 64, 2) void attn_kernel(
 #pragma unroll
   for (int nb = 0; nb < 4; ++nb) O[nb] = zero16();
 
-  if (kvlen > 0) {
+  // tiles tb .. tb + ntile - 1 of the task's, the last one partial or not (a
+  // part holds none only where the union has shrunk since the plan)
+  const int nall = (kvlen + TA_KT - 1) / TA_KT;
+  const int tb = SPLIT ? (int)((long long)part * nall / nparts) : 0;
+  const int ntile = SPLIT ? (int)((long long)(part + 1) * nall / nparts) - tb : nall;
+  if (ntile > 0) {
     // ---- queries: B operand fragments (dims 16 s + 8 hh .. + 7)
     u32x4 qb[8];
     {
@@ -592,10 +601,6 @@ __global__ __launch_bounds__(TA_WAVES * 64, 2) void attn_kernel(
     const uint32_t krow_bytes = KG ? (uint32_t)(skn * 2) : 256u;
     const char* vh = (const char*)(vp + (VG ? (size_t)h * svh : (size_t)h * N * TA_D));
     const uint32_t vrow_bytes = VG ? (uint32_t)(svn * 2) : 256u;
-    // tiles tb .. tb + ntile - 1 of the task's, the last one partial or not
-    const int nall = (kvlen + TA_KT - 1) / TA_KT;
-    const int tb = SPLIT ? (int)((long long)part * nall / nparts) : 0;
-    const int ntile = SPLIT ? (int)((long long)(part + 1) * nall / nparts) - tb : nall;
     const bool partial = kvlen % TA_KT != 0 && tb + ntile == nall;
     // source rows of tile `tile` -> sIdx[tile & 1]; past the end -> row 0
     // (its keys are masked and its values multiply a zero probability).
@@ -915,7 +920,7 @@ __global__ __launch_bounds__(TA_WAVES * 64, 2) void attn_kernel(
             *(f32x4*)(op + 32 * nb + 8 * g) =
                 f32x4{O[nb][4 * g], O[nb][4 * g + 1], O[nb][4 * g + 2], O[nb][4 * g + 3]};
         if (hh == 0) {
-          mlpart[2 * pr] = m;
+          mlpart[2 * pr] = kvlen > 0 ? m : -__builtin_inff();
           mlpart[2 * pr + 1] = lt;
         }
       }
@@ -960,7 +965,8 @@ static void launch_attn(const void* q, const void* kp, const void* vp, const int
                      (const uint16_t*)q, (const uint16_t*)kp, (const uint16_t*)vp,
                      (const uint32_t*)unip, qperm, kcounts, p.k_off, p.ntask, p.tasks,
                      (uint16_t*)attn_out, lse, (uint16_t*)out, kperm, H, N, CQ, p.maxT, sqh, sqn,
-                     skh, skn, soh, son, svh, svn, 1, (float*)nullptr, (float*)nullptr);
+                     skh, skn, soh, son, svh, svn, 1, (const int32_t*)nullptr, (float*)nullptr,
+                     (float*)nullptr);
 }
 
 // A sorted row's parts: the weight of each (0 past P), the log2-sum of the row.
@@ -977,12 +983,14 @@ struct PartSum {
       l[i] = i < P ? mlpart[2 * (row + i * HN) + 1] : 0.f;
       if (i < P) M = vmax(M, a[i]);
     }
+    const bool none = M == -__builtin_inff();  // no keys: zeros, log-sum -inf
+    if (none) M = 0.f;
 #pragma unroll
     for (int i = 0; i < TA_SPLIT_MAX; ++i) {
       a[i] = i < P ? __builtin_amdgcn_exp2f(a[i] - M) : 0.f;
       lt = i < P ? fmaf(a[i], l[i], lt) : lt;
     }
-    const float inv = 1.0f / lt;
+    const float inv = none ? 0.f : 1.0f / lt;
 #pragma unroll
     for (int i = 0; i < TA_SPLIT_MAX; ++i) a[i] *= inv;
     lse2 = M + __log2f(lt);
@@ -1056,7 +1064,7 @@ static void launch_attn_split(const void* q, const void* k, const void* v, const
                      (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v,
                      (const uint32_t*)unip, qperm, kcounts, p.k_off, p.ntask, p.tasks,
                      (uint16_t*)nullptr, lse, (uint16_t*)out, kperm, H, N, CQ, p.maxT, sd[0], sd[1],
-                     sd[2], sd[3], sd[6], sd[7], sd[4], sd[5], S, w.opart, w.mlpart);
+                     sd[2], sd[3], sd[6], sd[7], sd[4], sd[5], S, p.kvlen, w.opart, w.mlpart);
   if (!combine) return;  // the residual adds the parts
   hipLaunchKernelGGL(combine_kernel<T>, dim3(cdiv(N, 8), H), dim3(256), 0, st, w.opart, w.mlpart,
                      p.kvlen, qlab, qperm, (uint16_t*)out, lse, H, N, CQ, S, sd[6], sd[7]);
