@@ -296,3 +296,69 @@ def test_settings_and_buffers_replaced_after_construction(dev):
     deploy.QU = deploy.QU[:, :100].contiguous()
     with pytest.raises(ValueError, match="QU"):
         deploy.step(tq, tk, tv, dict(state))
+
+
+@pytest.mark.parametrize("form", ["full", pytest.param("reuse", marks=pytest.mark.skip(
+    reason="ending the capture of two forked streams that wait for each other crashed the "
+           "process; step() refuses a reuse call under capture"))])
+def test_captured_call_replays_as_eager(dev, form):
+    """A call captured into a graph and replayed on new contents of the same
+    tensors, with eager calls and synchronisations between the replays: the
+    eager results, bit for bit."""
+    from token2tile_amd.deploy_step import MaskedStepDeploy
+    deploy, q, k, v = make(dev, mask_refresh=4)
+    eager = MaskedStepDeploy(deploy.H, deploy.N, deploy.CQ, s_frac=0.05, mask_refresh=4, device=dev)
+    q, k, v = (torch.from_numpy(a).to(dev) for a in (q, k, v))
+    state = deploy.init_state(q, k, seed=1)
+
+    def call(op, key, form, out):
+        op.set_cfg_call(0 if form == "full" else 1, key=key, step=0)
+        st = dict(state)
+        op.step(q, k, v, st, out=out)
+        assert op.last_call_full == (form == "full")
+        return st
+
+    outs = [torch.empty_like(q) for _ in range(3)]
+    for op in (deploy, eager):                  # streams and queues are made here
+        for f in ("full", "reuse"):
+            call(op, 0, f, outs[2])
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        new = call(deploy, 1 if form == "full" else 0, form, outs[0])
+    gen = torch.Generator(device=dev).manual_seed(3)
+    noise = lambda t: 0.05 * torch.randn(t.shape, generator=gen, device=dev).to(t.dtype)  # noqa: E731
+    for _ in range(4):
+        q += noise(q)
+        v += noise(v)
+        graph.replay()
+        if form == "full":
+            eager.reset_cfg_reuse()
+        st = call(eager, 0, form, outs[1])
+        torch.cuda.synchronize()
+        assert torch.equal(outs[0], outs[1])
+        assert torch.equal(new["ck"], st["ck"]) and torch.equal(new["cq"], st["cq"])
+        v += noise(v)
+        if form == "full":                      # later calls on the replayed structure
+            call(deploy, 1, "reuse", outs[1])
+            call(eager, 0, "reuse", outs[2])
+            assert torch.equal(outs[1], outs[2]) and not torch.equal(outs[0], outs[1])
+
+
+def test_reuse_call_refuses_capture(dev, monkeypatch):
+    """Refused before anything is launched or forked, and the annotation spent."""
+    deploy, q, k, v = make(dev, mask_refresh=4)
+    q, k, v = (torch.from_numpy(a).to(dev) for a in (q, k, v))
+    state = deploy.init_state(q, k, seed=1)
+    deploy.set_cfg_call(0, key=0, step=0)
+    deploy.step(q, k, v, state)
+    deploy.set_cfg_call(1, key=0, step=0)
+    want = deploy.step(q, k, v, state).clone()
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    monkeypatch.setattr(deploy, "_launch", lambda *a: pytest.fail("launched"))
+    deploy.set_cfg_call(1, key=0, step=0)
+    with pytest.raises(RuntimeError, match="captured"):
+        deploy.step(q, k, v, state)
+    monkeypatch.undo()
+    deploy.set_cfg_call(1, key=0, step=0)
+    assert torch.equal(deploy.step(q, k, v, state), want)

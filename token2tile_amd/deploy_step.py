@@ -401,7 +401,8 @@ class MaskedStepDeploy:
         state: dict(Uq, Uk, ck, cq) fp16; ck/cq are replaced by fresh tensors
         holding the centroids that warm-start the next call.  Returns out
         [H, N, 128] in q's dtype: the given ``out`` view (written in place), or
-        a buffer reused by the next call."""
+        a buffer reused by the next call.  Under graph capture a rebuilding call
+        is recorded; a reuse call raises RuntimeError."""
         # the events and buffers serve one call at a time; the launches, events
         # and the capture query go to this object's GPU whichever is current
         with self._lock, torch.cuda.device(self.dev):
@@ -480,9 +481,6 @@ class MaskedStepDeploy:
                 self._ev[which].record(signals)
                 waits.wait_event(self._ev[which])
 
-        if caller != s0:
-            after(s0, 0, caller)
-
         snap = None
         held = None
         cfg_parity = self._cfg_parity
@@ -494,7 +492,14 @@ class MaskedStepDeploy:
             if held is not None and age >= 0 and not (cfg_parity == 0 and refresh_due):
                 snap = held
         recycle = held is not None and snap is None
+        if capturing and snap is not None:
+            # s_main and s_side, both forked from the capturing stream, wait for
+            # each other here: the end of such a capture crashed the process
+            raise RuntimeError("step: a reuse call cannot be captured into a graph; capture "
+                               "structure-rebuilding calls and run reuse calls outside")
         self.last_call_full = snap is None
+        if caller != s0:
+            after(s0, 0, caller)
 
         if snap is not None:
             st = snap
@@ -510,15 +515,14 @@ class MaskedStepDeploy:
             if self._fused_kv:
                 side += (("", _lib.STEP_VSTATS | _lib.STEP_TILES),)
             self._launch(a, side, s1)
-            joined = torch.cuda.Event() if capturing else self._ev[2]
-            joined.record(s1)
+            self._ev[2].record(s1)
             main = ()
             if not self.fuse_k_gather:
                 main += (("gather_k", _lib.STEP_GATHER_K),)
             if not self._fused_kv:
                 main += (("vstats", _lib.STEP_VSTATS),)
             self._launch(a, main + (("attention_exact", _lib.STEP_EXACT),), s0)
-            s0.wait_event(joined)
+            s0.wait_event(self._ev[2])
             tail = () if self._fused_kv else (("attention_prep", _lib.STEP_TILES),)
             self._launch(a, tail + (("attention_residual", _lib.STEP_RESIDUAL),), s0)
         else:
@@ -561,9 +565,6 @@ class MaskedStepDeploy:
                     else:  # qlab, klab and counts are this object's own: copied
                         own = dict(st, **{n: st[n].clone() for n in ("qlab", "klab", "counts")})
                     self._cfg_hold[self._cfg_key] = dict(own, Uq=state["Uq"], step=self._cfg_step)
-        if capturing:
-            s1.wait_stream(s0)
-            caller.wait_stream(s1)
         if caller != s0:
             after(caller, 3, s0)
         self._last = dict(unip=st["unip"], qperm=st["qperm"], tile_sizes=st["tile_sizes"],
