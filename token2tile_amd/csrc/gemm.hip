@@ -429,7 +429,8 @@ __device__ constexpr GrPairs GR_PAIR = gr_pairs();
 // G[c_i + l / 16 + 4 r][c_j + l % 16] in register r of lane l (rows
 // interleaved by four, as measured on the GPU).
 // Products of fp16 values are exact in fp64, and each output sums its rows in
-// a fixed order, so the result does not depend on the launch.
+// a fixed order, so calls of one (H, N) agree bit for bit; the splits, and with
+// them the rounding of the fp64 sums, follow H and N (gram_splits).
 // bad[s, h] = 1 when a row of the block holds an inf or NaN.
 // VEC: D == 128 and 16-byte aligned rows (16-byte loads); else element loads.
 template <typename T, bool VEC>

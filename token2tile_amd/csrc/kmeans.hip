@@ -291,10 +291,12 @@ static void launch_fast_assign32(const void* x, const void* c, int32_t* labels, 
 
 // ---------------------------------------------------------------------------
 // k-means assignment at rank 32: d = |c|^2 + x.(-2c),
-// argmin, ties to the lowest index.  One 8-wave work-group per 1024 rows, four
-// 32-row blocks per wave, so every centroid fragment and norm read from LDS
-// feeds four MFMA chains; the centroids (-2c and |c|^2 from cen_prep_kernel)
-// are staged in chunks of CMAX rows (34 KB at 512: four work-groups per CU).
+// argmin, ties to the lowest index.  One work-group per 256 RB rows: RB 32-row
+// blocks per wave, so every centroid fragment and norm read from LDS feeds RB
+// MFMA chains, and CS groups of eight waves that share the rows and take the
+// centroid blocks in turn (below).  The centroids (-2c and |c|^2 from
+// cen_prep_kernel) are staged in chunks of CMAX rows (34 KB at 512: four
+// work-groups of eight waves per CU, two of sixteen).
 // Centroid row r keeps its 16-byte chunk c at c ^ ((r >> 2) & 3), so the 32
 // rows a fragment read touches fall on distinct banks.
 //

@@ -62,9 +62,9 @@ extern "C" size_t t2t_tile_plan_ints(int H, int N, int CQ) {
 
 #define PLAN_SORT_MAX 4096
 
-// One work-group per head: its ~15 us are latency, of which reading a union
+// One work-group per head: its 11-45 us are latency, of which reading a union
 // word per cluster one after the other and a barrier for every step of a
-// task sort were most (28 us at 201 clusters, 52 at 512, 77 at 768; now 17, 30, 40).  The words of
+// task sort were most (28 us at 201 clusters, 52 at 512, 77 at 768; now 18, 32, 45).  The words of
 // sixteen clusters are in flight per wave, and a word's clusters are summed from
 // the bit planes of their sizes (one bit count per plane that any size has,
 // not one LDS read per cluster); the clusters are sorted, not their tasks (a
